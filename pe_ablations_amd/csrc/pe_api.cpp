@@ -259,6 +259,7 @@ pe::CoreArgs core_args(const pe_attn_params* p, const Layout& L, const char* ws,
   memset(&c, 0, sizeof(c));
   c.q = ws + L.q_off;
   c.k = ws + L.k_off;
+  c.k_rows = p->Sk;
   if (v_direct(p, v, L.dv)) {
     c.v = v->data; c.v_sb = v->stride[0]; c.v_sh = v->stride[1]; c.v_ss = v->stride[2];
   } else {
@@ -567,8 +568,19 @@ namespace {
 // Work split and workspace of pe_attn_decode: transformed queries, then the per-range partials.
 struct DecodePlan {
   int nqt, nunit;
+  bool chunk;         // many query rows: the forward kernel over key ranges (cp), not the decode kernel
+  pe::ChunkPlan cp;
   size_t q_bytes, po_off, pm_off, pl_off, total;
 };
+
+// The decode kernel re-reads a kv head's cache, from L2, for every 32 query rows and runs one wave per
+// SIMD; the forward kernel shares a tile of it between 128 or 256 rows, but pays for a whole block.
+// Measured per call, decode kernel against forward kernel (us): 16 heads of 128, 6000 rows cached, 64 new
+// rows 38.8 / 29.8, 200: 128 / 38, 700: 278 / 73; 32 rows 30.3 on the decode kernel.  With few rows in
+// all the forward kernel is no faster: one kv head of 128, 200 rows 22.5 / 25.8 against 1024 cached
+// rows and 42 / 34 against 16000, 800 rows 27.8 / 22.5 and 78 / 36; 4 kv heads of the split form, 64 rows
+// each 22.9 / 27.0 against 16000.
+constexpr int64_t CHUNK_MIN_ROWS = 64, CHUNK_MIN_ALL_ROWS = 640;
 
 DecodePlan decode_plan(const pe_attn_params* p) {
   DecodePlan d{};
@@ -584,7 +596,13 @@ DecodePlan decode_plan(const pe_attn_params* p) {
   nu = std::min<int64_t>(nu, (nkb + 1) / 2);
   nu = std::max<int64_t>(4, std::min<int64_t>(512, (nu + 3) / 4 * 4));
   d.nunit = (int)nu;
-  const size_t rows = (size_t)tiles * d.nunit * 32;
+  size_t rows = (size_t)tiles * d.nunit * 32;
+  const int64_t crows = (int64_t)grp * p->Sq;
+  d.chunk = half_dt(p->dtype) && crows >= CHUNK_MIN_ROWS && crows * p->B * p->Hkv >= CHUNK_MIN_ALL_ROWS;
+  if (d.chunk) {
+    d.cp = pe::chunk_plan(crows, (int64_t)p->B * p->Hkv, p->Sk, pad_qk(qk_width(p)));
+    rows = (size_t)d.cp.nblk * d.cp.bm * d.cp.nsplit * p->B * p->Hkv;
+  }
   d.q_bytes = align_up((size_t)p->B * p->Hq * p->Sq * pad_qk(qk_width(p)) * esz(p));
   d.po_off = d.q_bytes;
   d.pm_off = d.po_off + align_up(rows * pad_v(p->Dv) * 4);
@@ -687,6 +705,17 @@ int pe_attn_decode(const pe_attn_params* p, const pe_tensor_t* qc, const pe_tens
   da.o = (void*)out->data; da.o_sb = out->stride[0]; da.o_sh = out->stride[1]; da.o_ss = out->stride[2];
   da.o_dtype = out->dtype; da.dv_real = p->Dv;
   da.lse = lse;
+  if (d.chunk) {
+    pe::CoreArgs c;
+    memset(&c, 0, sizeof(c));
+    c.q = ws; c.k = k_cache; c.k_rows = capacity;
+    c.v = v_cache; c.v_ss = dv; c.v_sh = (int64_t)capacity * dv; c.v_sb = (int64_t)p->Hkv * capacity * dv;
+    c.B = p->B; c.Hq = p->Hkv; c.Hkv = p->Hkv; c.Sq = p->Hq / p->Hkv * p->Sq; c.Sk = p->Sk;
+    c.causal = da.causal; c.causal_off = da.off; c.scale = p->scale;
+    c.chunk_q = p->Sq; c.nsplit = d.cp.nsplit;
+    c.part_o = da.part_o; c.part_m = da.part_m; c.part_l = da.part_l;
+    return pe::launch_fwd_chunk(p->dtype, dqk, dv, d.cp, c, da, s);
+  }
   return pe::launch_decode(p->dtype, dqk, dv, da, s);
 }
 

@@ -13,7 +13,8 @@
 //
 // Query rows of one kv head's GQA group share the tile: row r of tile qt is query head
 // hk * grp + r / Sq, query r % Sq (Sq new queries, grp = Hq / Hkv), so one decoded token of eight
-// query heads per kv head fills eight MFMA columns instead of one.
+// query heads per kv head fills eight MFMA columns instead of one.  Calls with many query rows (a
+// prompt prefilled in chunks) go to the forward kernel over key ranges instead (launch_fwd_chunk).
 #include "pe_common.h"
 #include "pe_internal.h"
 

@@ -7,6 +7,8 @@
 // O^T += v^T P^T  (A = v read with the transpose load, B = P^T straight from the C registers).
 // The scores are the reference's SDPA scores on [content | mu cos | mu sin] operands
 // (src/model/fpope_attention.py:166-177, src/model/fpope.py:409-417).
+#include <algorithm>
+
 #include "pe_common.h"
 #include "pe_internal.h"
 
@@ -50,7 +52,7 @@ __global__ __launch_bounds__(NW * 64, 1) void fwd_kernel(CoreArgs a, int o_vec) 
   int kend = a.Sk;
   if (a.causal) kend = min(a.Sk, q0 + BM + off);
   const int nkb = kend > 0 ? (kend + BN - 1) / BN : 0;
-  const char* kbase = (const char*)((const E*)a.k + (int64_t)(b * a.Hkv + hk) * a.Sk * DQK);
+  const char* kbase = (const char*)((const E*)a.k + (int64_t)(b * a.Hkv + hk) * a.k_rows * DQK);
   const char* vbase = (const char*)((const E*)a.v + b * a.v_sb + hk * a.v_sh);
   const int64_t krs = (int64_t)DQK * ESZ, vrs = a.v_ss * ESZ;
 
@@ -175,7 +177,9 @@ __global__ __launch_bounds__(NW * 64, 1) void fwd_kernel(CoreArgs a, int o_vec) 
 // MFMAs.  The running max is raised lazily: O and l are rescaled only when some query's block
 // max exceeds the current one by more than TAU (in log2 units), which bounds p by 2^TAU.
 // MB: the explicit-mask instantiation, which adds mask_l2 to the scaled scores before the softmax.
-template <int HT, int DQK, int DV, int BN, int NW, int NDW, int NSTG, bool MB = false>
+// SK: the key-split instantiation over a KV cache (CoreArgs::nsplit): rows are the query heads of one
+// kv head after another, and the workgroup walks its range of the block's key tiles.
+template <int HT, int DQK, int DV, int BN, int NW, int NDW, int NSTG, bool MB = false, bool SK = false>
 __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void fwd_bf16_kernel(CoreArgs a, int o_vec) {
   using M = MT<HT>;  // HT: the 16-bit operand type, bf16 (0) or fp16 (2)
   constexpr int BM = NW * 32;
@@ -197,11 +201,26 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void fwd_bf16_kernel(Core
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 5, l32 = lane & 31;
   const int nqb = (a.Sq + BM - 1) / BM;
-  int qb, bh;
-  map_block(blockIdx.x, nqb, a.B * a.Hq, a.causal != 0, qb, bh);
+  int qb, bh, sp = 0;
+  map_block(blockIdx.x, SK ? nqb * a.nsplit : nqb, a.B * a.Hq, !SK && a.causal != 0, qb, bh);
+  if constexpr (SK) {
+    sp = qb / nqb;
+    qb -= sp * nqb;
+  }
   const int b = bh / a.Hq, h = bh % a.Hq, hk = h / (a.Hq / a.Hkv);
   const int q0 = qb * BM, qw = q0 + w * 32, myq = qw + l32;
   const int off = a.causal_off;
+  // the causal positions: this lane's query, and the first and last query of the wave's 32 rows and
+  // the last one of the block's (SK: 0 and chunk_q - 1 where the rows pass from one head to the next)
+  int pq = myq, pw0 = qw, pw1 = qw + 31, pb1 = q0 + BM - 1;
+  if constexpr (SK) {
+    const int n = a.chunk_q;
+    pq = myq % n;
+    pw0 = qw % n;
+    pw1 = pw0 + 31 < n ? pw0 + 31 : n - 1;
+    if (pw0 + 31 >= n) pw0 = 0;
+    pb1 = q0 % n + BM - 1 < n ? q0 % n + BM - 1 : n - 1;
+  }
 
   u32x4 qf[NQF];
   {
@@ -217,9 +236,14 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void fwd_bf16_kernel(Core
   }
 
   int kend = a.Sk;
-  if (a.causal) kend = min(a.Sk, q0 + BM + off);
-  const int nkb = kend > 0 ? (kend + BN - 1) / BN : 0;
-  const char* kbase = (const char*)((const uint16_t*)a.k + (int64_t)(b * a.Hkv + hk) * a.Sk * DQK);
+  if (a.causal) kend = min(a.Sk, pb1 + 1 + off);
+  int nkb = kend > 0 ? (kend + BN - 1) / BN : 0, kb0 = 0;
+  if constexpr (SK) {
+    // nkb * nsplit < 2^31 (at most 128 ranges of at most 2^24 tiles); wave-uniform, in scalar registers
+    kb0 = __builtin_amdgcn_readfirstlane((uint32_t)(nkb * sp) / (uint32_t)a.nsplit);
+    nkb = __builtin_amdgcn_readfirstlane((uint32_t)(nkb * (sp + 1)) / (uint32_t)a.nsplit);
+  }
+  const char* kbase = (const char*)((const uint16_t*)a.k + (int64_t)(b * a.Hkv + hk) * a.k_rows * DQK);
   const char* vbase = (const char*)((const uint16_t*)a.v + b * a.v_sb + hk * a.v_sh);
   const int64_t krs = (int64_t)DQK * 2, vrs = a.v_ss * 2;
 
@@ -265,8 +289,8 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void fwd_bf16_kernel(Core
   };
 #pragma unroll
   for (int i = 0; i < NSTG - 1; ++i)
-    if (i < nkb) issue(i);
-  for (int kb = 0; kb < nkb; ++kb) {
+    if (kb0 + i < nkb) issue(kb0 + i);
+  for (int kb = kb0; kb < nkb; ++kb) {
     const int k0 = kb * BN;
     // the slot offset is opaque to the compiler, which would otherwise keep a set of per-lane
     // fragment addresses for each slot
@@ -279,7 +303,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void fwd_bf16_kernel(Core
     else dma_wait();
     __syncthreads();
     if (kb + NSTG - 1 < nkb) issue(kb + NSTG - 1);  // its slot held tile kb - 1
-    if (a.causal && k0 > qw + 31 + off) continue;  // whole tile above this wave's diagonal
+    if (a.causal && k0 > pw1 + off) continue;  // whole tile above this wave's diagonal
 
     f32x16 s[NKT];
 #pragma unroll
@@ -310,7 +334,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void fwd_bf16_kernel(Core
     __builtin_amdgcn_s_setprio(0);
     // the running max is kept in log2 units; as sl2 > 0 it is the max of the raw scores times
     // sl2, and each probability is one fma and one exp2 of a raw score
-    const bool edge = (a.causal && k0 + BN - 1 > qw + off) || (k0 + BN > a.Sk);
+    const bool edge = (a.causal && k0 + BN - 1 > pw0 + off) || (k0 + BN > a.Sk);
     if constexpr (MB) {  // the scores in log2 units with the mask added; the softmax takes them as they are
       if (a.mask_vec) {  // values j = 8 hf .. 8 hf + 7 of tile nt are 8 consecutive keys: one vector read
         const int qc = myq < a.Sq ? myq : a.Sq - 1;
@@ -344,7 +368,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void fwd_bf16_kernel(Core
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
           const int key = k0 + nt * 32 + c_logical<0>(j, g);
-          if (key >= a.Sk || (a.causal && key > myq + off)) s[nt][j] = -INFINITY;
+          if (key >= a.Sk || (a.causal && key > pq + off)) s[nt][j] = -INFINITY;
         }
     }
     float mx = -INFINITY;
@@ -395,6 +419,21 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void fwd_bf16_kernel(Core
   }
 
   const float lt = l + xor32(l);
+  if constexpr (SK) {  // this range's partials; rows past the end are neither written nor read
+    if (myq < a.Sq) {
+      const int64_t row = ((int64_t)(bh * nqb + qb) * a.nsplit + sp) * BM + w * 32 + l32;
+#pragma unroll
+      for (int t = 0; t < NOT; ++t)
+#pragma unroll
+        for (int j = 0; j < 16; j += 4)
+          *(f32x4*)(a.part_o + row * DV + t * 32 + c_row(j, g)) = f32x4{o[t][j], o[t][j + 1], o[t][j + 2], o[t][j + 3]};
+      if (g == 0) {
+        a.part_m[row] = m;
+        a.part_l[row] = lt;
+      }
+    }
+    return;
+  }
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
   __syncthreads();
 #pragma unroll
@@ -512,6 +551,102 @@ int launch_fwd(int dt, int dqk, int dv, const CoreArgs& a, hipStream_t s) {
   if (dt == 0) return fwd_dt<0>(dqk, dv, a, s);
   if (dt == 2) return fwd_dt<2>(dqk, dv, a, s);
   return fwd_dt<1>(dqk, dv, a, s);
+}
+
+
+// One thread per four columns of a query row: the nsplit ranges' partials merged in range order, as
+// decode_merge_kernel does.  `d` gives the output view.
+template <int DV>
+__global__ __launch_bounds__(256) void chunk_merge_kernel(CoreArgs a, DecodeArgs d, int bm, int nqb) {
+  constexpr int TPR = DV / 4;
+  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t grow = gid / TPR;
+  const int c = (int)(gid % TPR) * 4;
+  if (grow >= (int64_t)a.B * a.Hkv * a.Sq) return;
+  const int r = (int)(grow % a.Sq), bh = (int)(grow / a.Sq);
+  const int b = bh / a.Hkv, h = (bh % a.Hkv) * (a.Sq / a.chunk_q) + r / a.chunk_q, qi = r % a.chunk_q;
+  const int64_t row0 = (int64_t)(bh * nqb + r / bm) * a.nsplit * bm + r % bm;
+  // ranges eight at a time, their loads issued together (one at a time, 62 ranges took 30 us)
+  float M = -1e30f, l = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int i0 = 0; i0 < a.nsplit; i0 += 8) {
+    float m[8], pl[8];
+    f32x4 x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int64_t row = row0 + (int64_t)min(i0 + u, a.nsplit - 1) * bm;
+      m[u] = a.part_m[row];
+      pl[u] = a.part_l[row];
+      x[u] = *(const f32x4*)(a.part_o + row * DV + c);
+    }
+    float mn = M;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) mn = fmaxf(mn, m[u]);
+    const float al = exp2f(M - mn);
+    M = mn;
+    l *= al;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] *= al;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const float wt = i0 + u < a.nsplit ? exp2f(m[u] - M) : 0.f;
+      l += pl[u] * wt;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] += x[u][e] * wt;
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const int64_t o0 = b * d.o_sb + h * d.o_sh + (int64_t)qi * d.o_ss + c;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (c + e < d.dv_real) store_from_float(d.o, o0 + e, d.o_dtype, acc[e] * inv);
+  if (c == 0) d.lse[(int64_t)(b * d.Hq + h) * a.chunk_q + qi] = l > 0.f ? (M + log2f(l)) * LN2 : -INFINITY;
+}
+
+// 256-row blocks of eight waves, or 128-row blocks of four where those pad the rows to less; at QK
+// width 256 a 128-row block has its CU to itself (98 KiB of LDS) and leaves half of each SIMD's wave
+// slots empty, so there only rows that fit one of them take it (6000 rows x 4 heads against 16000 cached
+// rows: 492 us in 128-row blocks, 318 us in 256-row blocks).  Then as many key ranges as the CUs hold
+// workgroups at once, each of at least 192 keys (two or three tiles).  Both grow with sk only.
+ChunkPlan chunk_plan(int64_t rows, int64_t heads, int sk, int dqk) {
+  ChunkPlan p;
+  p.bm = (dqk < 256 ? (rows + 127) / 128 * 128 < (rows + 255) / 256 * 256 : rows <= 128) ? 128 : 256;
+  p.nblk = (int)((rows + p.bm - 1) / p.bm);
+  const int64_t slots = p.bm == 128 && dqk < 256 ? 512 : 256, tiles = p.nblk * heads;
+  int64_t n = slots / tiles;
+  n = std::min<int64_t>(n, sk / 192);
+  p.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>(n, 128));
+  return p;
+}
+
+template <int HT, int DQK, int DV>
+static int run_fwd_chunk(const ChunkPlan& cp, const CoreArgs& a, const DecodeArgs& d, hipStream_t s) {
+  const int64_t grid = (int64_t)cp.nblk * cp.nsplit * a.B * a.Hkv;
+  const int64_t mthr = (int64_t)a.B * a.Hkv * a.Sq * (DV / 4);
+  if (grid > 0x7fffffff || (mthr + 255) / 256 > 0x7fffffff) return -2;
+  if (cp.bm == 128)
+    hipLaunchKernelGGL((fwd_bf16_kernel<HT, DQK, DV, 64, 4, 4, 2, false, true>), dim3((unsigned)grid), dim3(256), 0, s, a, 0);
+  else
+    hipLaunchKernelGGL((fwd_bf16_kernel<HT, DQK, DV, 96, 8, 4, 2, false, true>), dim3((unsigned)grid), dim3(512), 0, s, a, 0);
+  hipLaunchKernelGGL((chunk_merge_kernel<DV>), dim3((unsigned)((mthr + 255) / 256)), dim3(256), 0, s, a, d, cp.bm, cp.nblk);
+  return hipGetLastError() == hipSuccess ? 0 : -7;
+}
+
+template <int HT>
+static int chunk_dt(int dqk, int dv, const ChunkPlan& cp, const CoreArgs& a, const DecodeArgs& d, hipStream_t s) {
+  if (dqk == 64 && dv == 64) return run_fwd_chunk<HT, 64, 64>(cp, a, d, s);
+  if (dqk == 64 && dv == 128) return run_fwd_chunk<HT, 64, 128>(cp, a, d, s);
+  if (dqk == 128 && dv == 64) return run_fwd_chunk<HT, 128, 64>(cp, a, d, s);
+  if (dqk == 128 && dv == 128) return run_fwd_chunk<HT, 128, 128>(cp, a, d, s);
+  if (dqk == 256 && dv == 64) return run_fwd_chunk<HT, 256, 64>(cp, a, d, s);
+  if (dqk == 256 && dv == 128) return run_fwd_chunk<HT, 256, 128>(cp, a, d, s);
+  return -3;
+}
+
+int launch_fwd_chunk(int dt, int dqk, int dv, const ChunkPlan& cp, const CoreArgs& a, const DecodeArgs& d, hipStream_t s) {
+  if (dt == 0) return chunk_dt<0>(dqk, dv, cp, a, d, s);
+  if (dt == 2) return chunk_dt<2>(dqk, dv, cp, a, d, s);
+  return -4;
 }
 
 }  // namespace pe

@@ -40,7 +40,8 @@ __host__ __device__ inline int64_t ds_row_base(int r, int e, int nqt, int causal
 // Attention core over transformed operands.
 struct CoreArgs {
   const void* q;    // (B, Hq, Sq, DQK) contiguous, compute dtype
-  const void* k;    // (B, Hkv, Sk, DQK)
+  const void* k;    // (B, Hkv, k_rows, DQK), the first Sk rows of each head (forward; k_rows = Sk elsewhere)
+  int k_rows;
   const void* v;    // (B, Hkv, Sk, DV) rows of v_row elements (>= DV), compute dtype
   int64_t v_sb, v_sh, v_ss;  // element strides of v
   int B, Hq, Hkv, Sq, Sk;
@@ -103,6 +104,12 @@ struct CoreArgs {
   // set by the host when the view takes 8-element vector reads: unit key stride, every other stride
   // a multiple of 8 elements, Sk % 8 == 0 and a 16-byte aligned base (mask_row8)
   int mask_vec;
+  // key-split forward over a KV cache (launch_fwd_chunk): Hq = Hkv and Sq = (query heads per kv head) *
+  // chunk_q rows of one kv head, row r being its query head r / chunk_q, new query r % chunk_q; the key
+  // tiles a 32 NW-row block sees are cut into nsplit ranges, one per workgroup, each leaving its
+  // unnormalised O, running max (log2 units) and row sum in [block][range][32 NW rows] partials
+  int chunk_q, nsplit;
+  float* part_o; float* part_m; float* part_l;
 };
 
 int launch_fwd(int dt, int dqk, int dv, const CoreArgs& a, hipStream_t s);
@@ -186,6 +193,13 @@ struct DecodeArgs {
   const void* qraw; int64_t qr_s[4]; const float* freqs; int Dr, start_pos, pos_round;
 };
 int launch_decode(int dt, int dqk, int dv, const DecodeArgs& a, hipStream_t s);
+// Many new query rows against a cache (a prompt prefilled in chunks), 16-bit operands: the forward
+// kernel over key ranges.  chunk_plan gives the query rows per workgroup and the number of ranges for
+// `rows` query rows of each of `heads` kv heads; launch_fwd_chunk runs the kernel (a: the fields above)
+// and merges the ranges into o / lse through `d`'s output fields.
+struct ChunkPlan { int bm, nblk, nsplit; };
+ChunkPlan chunk_plan(int64_t rows, int64_t heads, int sk, int dqk);
+int launch_fwd_chunk(int dt, int dqk, int dv, const ChunkPlan& cp, const CoreArgs& a, const DecodeArgs& d, hipStream_t s);
 // most query rows per tile that the decode split kernel transforms itself
 constexpr int DECODE_FUSED_ROWS = 8;
 
