@@ -128,6 +128,28 @@ __device__ __forceinline__ void store8(void* p, int64_t i, int dtype, const floa
   }
 }
 
+// 8 consecutive elements of type XT kept as loaded (16 or 32 bytes) until they are used
+template <int XT> struct Raw8 {
+  u32x4 r[XT == 1 ? 2 : 1];
+  __device__ __forceinline__ void load(const void* p, int64_t i) {
+    if constexpr (XT == 1) {
+      r[0] = *(const u32x4*)((const float*)p + i);
+      r[1] = *(const u32x4*)((const float*)p + i + 4);
+    } else {
+      r[0] = *(const u32x4*)((const uint16_t*)p + i);
+    }
+  }
+  __device__ __forceinline__ void get(float (&x)[8]) const {
+    if constexpr (XT == 0) unpack8(r[0], x);
+    else if constexpr (XT == 2) unpack8_h(r[0], x);
+    else {
+      const f32x4 a = __builtin_bit_cast(f32x4, r[0]), b = __builtin_bit_cast(f32x4, r[1]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { x[e] = a[e]; x[e + 4] = b[e]; }
+    }
+  }
+};
+
 // The same accesses inside the 16-bit kernels' epilogues, whose views hold either fp32 (dtype 1) or
 // the kernel's own 16-bit type HT (the host passes nothing else): two cases, chosen at compile time,
 // so the other 16-bit type adds no code to the kernels.

@@ -273,15 +273,19 @@ __global__ __launch_bounds__(RW * 64) void reduce_kernel(ReduceArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Vector forms of prep_kernel (PoPE / FoPE) and prebwd_kernel for bf16 rows with unit inner stride
-// and 16-byte aligned row starts, the layout training hands over.  One thread owns 8 consecutive
-// columns of one row: 16-byte loads and stores, same per-element arithmetic (bitwise identical
-// operands), rows spread over as many threads as there are 8-column chunks.
+// Vector forms of prep_kernel (PoPE / FoPE) and prebwd_kernel for rows with unit inner stride and
+// 16-byte aligned row starts, the layout training hands over.  One thread owns 8 consecutive columns
+// of one row: 16-byte loads and stores, same per-element arithmetic (bitwise identical operands), rows
+// spread over as many threads as there are 8-column chunks.  Built for every element type: the
+// one-wave-per-row forms move 2 or 4 bytes a lane, and an fp16 training step (8 x 12 heads of 64, 1000
+// rows) spent 102 of its 292 us in them; with these it takes 217 us.
 // ---------------------------------------------------------------------------------------------
 // thread t of a row: transform chunk t (cos chunk t, sin chunk t), then content chunks t, t + TPR,
 // ... and zero padding chunks the same way; TPR = Dr / 8
 // tab_out (query side, phases evaluated here): the rows of (b, h) = (0, 0) also write their cos /
-// sin to the [S][2][Dr] phase table, the values launch_phase_table would write
+// sin to the [S][2][Dr] phase table, the values launch_phase_table would write.  XT / DT: element types
+// of the raw positional rows and of the operand rows (the content rows' type is read at run time)
+template <int XT, int DT>
 __device__ __forceinline__ void prep_pope_vec_body(const PrepArgs& a, int64_t gid, float* tab_out = nullptr) {
   const int tpr = a.Dr >> 3;
   const int64_t row = gid / tpr;
@@ -291,8 +295,9 @@ __device__ __forceinline__ void prep_pope_vec_body(const PrepArgs& a, int64_t gi
   const int bh = (int)(row / a.S);
   const int h = bh % a.H, b = bh / a.H;
   const float pos = pe_pos(a.start_pos + s, a.pos_round);
-  uint16_t* drow = (uint16_t*)a.dst + ((int64_t)bh * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s) * a.width;
-  const u32x4 xv = *(const u32x4*)((const uint16_t*)a.xr + b * a.xr_s[0] + h * a.xr_s[1] + (int64_t)s * a.xr_s[2] + t * 8);
+  const int64_t drow = ((int64_t)bh * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s) * a.width;
+  float x[8];
+  load8(a.xr, b * a.xr_s[0] + h * a.xr_s[1] + (int64_t)s * a.xr_s[2] + t * 8, XT, x);
   const f32x4 f0 = *(const f32x4*)(a.freqs + t * 8), f1 = *(const f32x4*)(a.freqs + t * 8 + 4);
   f32x4 d0 = {0.f, 0.f, 0.f, 0.f}, d1 = d0;
   const bool add = a.is_key && a.delta;
@@ -300,8 +305,6 @@ __device__ __forceinline__ void prep_pope_vec_body(const PrepArgs& a, int64_t gi
     d0 = *(const f32x4*)(a.delta + h * a.delta_hs + t * 8);
     d1 = *(const f32x4*)(a.delta + h * a.delta_hs + t * 8 + 4);
   }
-  float x[8];
-  unpack8(xv, x);
   float cv[8], sv[8];
   if (a.tab && !a.is_key) {  // query phases from the table (shared by every batch and head)
     const float* tr = a.tab + (int64_t)s * 2 * a.Dr + t * 8;
@@ -329,16 +332,19 @@ __device__ __forceinline__ void prep_pope_vec_body(const PrepArgs& a, int64_t gi
       }
     }
   }
-  *(u32x4*)(drow + a.Dc + t * 8) =
-      u32x4{pack_bf2(cv[0], cv[1]), pack_bf2(cv[2], cv[3]), pack_bf2(cv[4], cv[5]), pack_bf2(cv[6], cv[7])};
-  *(u32x4*)(drow + a.Dc + a.Dr + t * 8) =
-      u32x4{pack_bf2(sv[0], sv[1]), pack_bf2(sv[2], sv[3]), pack_bf2(sv[4], sv[5]), pack_bf2(sv[6], sv[7])};
+  store8(a.dst, drow + a.Dc + t * 8, DT, cv);
+  store8(a.dst, drow + a.Dc + a.Dr + t * 8, DT, sv);
   if (a.Dc > 0) {
-    const uint16_t* xc = (const uint16_t*)a.xc + b * a.xc_s[0] + h * a.xc_s[1] + (int64_t)s * a.xc_s[2];
-    for (int j = t; j < a.Dc / 8; j += tpr) *(u32x4*)(drow + j * 8) = *(const u32x4*)(xc + j * 8);
+    const int64_t xc0 = b * a.xc_s[0] + h * a.xc_s[1] + (int64_t)s * a.xc_s[2];
+    for (int j = t; j < a.Dc / 8; j += tpr) {
+      float c[8];
+      load8(a.xc, xc0 + j * 8, a.xc_dtype, c);
+      store8(a.dst, drow + j * 8, DT, c);
+    }
   }
-  for (int j = (a.Dc + 2 * a.Dr) / 8 + t; j < a.width / 8; j += tpr) *(u32x4*)(drow + j * 8) = u32x4{0u, 0u, 0u, 0u};
-  if (a.cdst) {  // the row's companion copy (KV-cache append: the value row)
+  const float zero[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int j = (a.Dc + 2 * a.Dr) / 8 + t; j < a.width / 8; j += tpr) store8(a.dst, drow + j * 8, DT, zero);
+  if (a.cdst) {  // the row's companion copy (KV-cache append: the value row), 16-bit elements
     const uint16_t* crow = (const uint16_t*)a.cv + b * a.cv_s[0] + h * a.cv_s[1] + (int64_t)s * a.cv_s[2];
     uint16_t* cd = (uint16_t*)a.cdst + ((int64_t)bh * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s) * a.cwidth;
     for (int j = t; j < a.cwidth / 8; j += tpr)
@@ -346,8 +352,8 @@ __device__ __forceinline__ void prep_pope_vec_body(const PrepArgs& a, int64_t gi
   }
 }
 
-__global__ __launch_bounds__(256) void prep_pope_vec_kernel(PrepArgs a) {
-  prep_pope_vec_body(a, (int64_t)blockIdx.x * 256 + threadIdx.x);
+template <int XT, int DT> __global__ __launch_bounds__(256) void prep_pope_vec_kernel(PrepArgs a) {
+  prep_pope_vec_body<XT, DT>(a, (int64_t)blockIdx.x * 256 + threadIdx.x);
 }
 
 // The same key-side work for a few rows (a decoded token's cache append): one thread per
@@ -356,7 +362,7 @@ __global__ __launch_bounds__(256) void prep_pope_vec_kernel(PrepArgs a) {
 // body's, so the rows are bitwise the same.  Threads past the elements copy or clear one 16-byte
 // chunk each: the content part, the operand row's zero padding and the companion value row.
 constexpr int64_t PREP_SMALL_ELEMS = 8192;  // rows x Dr at most, for this path
-__global__ __launch_bounds__(256) void prep_pope_small_kernel(PrepArgs a) {
+template <int HT> __global__ __launch_bounds__(256) void prep_pope_small_kernel(PrepArgs a) {
   const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t nrows = (int64_t)a.B * a.H * a.S, nel = nrows * a.Dr;
   const int ncc = a.Dc / 8, npad = (a.width - a.Dc - 2 * a.Dr) / 8, nval = a.cdst ? a.cwidth / 8 : 0;
@@ -369,13 +375,12 @@ __global__ __launch_bounds__(256) void prep_pope_small_kernel(PrepArgs a) {
   uint16_t* drow = (uint16_t*)a.dst + orow * a.width;
   if (gid < nel) {
     const int d = (int)(gid - row * a.Dr);
-    const uint16_t raw = ((const uint16_t*)a.xr)[b * a.xr_s[0] + h * a.xr_s[1] + (int64_t)s * a.xr_s[2] + d];
-    const float mu = softplus_f(__builtin_bit_cast(float, (uint32_t)raw << 16));
+    const float mu = softplus_f(load_as_float_t<HT>(a.xr, b * a.xr_s[0] + h * a.xr_s[1] + (int64_t)s * a.xr_s[2] + d, HT));
     float ph = mul_nc(pe_pos(a.start_pos + s, a.pos_round), a.freqs[d]);
     if (a.delta) ph = add_nc(ph, a.delta[h * a.delta_hs + d]);
     float sn, cs;
     pe_sincos(ph, sn, cs);
-    const uint32_t pr = pack_bf2(mul_nc(mu, cs), mul_nc(mu, sn));
+    const uint32_t pr = pack2<HT>(mul_nc(mu, cs), mul_nc(mu, sn));
     drow[a.Dc + d] = (uint16_t)pr;
     drow[a.Dc + a.Dr + d] = (uint16_t)(pr >> 16);
     return;
@@ -395,8 +400,8 @@ __global__ __launch_bounds__(256) void prep_pope_small_kernel(PrepArgs a) {
 }
 
 // one group of TPR = Dv / 8 lanes per padded row (TPR a power of two, groups never straddle a
-// wave); Di is the group's fixed-order butterfly sum
-__global__ __launch_bounds__(256) void prebwd_vec_kernel(PreBwdArgs a, int lg_tpr) {
+// wave); Di is the group's fixed-order butterfly sum.  XT: the element type of dO and out
+template <int XT> __global__ __launch_bounds__(256) void prebwd_vec_kernel(PreBwdArgs a, int lg_tpr) {
   const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t prow = gid >> lg_tpr;
   const int t = (int)(gid & ((1 << lg_tpr) - 1));
@@ -409,12 +414,10 @@ __global__ __launch_bounds__(256) void prebwd_vec_kernel(PreBwdArgs a, int lg_tp
   }
   const int h = bh % a.H, b = bh / a.H;
   const int64_t row = (int64_t)bh * a.S + s;
-  const u32x4 dv = *(const u32x4*)((const uint16_t*)a.dout + b * a.do_s[0] + h * a.do_s[1] + (int64_t)s * a.do_s[2] + t * 8);
-  const u32x4 ov = *(const u32x4*)((const uint16_t*)a.out + b * a.o_s[0] + h * a.o_s[1] + (int64_t)s * a.o_s[2] + t * 8);
-  if (a.dO_op) *(u32x4*)((uint16_t*)a.dO_op + row * a.width + t * 8) = dv;
   float d[8], o[8];
-  unpack8(dv, d);
-  unpack8(ov, o);
+  load8(a.dout, b * a.do_s[0] + h * a.do_s[1] + (int64_t)s * a.do_s[2] + t * 8, XT, d);
+  load8(a.out, b * a.o_s[0] + h * a.o_s[1] + (int64_t)s * a.o_s[2] + t * 8, XT, o);
+  if (a.dO_op) store8(a.dO_op, row * a.width + t * 8, XT, d);
   float acc = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc += d[e] * o[e];
@@ -500,7 +503,7 @@ __global__ __launch_bounds__(256) void inv_rope_vec_kernel(InvArgs a, int lg_tpr
   store8(a.dxr, b * a.dxr_s[0] + h * a.dxr_s[1] + (int64_t)s * a.dxr_s[2] + t * 8, a.dxr_dtype, dx);
 }
 
-bool aligned16(const void* p, int64_t s0, int64_t s1, int64_t s2) {
+static bool aligned16(const void* p, int64_t s0, int64_t s1, int64_t s2) {
   return ((uintptr_t)p % 16) == 0 && s0 % 8 == 0 && s1 % 8 == 0 && s2 % 8 == 0;
 }
 
@@ -538,35 +541,58 @@ static int inv_rope_vec_lg(const InvArgs& a) {
   return lg;
 }
 
+// element types the vectorised PoPE prologue is built for: raw rows and operands of one type, and fp32
+// rows (RMS-normed projections under autocast) into 16-bit operands; -1 for any other pair
+static int prep_vec_types(int xt, int dt) {
+  if (xt == dt && dt >= 0 && dt <= 2) return dt;
+  return xt == 1 ? (dt == 0 ? 3 : dt == 2 ? 4 : -1) : -1;
+}
+// calls f with the raw and operand element types of prep_vec_types' pair as compile-time constants
+template <typename F> static void with_prep_types(int pair, F&& f) {
+  switch (pair) {
+    case 0: f(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}); break;
+    case 1: f(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{}); break;
+    case 3: f(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{}); break;
+    default: f(std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{}); break;
+  }
+}
+static int prep_vec_types(const PrepArgs& a) { return prep_vec_types(a.xr_dtype, a.dst_dtype); }
+
 static bool prep_vec_ok(const PrepArgs& a) {
-  return a.mode == 0 && a.dst_dtype == 0 && a.xr_dtype == 0 && a.Dr > 0 && a.Dr % 8 == 0 &&
-         a.Dc % 8 == 0 && a.width % 8 == 0 && a.xr_s[3] == 1 &&
-         aligned16(a.xr, a.xr_s[0], a.xr_s[1], a.xr_s[2]) && ((uintptr_t)a.dst % 16) == 0 &&
-         ((uintptr_t)a.freqs % 16) == 0 &&
+  return a.mode == 0 && prep_vec_types(a) >= 0 && a.Dr > 0 && a.Dr % 8 == 0 && a.Dc % 8 == 0 && a.width % 8 == 0 &&
+         rows16(a.xr, a.xr_dtype, a.xr_s) && ((uintptr_t)a.dst % 16) == 0 && ((uintptr_t)a.freqs % 16) == 0 &&
          (!a.is_key || !a.delta || (((uintptr_t)a.delta % 16) == 0 && a.delta_hs % 4 == 0)) &&
-         (a.Dc == 0 || (a.xc_dtype == 0 && a.xc_s[3] == 1 && aligned16(a.xc, a.xc_s[0], a.xc_s[1], a.xc_s[2])));
+         (a.Dc == 0 || rows16(a.xc, a.xc_dtype, a.xc_s));
 }
 
 bool prep_vec_copy_ok(const PrepArgs& a) {
-  return prep_vec_ok(a) && a.cv && a.cdst && a.cv_s[3] == 1 && aligned16(a.cv, a.cv_s[0], a.cv_s[1], a.cv_s[2]) &&
+  return prep_vec_ok(a) && a.dst_dtype != 1 && a.cv && a.cdst && a.cv_s[3] == 1 && aligned16(a.cv, a.cv_s[0], a.cv_s[1], a.cv_s[2]) &&
          ((uintptr_t)a.cdst % 16) == 0 && a.cv_cols % 8 == 0 && a.cwidth % 8 == 0 && a.cv_cols <= a.cwidth;
 }
 
 bool prep_vec_query_ok(const PrepArgs& a) {
-  return prep_vec_ok(a) && !a.is_key && a.Dc == 0 && a.width == 2 * a.Dr;
+  return prep_vec_ok(a) && a.xr_dtype == a.dst_dtype && a.dst_dtype != 1 && !a.is_key && a.Dc == 0 &&
+         a.width == 2 * a.Dr;
 }
 
 int launch_prep(const PrepArgs& a, hipStream_t s) {
   const int64_t nrows = (int64_t)a.B * a.H * a.S;
   const bool vec = prep_vec_ok(a);
   if (a.cdst && !(vec && prep_vec_copy_ok(a))) return -2;  // the caller checks prep_vec_copy_ok first
-  if (vec && a.is_key && nrows * a.Dr <= PREP_SMALL_ELEMS) {
+  if (vec && a.is_key && a.dst_dtype != 1 && a.xr_dtype == a.dst_dtype && (a.Dc == 0 || a.xc_dtype == a.dst_dtype) &&
+      nrows * a.Dr <= PREP_SMALL_ELEMS) {
     const int64_t nch = a.Dc / 8 + (a.width - a.Dc - 2 * a.Dr) / 8 + (a.cdst ? a.cwidth / 8 : 0);
     const int64_t nthr = nrows * (a.Dr + nch);
-    hipLaunchKernelGGL(prep_pope_small_kernel, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, s, a);
+    const dim3 grid((unsigned)((nthr + 255) / 256));
+    if (a.dst_dtype == 0) hipLaunchKernelGGL(prep_pope_small_kernel<0>, grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(prep_pope_small_kernel<2>, grid, dim3(256), 0, s, a);
   } else if (vec) {
     const int64_t nthr = nrows * (a.Dr / 8);
-    hipLaunchKernelGGL(prep_pope_vec_kernel, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, s, a);
+    with_prep_types(prep_vec_types(a), [&](auto xt, auto dt) {
+      hipLaunchKernelGGL((prep_pope_vec_kernel<decltype(xt)::value, decltype(dt)::value>),
+                         dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, s, a);
+    });
   } else if (const int lg = prep_rope_vec_lg(a); lg >= 0) {
     const int64_t nthr = nrows << lg;
     hipLaunchKernelGGL(prep_rope_vec_kernel, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, s, a, lg);
@@ -593,9 +619,10 @@ __global__ __launch_bounds__(256) void phase_table_kernel(const float* freqs, in
 
 // the key prologue (vectorised path) and the query phase table in one launch: blocks below nblk
 // transform key rows, the rest write the table; the two share no data
+template <int XT, int DT>
 __global__ __launch_bounds__(256) void prep_vec_and_table_kernel(PrepArgs a, unsigned nblk, const float* freqs,
                                                                  int start, int S, int Dr, int pos_round, float* tab) {
-  if (blockIdx.x < nblk) prep_pope_vec_body(a, (int64_t)blockIdx.x * 256 + threadIdx.x);
+  if (blockIdx.x < nblk) prep_pope_vec_body<XT, DT>(a, (int64_t)blockIdx.x * 256 + threadIdx.x);
   else phase_table_body(freqs, start, S, Dr, pos_round, tab, (int64_t)(blockIdx.x - nblk) * 256 + threadIdx.x);
 }
 
@@ -603,9 +630,10 @@ __global__ __launch_bounds__(256) void prep_vec_and_table_kernel(PrepArgs a, uns
 // query rows, which evaluate their own phases (no table to wait for) and, in the rows of (0, 0),
 // write the phase table.  The per-element arithmetic is the two-launch path's, so every value is
 // bitwise the same.
+template <int XT, int DT>
 __global__ __launch_bounds__(256) void prep_qk_vec_kernel(PrepArgs ak, PrepArgs aq, unsigned nkblk, float* tab) {
-  if (blockIdx.x < nkblk) prep_pope_vec_body(ak, (int64_t)blockIdx.x * 256 + threadIdx.x);
-  else prep_pope_vec_body(aq, (int64_t)(blockIdx.x - nkblk) * 256 + threadIdx.x, tab);
+  if (blockIdx.x < nkblk) prep_pope_vec_body<XT, DT>(ak, (int64_t)blockIdx.x * 256 + threadIdx.x);
+  else prep_pope_vec_body<XT, DT>(aq, (int64_t)(blockIdx.x - nkblk) * 256 + threadIdx.x, tab);
 }
 
 // Query rows without a content part or padding, QHG heads per thread: thread (b, head group, s,
@@ -616,6 +644,7 @@ __global__ __launch_bounds__(256) void prep_qk_vec_kernel(PrepArgs ak, PrepArgs 
 // Per element the arithmetic is prep_pope_vec_body's, so the rows and the table are bitwise those
 // of the table launch plus the table-reading query launch.
 constexpr int QHG = 8;
+template <int XT, int DT>
 __device__ __forceinline__ void prep_pope_qheads_body(const PrepArgs& a, int64_t gid, float* tab) {
   const int tpr = a.Dr >> 3, ngrp = (a.H + QHG - 1) / QHG;
   const int64_t unit = gid / tpr;
@@ -624,11 +653,11 @@ __device__ __forceinline__ void prep_pope_qheads_body(const PrepArgs& a, int64_t
   const int s = (int)(unit % a.S);
   const int64_t bg = unit / a.S;
   const int hg = (int)(bg % ngrp), b = (int)(bg / ngrp), h0 = hg * QHG;
-  const uint16_t* xb = (const uint16_t*)a.xr + b * a.xr_s[0] + (int64_t)s * a.xr_s[2] + t * 8;
-  u32x4 xv[QHG];
+  const int64_t xb = b * a.xr_s[0] + (int64_t)s * a.xr_s[2] + t * 8;
+  Raw8<XT> xv[QHG];
 #pragma unroll
   for (int j = 0; j < QHG; ++j)
-    if (h0 + j < a.H) xv[j] = *(const u32x4*)(xb + (int64_t)(h0 + j) * a.xr_s[1]);
+    if (h0 + j < a.H) xv[j].load(a.xr, xb + (int64_t)(h0 + j) * a.xr_s[1]);
   const float pos = pe_pos(a.start_pos + s, a.pos_round);
   const f32x4 f0 = *(const f32x4*)(a.freqs + t * 8), f1 = *(const f32x4*)(a.freqs + t * 8 + 4);
   float cs[8], sn[8];
@@ -646,18 +675,16 @@ __device__ __forceinline__ void prep_pope_qheads_body(const PrepArgs& a, int64_t
     const int h = h0 + j;
     if (h >= a.H) break;
     float x[8], cv[8], sv[8];
-    unpack8(xv[j], x);
+    xv[j].get(x);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float mu = softplus_f(x[e]);
       cv[e] = mul_nc(mu, cs[e]);
       sv[e] = mul_nc(mu, sn[e]);
     }
-    uint16_t* drow = (uint16_t*)a.dst + ((int64_t)(b * a.H + h) * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s) * a.width;
-    *(u32x4*)(drow + t * 8) =
-        u32x4{pack_bf2(cv[0], cv[1]), pack_bf2(cv[2], cv[3]), pack_bf2(cv[4], cv[5]), pack_bf2(cv[6], cv[7])};
-    *(u32x4*)(drow + a.Dr + t * 8) =
-        u32x4{pack_bf2(sv[0], sv[1]), pack_bf2(sv[2], sv[3]), pack_bf2(sv[4], sv[5]), pack_bf2(sv[6], sv[7])};
+    const int64_t drow = ((int64_t)(b * a.H + h) * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s) * a.width;
+    store8(a.dst, drow + t * 8, DT, cv);
+    store8(a.dst, drow + a.Dr + t * 8, DT, sv);
   }
 }
 
@@ -666,12 +693,13 @@ __device__ __forceinline__ void prep_pope_qheads_body(const PrepArgs& a, int64_t
 // softplus per element, phases shared over QHG heads), so that both kinds share every CU.  Block i
 // is the query block cq(i) = floor(i * nqblk / n) when cq(i + 1) > cq(i), else the key block
 // i - cq(i); over the n = nkblk + nqblk blocks this takes each index of either kind once.
+template <int XT, int DT>
 __global__ __launch_bounds__(256) void prep_k_qheads_kernel(PrepArgs ak, PrepArgs aq, unsigned nkblk, unsigned nqblk,
                                                             float* tab) {
   const uint64_t i = blockIdx.x, n = (uint64_t)nkblk + nqblk;
   const uint64_t cq = i * nqblk / n, cq1 = (i + 1) * nqblk / n;
-  if (cq1 > cq) prep_pope_qheads_body(aq, (int64_t)cq * 256 + threadIdx.x, tab);
-  else prep_pope_vec_body(ak, (int64_t)(i - cq) * 256 + threadIdx.x);
+  if (cq1 > cq) prep_pope_qheads_body<XT, DT>(aq, (int64_t)cq * 256 + threadIdx.x, tab);
+  else prep_pope_vec_body<XT, DT>(ak, (int64_t)(i - cq) * 256 + threadIdx.x);
 }
 
 // prologues of at most this many 256-thread blocks (keys and queries together) take one launch:
@@ -679,7 +707,8 @@ __global__ __launch_bounds__(256) void prep_k_qheads_kernel(PrepArgs ak, PrepArg
 constexpr int64_t PREP_QK_MAX_BLOCKS = 1024;
 
 int launch_prep_k_qheads(const PrepArgs& ak, const PrepArgs& aq, float* tab, hipStream_t s) {
-  if (!prep_vec_ok(ak) || !prep_vec_query_ok(aq) || ak.cdst || aq.cdst || aq.tab || !ak.is_key || aq.Dr != ak.Dr ||
+  if (!prep_vec_ok(ak) || !prep_vec_ok(aq) || prep_vec_types(ak) != prep_vec_types(aq) || aq.is_key || aq.Dc != 0 ||
+      aq.width != 2 * aq.Dr || ak.cdst || aq.cdst || aq.tab || !ak.is_key || aq.Dr != ak.Dr ||
       !tab || (uintptr_t)tab % 16 != 0)
     return 1;
   const int64_t nk = (int64_t)ak.B * ak.H * ak.S * (ak.Dr / 8);
@@ -687,20 +716,24 @@ int launch_prep_k_qheads(const PrepArgs& ak, const PrepArgs& aq, float* tab, hip
   const int64_t nkblk = (nk + 255) / 256, nqblk = (nq + 255) / 256;
   if (nk == 0 || nq == 0) return 1;
   if (nkblk + nqblk > 0x7fffffff) return -2;
-  hipLaunchKernelGGL(prep_k_qheads_kernel, dim3((unsigned)(nkblk + nqblk)), dim3(256), 0, s, ak, aq, (unsigned)nkblk,
-                     (unsigned)nqblk, tab);
+  with_prep_types(prep_vec_types(ak), [&](auto xt, auto dt) {
+    hipLaunchKernelGGL((prep_k_qheads_kernel<decltype(xt)::value, decltype(dt)::value>), dim3((unsigned)(nkblk + nqblk)),
+                       dim3(256), 0, s, ak, aq, (unsigned)nkblk, (unsigned)nqblk, tab);
+  });
   return hipGetLastError() == hipSuccess ? 0 : -7;
 }
 
 int launch_prep_qk(const PrepArgs& ak, const PrepArgs& aq, float* tab, hipStream_t s) {
-  if (!prep_vec_ok(ak) || !prep_vec_ok(aq) || ak.cdst || aq.cdst || aq.tab || !ak.is_key || aq.is_key ||
-      aq.Dr != ak.Dr)
+  if (!prep_vec_ok(ak) || !prep_vec_ok(aq) || prep_vec_types(ak) != prep_vec_types(aq) || ak.cdst || aq.cdst ||
+      aq.tab || !ak.is_key || aq.is_key || aq.Dr != ak.Dr)
     return 1;
   const int64_t nk = (int64_t)ak.B * ak.H * ak.S * (ak.Dr / 8), nq = (int64_t)aq.B * aq.H * aq.S * (aq.Dr / 8);
   const int64_t nkblk = (nk + 255) / 256, nqblk = (nq + 255) / 256;
   if (nkblk + nqblk > PREP_QK_MAX_BLOCKS || nk * 8 <= PREP_SMALL_ELEMS || nk == 0 || nq == 0) return 1;
-  hipLaunchKernelGGL(prep_qk_vec_kernel, dim3((unsigned)(nkblk + nqblk)), dim3(256), 0, s, ak, aq, (unsigned)nkblk,
-                     tab);
+  with_prep_types(prep_vec_types(ak), [&](auto xt, auto dt) {
+    hipLaunchKernelGGL((prep_qk_vec_kernel<decltype(xt)::value, decltype(dt)::value>), dim3((unsigned)(nkblk + nqblk)),
+                       dim3(256), 0, s, ak, aq, (unsigned)nkblk, tab);
+  });
   return hipGetLastError() == hipSuccess ? 0 : -7;
 }
 
@@ -714,8 +747,10 @@ int launch_prep_and_table(const PrepArgs& a, const float* freqs, int start, int 
   }
   const int64_t nblk = (nrows * (a.Dr / 8) + 255) / 256, ntab = (nt + 255) / 256;
   if (nblk + ntab > 0x7fffffff) return -2;
-  hipLaunchKernelGGL(prep_vec_and_table_kernel, dim3((unsigned)(nblk + ntab)), dim3(256), 0, s, a, (unsigned)nblk,
-                     freqs, start, S, Dr, pos_round, tab);
+  with_prep_types(prep_vec_types(a), [&](auto xt, auto dt) {
+    hipLaunchKernelGGL((prep_vec_and_table_kernel<decltype(xt)::value, decltype(dt)::value>), dim3((unsigned)(nblk + ntab)),
+                       dim3(256), 0, s, a, (unsigned)nblk, freqs, start, S, Dr, pos_round, tab);
+  });
   return hipGetLastError() == hipSuccess ? 0 : -7;
 }
 
@@ -729,15 +764,17 @@ int launch_phase_table(const float* freqs, int start, int S, int Dr, int pos_rou
 
 int launch_prebwd(const PreBwdArgs& a, hipStream_t s) {
   const int tpr = a.Dv / 8;
-  const bool vec = a.dout_dtype == 0 && a.out_dtype == 0 && a.Dv % 8 == 0 && tpr <= 64 && (tpr & (tpr - 1)) == 0 &&
-                   a.do_s[3] == 1 && a.o_s[3] == 1 && aligned16(a.dout, a.do_s[0], a.do_s[1], a.do_s[2]) &&
-                   aligned16(a.out, a.o_s[0], a.o_s[1], a.o_s[2]) &&
-                   (!a.dO_op || (a.op_dtype == 0 && a.width == a.Dv && ((uintptr_t)a.dO_op % 16) == 0));
+  const bool vec = a.dout_dtype == a.out_dtype && a.Dv % 8 == 0 && tpr <= 64 && (tpr & (tpr - 1)) == 0 &&
+                   rows16(a.dout, a.dout_dtype, a.do_s) && rows16(a.out, a.out_dtype, a.o_s) &&
+                   (!a.dO_op || (a.op_dtype == a.dout_dtype && a.width == a.Dv && ((uintptr_t)a.dO_op % 16) == 0));
   const int64_t nrows = (int64_t)a.B * a.H * a.s_pad;
   if (vec) {
     int lg = 0;
     while ((1 << lg) < tpr) ++lg;
-    hipLaunchKernelGGL(prebwd_vec_kernel, dim3((unsigned)((nrows * tpr + 255) / 256)), dim3(256), 0, s, a, lg);
+    const dim3 grid((unsigned)((nrows * tpr + 255) / 256));
+    if (a.dout_dtype == 0) hipLaunchKernelGGL(prebwd_vec_kernel<0>, grid, dim3(256), 0, s, a, lg);
+    else if (a.dout_dtype == 2) hipLaunchKernelGGL(prebwd_vec_kernel<2>, grid, dim3(256), 0, s, a, lg);
+    else hipLaunchKernelGGL(prebwd_vec_kernel<1>, grid, dim3(256), 0, s, a, lg);
   } else {
     hipLaunchKernelGGL(prebwd_kernel, dim3((unsigned)((nrows + 3) / 4)), dim3(256), 0, s, a);
   }
