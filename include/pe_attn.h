@@ -205,7 +205,9 @@ typedef struct {
  * (under the HIP runtime's default deferred loading: the first call of this entry on that GPU) to
  * process exit).  No counterpart in the reference: it is for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  Calls whose
- * forward workspace (pe_attn_fwd_workspace_bytes) exceeds the scratch return PE_ERR_SCRATCH_LIMIT.
+ * forward workspace (pe_attn_fwd_workspace_bytes) exceeds the scratch return PE_ERR_SCRATCH_LIMIT,
+ * except fp32 ones that fit with fp32 operands (two thirds of that workspace): those run on the fp32
+ * matrix unit, slower and with its rounding.
  * All calls on one GPU share its scratch: calls that overlap in time on one GPU (different streams
  * or threads) race and must be serialised by the caller.  Outputs are as for pe_attn_fwd; the
  * scratch cannot serve pe_attn_bwd (use pe_attn_fwd with a caller workspace for training). */

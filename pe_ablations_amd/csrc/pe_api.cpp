@@ -38,6 +38,7 @@ bool valid_dt(int dtype) { return dtype == PE_DTYPE_BF16 || dtype == PE_DTYPE_FP
 
 struct Layout {
   int dqk, dv;
+  bool split;  // fp32 compute with its operands as three bf16 planes (pe_split.hip)
   size_t q_off, k_off, v_off, tab_off, fwd_total;
   size_t do_off, di_off, l2_off, dq_off, dk_off, pq_off, pk_off, pkd_off, dvp_off, ds_off, bwd_total;
   int ksplit;    // query-head split of the dK/dV pair kernel (pe::CoreArgs::qsplit)
@@ -75,6 +76,18 @@ int key_split(const pe_attn_params* p, int dqk, int dv) {
   return ks;
 }
 
+// Ranges that the split backward (pe_split.hip) cuts each 128-key block's list of (query head, query tile)
+// into: doubled up to 4 while the key blocks give fewer workgroups than two per compute unit and the first
+// block keeps at least eight tiles a range (4 x 8 -> 4 heads, 1024 rows, 128 key blocks, the longest of 64
+// tiles: see split_sum_kernel).  `batch` 1: the ranges that the workspace reserves, whatever the batch.
+int split_ranges(const pe_attn_params* p, int batch) {
+  const int64_t blocks = (int64_t)batch * p->Hkv * ((p->Sk + 127) / 128);
+  const int tiles = p->Hq / p->Hkv * ((p->Sq + 31) / 32);
+  int n = 1;
+  while (n < 4 && blocks * n < 2 * kSplitCus && tiles / (2 * n) >= 8) n *= 2;
+  return n;
+}
+
 // a view the vectorised epilogues can read or write 8 elements at a time: unit dim stride and
 // every row 16-byte aligned
 bool vec16(const pe_tensor_t* t) {
@@ -102,17 +115,20 @@ bool generic_masked(const pe_attn_params* p, bool masked) {
   return masked && !(half_dt(p->dtype) && pe::pair_shape(pad_qk(qk_width(p)), pad_v(p->Dv)));
 }
 
-Layout layout(const pe_attn_params* p, bool masked = false) {
+// unit: an fp32 forward whose operands stay fp32, for the fp32 matrix unit (as an explicit mask's do)
+Layout layout(const pe_attn_params* p, bool masked = false, bool unit = false) {
   Layout L{};
   L.dqk = pad_qk(qk_width(p));
   L.dv = pad_v(p->Dv);
   const bool gm = generic_masked(p, masked);
   const size_t e = esz(p);
+  L.split = p->dtype == PE_DTYPE_FP32 && !masked && !unit;
+  const size_t oe = L.split ? 6 : e;  // bytes of an operand element
   const size_t nq = (size_t)p->B * p->Hq * p->Sq, nk = (size_t)p->B * p->Hkv * p->Sk;
   L.q_off = 0;
-  L.k_off = L.q_off + align_up(nq * L.dqk * e);
-  L.v_off = L.k_off + align_up(nk * L.dqk * e);
-  L.tab_off = L.v_off + align_up(nk * L.dv * e);
+  L.k_off = L.q_off + align_up(nq * L.dqk * oe);
+  L.v_off = L.k_off + align_up(nk * L.dqk * oe);
+  L.tab_off = L.v_off + align_up(nk * L.dv * oe);
   // query phase table (cos / sin of fl(pos * freq), fp32 [Sq][2][Dr]) for the PoPE prologue and the
   // dQ epilogue
   L.fwd_total = L.tab_off + (use_qtab(p) ? align_up((size_t)p->Sq * 2 * p->Dr * 4) : 0);
@@ -125,18 +141,23 @@ Layout layout(const pe_attn_params* p, bool masked = false) {
   L.do_off = 0;
   L.sq_pad = (p->Sq + 127) / 128 * 128;
   const size_t nq_pad = (size_t)p->B * p->Hq * L.sq_pad;
-  L.di_off = L.do_off + align_up(nq * L.dv * e);
+  L.di_off = L.do_off + align_up(nq * L.dv * oe);
   L.l2_off = L.di_off + align_up(nq_pad * 4);
   L.dq_off = L.l2_off + align_up(nq_pad * 4);
   const bool fb = !gm && fused_bwd(p);
   L.ksplit = masked ? 1 : key_split(p, L.dqk, L.dv);
+  int slices = L.ksplit;
+  if (L.split) {
+    L.ksplit = split_ranges(p, p->B);
+    slices = split_ranges(p, 1);
+  }
   L.dk_off = L.dq_off + (fb ? 0 : align_up(nq * L.dqk * 4));
   // dk~ (unfused) or the split's partial dk~ slices
-  L.pq_off = L.dk_off + (fb && L.ksplit == 1 ? 0 : align_up(nk * L.dqk * 4 * L.ksplit));
+  L.pq_off = L.dk_off + (fb && slices == 1 ? 0 : align_up(nk * L.dqk * 4 * slices));
   L.pk_off = L.pq_off + align_up((size_t)L.nq_blocks * p->Dr * 4);
   L.pkd_off = L.pk_off + align_up((size_t)L.nk_blocks * p->Dr * 4);
   L.dvp_off = L.pkd_off + align_up((size_t)L.nk_blocks * p->Dr * 4);
-  L.ds_off = L.dvp_off + (L.ksplit > 1 ? align_up(nk * L.dv * 4 * L.ksplit) : 0);
+  L.ds_off = L.dvp_off + (slices > 1 ? align_up(nk * L.dv * 4 * slices) : 0);
   // bf16 path: dS in fragment order, 4 KiB blocks packed per (b, h) to the blocks the causal
   // dK/dV kernel stores (pe::ds_row_base), written by it for the dQ GEMM.  The dQ GEMM's masked
   // edge steps also load up to four blocks before a key row's first stored one; those lie in the
@@ -260,7 +281,9 @@ pe::CoreArgs core_args(const pe_attn_params* p, const Layout& L, const char* ws,
   c.q = ws + L.q_off;
   c.k = ws + L.k_off;
   c.k_rows = p->Sk;
-  if (v_direct(p, v, L.dv)) {
+  if (L.split) {
+    c.v = ws + L.v_off;  // rows of three planes
+  } else if (v_direct(p, v, L.dv)) {
     c.v = v->data; c.v_sb = v->stride[0]; c.v_sh = v->stride[1]; c.v_ss = v->stride[2];
   } else {
     c.v = ws + L.v_off; c.v_ss = L.dv; c.v_sh = (int64_t)p->Sk * L.dv; c.v_sb = (int64_t)p->Hkv * p->Sk * L.dv;
@@ -422,7 +445,8 @@ int pe_attn_transform_bwd(const pe_attn_params* p, int is_key, const float* g, c
 static int fwd_impl(const pe_attn_params* p, const pe_norm_params* nrm, const pe_tensor_t* qc,
                     const pe_tensor_t* qr, const pe_tensor_t* kc, const pe_tensor_t* kr, const pe_tensor_t* v,
                     const float* freqs, const float* delta, const pe_tensor_t* out, float* lse,
-                    void* fwd_workspace, size_t fwd_ws_bytes, void* stream, const pe_tensor_t* mask = nullptr) {
+                    void* fwd_workspace, size_t fwd_ws_bytes, void* stream, const pe_tensor_t* mask = nullptr,
+                    bool unit = false) {
   int rc = pe_attn_check(p);
   if (rc) return rc;
   if (mask && (rc = check_mask(mask))) return rc;
@@ -437,7 +461,8 @@ static int fwd_impl(const pe_attn_params* p, const pe_norm_params* nrm, const pe
     return rc;
   if (!lse || (p->mode != PE_MODE_NONE && p->Dr > 0 && !freqs)) return PE_ERR_NULL;
   if (out->dtype != p->dtype) return PE_ERR_MODE;
-  const Layout L = layout(p);
+  const Layout L = layout(p, mask != nullptr, unit);
+  const int opd = L.split ? pe::DT_SPLIT_CODE : p->dtype;  // element type of the operand rows
   if (!fwd_workspace || fwd_ws_bytes < L.fwd_total) return PE_ERR_WORKSPACE;
   if ((rc = device_ok())) return rc;
   hipStream_t s = (hipStream_t)stream;
@@ -450,10 +475,12 @@ static int fwd_impl(const pe_attn_params* p, const pe_norm_params* nrm, const pe
     if (qtab && (rc = pe::launch_phase_table(freqs, p->start_pos_q, p->Sq, p->Dr, p->position_rounding, qtab, s)))
       return rc;
     fill_prep(a, p, 0, qc, qr, freqs, nullptr, ws + L.q_off, L.dqk);
+    a.dst_dtype = opd;
     a.tab = qtab;
     a.norm_w = nrm->q_weight; a.norm_w_dtype = nrm->weight_dtype; a.norm_eps = nrm->eps;
     if ((rc = pe::launch_prep_norm(a, s))) return rc;
     fill_prep(a, p, 1, kc, kr, freqs, delta, ws + L.k_off, L.dqk);
+    a.dst_dtype = opd;
     a.norm_w = nrm->k_weight; a.norm_w_dtype = nrm->weight_dtype; a.norm_eps = nrm->eps;
     if ((rc = pe::launch_prep_norm(a, s))) return rc;
   } else {
@@ -463,6 +490,7 @@ static int fwd_impl(const pe_attn_params* p, const pe_norm_params* nrm, const pe
     fill_prep(a, p, 1, kc, kr, freqs, delta, ws + L.k_off, L.dqk);
     pe::PrepArgs aq;
     fill_prep(aq, p, 0, qc, qr, freqs, nullptr, ws + L.q_off, L.dqk);
+    a.dst_dtype = aq.dst_dtype = opd;
     rc = qtab ? pe::launch_prep_qk(a, aq, qtab, s) : 1;
     if (rc == 1 && qtab) rc = pe::launch_prep_k_qheads(a, aq, qtab, s);
     if (rc == 1) {
@@ -474,10 +502,11 @@ static int fwd_impl(const pe_attn_params* p, const pe_norm_params* nrm, const pe
     }
     if (rc) return rc;
   }
-  if (!v_direct(p, v, L.dv)) {
+  if (L.split || !v_direct(p, v, L.dv)) {
     pe_attn_params pv = *p;
     pv.mode = PE_MODE_NONE; pv.Dc = 0; pv.Dr = p->Dv; pv.qk_l2norm = 0;
     fill_prep(a, &pv, 1, nullptr, v, nullptr, nullptr, ws + L.v_off, L.dv);
+    a.dst_dtype = opd;
     if ((rc = pe::launch_prep(a, s))) return rc;
   }
   stage_mark(PE_STAGE_FWD_PREP, 1, s);
@@ -487,7 +516,7 @@ static int fwd_impl(const pe_attn_params* p, const pe_norm_params* nrm, const pe
   c.lse = lse;
   set_mask(c, mask);
   stage_mark(PE_STAGE_FWD_CORE, 0, s);
-  rc = pe::launch_fwd(p->dtype, L.dqk, L.dv, c, s);
+  rc = L.split ? pe::launch_fwd_split(L.dqk, L.dv, c, s) : pe::launch_fwd(p->dtype, L.dqk, L.dv, c, s);
   stage_mark(PE_STAGE_FWD_CORE, 1, s);
   return rc;
 }
@@ -547,13 +576,17 @@ int pe_attn_fwd_noalloc(const pe_attn_params* p, const pe_tensor_t* qc, const pe
                         void* stream) {
   int rc = pe_attn_check(p);
   if (rc) return rc;
-  if (layout(p).fwd_total > PE_NOALLOC_SCRATCH_BYTES) return PE_ERR_SCRATCH_LIMIT;
+  // fp32 operands as three bf16 planes take half as much again as fp32 ones: where only those fit, the
+  // forward runs on the fp32 unit
+  const bool unit = p->dtype == PE_DTYPE_FP32 && layout(p).fwd_total > PE_NOALLOC_SCRATCH_BYTES;
+  if (layout(p, false, unit).fwd_total > PE_NOALLOC_SCRATCH_BYTES) return PE_ERR_SCRATCH_LIMIT;
   if ((rc = device_ok())) return rc;
   void* ws = nullptr;
   if ((rc = scratch_on_current_device(&ws))) return rc;
   // every byte the kernels read from the workspace is written earlier in the same call (operand
   // rows including their zero padding, the phase table, the value repack), so nothing is cleared
-  return fwd_impl(p, nullptr, qc, qr, kc, kr, v, freqs, delta, out, lse, ws, PE_NOALLOC_SCRATCH_BYTES, stream);
+  return fwd_impl(p, nullptr, qc, qr, kc, kr, v, freqs, delta, out, lse, ws, PE_NOALLOC_SCRATCH_BYTES, stream,
+                  nullptr, unit);
 }
 
 int pe_attn_value_width(const pe_attn_params* p) {
@@ -824,7 +857,8 @@ static int bwd_impl(const pe_attn_params* p, const pe_tensor_t* qc, const pe_ten
   // the bf16 dK/dV kernel reads dO in place when its rows are 16-byte aligned and exactly Dv wide
   const bool gm = generic_masked(p, masked);
   const bool do_direct = half_dt(dt) && !gm && v_direct(p, dout, L.dv);
-  pb.dO_op = do_direct ? nullptr : bws + L.do_off; pb.op_dtype = p->dtype; pb.width = L.dv;
+  pb.dO_op = do_direct ? nullptr : bws + L.do_off; pb.op_dtype = L.split ? pe::DT_SPLIT_CODE : p->dtype; pb.width = L.dv;
+  pb.nat = L.split;
   pb.Di = (float*)(bws + L.di_off);
   pb.L2 = (float*)(bws + L.l2_off);
   pb.lse = lse;
@@ -912,6 +946,10 @@ static int bwd_impl(const pe_attn_params* p, const pe_tensor_t* qc, const pe_ten
   for (int g0 = 0; g0 < units; g0 += group) {
     c.bh0 = g0;
     c.nbh = std::min(group, units - g0);
+    if (L.split) {  // both halves in one launch
+      if ((rc = pe::launch_bwd_split(L.dqk, L.dv, c, s))) return rc;
+      break;
+    }
     if ((rc = pe::launch_bwd_dkdv(dt, L.dqk, L.dv, c, s))) return rc;
     if (group == units) {
       stage_mark(PE_STAGE_BWD_DKDV, 1, s);
@@ -919,7 +957,7 @@ static int bwd_impl(const pe_attn_params* p, const pe_tensor_t* qc, const pe_ten
     }
     if ((rc = pe::launch_bwd_dq(dt, L.dqk, L.dv, c, s))) return rc;
   }
-  if (group != units) {
+  if (group != units || L.split) {
     stage_mark(PE_STAGE_BWD_DKDV, 1, s);
     stage_mark(PE_STAGE_BWD_DQ, 0, s);
   }

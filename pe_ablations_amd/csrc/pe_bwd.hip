@@ -15,7 +15,9 @@
 
 namespace pe {
 
-// The fp32 kernels recompute P in natural units, exp(fma(s, scale, -lse)): the one rounding of the
+// These kernels serve explicit masks, in fp32 and at the 16-bit widths outside the dK/dV pair kernel's; fp32
+// without a mask runs on the bf16 matrix cores (pe_split.hip).
+// In fp32 they recompute P in natural units, exp(fma(s, scale, -lse)): the one rounding of the
 // exponent is at the size of s * scale - lse, which is small exactly where P is large, as in the
 // reference's fp32 softmax.  The log2-unit form exp2(s * (scale log2 e) - lse log2 e) rounds at the
 // size of the raw score (tens), and its P carried about three times the reference's error into dV
@@ -27,19 +29,13 @@ __device__ __forceinline__ float lse_nat(const CoreArgs& a, int bh, int q) {
   const float x = a.lse_in[(int64_t)bh * a.Sq + q];
   return x > -INFINITY ? x : INFINITY;
 }
-template <int DT> __device__ __forceinline__ float prob(float s, float scale, float sl2, float l) {
-  if constexpr (DT == 1) return exp2f(__builtin_fmaf(s, scale, -l) * LOG2E);
-  else return exp2f(s * sl2 - l);
-}
-
 // P with the explicit mask's log2-unit term ml2 (mask_l2) added to the score
 template <int DT> __device__ __forceinline__ float prob_m(float s, float scale, float sl2, float l, float ml2) {
   if constexpr (DT == 1) return exp2f(__builtin_fmaf(s, scale, -l) * LOG2E + ml2);
   else return exp2f(s * sl2 + ml2 - l);
 }
 
-// MB (here and in dq_kernel): the explicit-mask instantiation, for any operand type.
-template <int DT, int DQK, int DV, int BMQ, int NW, bool MB>
+template <int DT, int DQK, int DV, int BMQ, int NW>
 __global__ __launch_bounds__(NW * 64, 1) void dkdv_kernel(CoreArgs a) {
   using E = typename Elem<DT>::T;
   using M = MT<DT>;
@@ -145,9 +141,7 @@ __global__ __launch_bounds__(NW * 64, 1) void dkdv_kernel(CoreArgs a) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int qi = mt * 32 + c_logical<DT>(j, g);
-        float p;
-        if constexpr (MB) p = prob_m<DT>(s[j], a.scale, sl2, sL[qi], mask_l2(a, b, h, q0 + qi, myk));
-        else p = prob<DT>(s[j], a.scale, sl2, sL[qi]);
+        float p = prob_m<DT>(s[j], a.scale, sl2, sL[qi], mask_l2(a, b, h, q0 + qi, myk));
         if (edge && myk > q0 + qi + off) p = 0.f;
         s[j] = p;
         dp[j] = p * (dp[j] - sD[qi]);
@@ -197,7 +191,7 @@ __global__ __launch_bounds__(NW * 64, 1) void dkdv_kernel(CoreArgs a) {
     }
 }
 
-template <int DT, int DQK, int DV, int BN, int NW, bool MB>
+template <int DT, int DQK, int DV, int BN, int NW>
 __global__ __launch_bounds__(NW * 64, 1) void dq_kernel(CoreArgs a) {
   using E = typename Elem<DT>::T;
   using M = MT<DT>;
@@ -279,9 +273,7 @@ __global__ __launch_bounds__(NW * 64, 1) void dq_kernel(CoreArgs a) {
       for (int kk = 0; kk < NVF; ++kk) dp = M::mma(lds_row_frag<NCV>(sV, row, 2 * kk + g), of[kk], dp);
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        float p;
-        if constexpr (MB) p = prob_m<DT>(s[j], a.scale, sl2, lse2, mask_l2(a, b, h, myq, k0 + nt * 32 + c_logical<DT>(j, g)));
-        else p = prob<DT>(s[j], a.scale, sl2, lse2);
+        float p = prob_m<DT>(s[j], a.scale, sl2, lse2, mask_l2(a, b, h, myq, k0 + nt * 32 + c_logical<DT>(j, g)));
         if (edge) {
           const int key = k0 + nt * 32 + c_logical<DT>(j, g);
           if (key >= a.Sk || (a.causal && key > myq + off)) p = 0.f;
@@ -1777,17 +1769,16 @@ __global__ __launch_bounds__(NW * 64, 1) void dq_gemm_kernel(CoreArgs a) {
       }
 }
 
-// the generic kernels: fp32 operands, and the explicit-mask instantiations (MB) of fp32 and of the
-// 16-bit widths outside the pair kernel's
-template <int DT, int DQK, int DV, bool MB>
+// the generic kernels: explicit masks in fp32 and at the 16-bit widths outside the pair kernel's
+template <int DT, int DQK, int DV>
 static int run_bwd_generic(int which, const CoreArgs& a, hipStream_t s) {
   constexpr int NW = 4, BMQ = 32, BN = 32;
   if (which == 0) {
     const int nkb = (a.Sk + NW * 32 - 1) / (NW * 32);
-    hipLaunchKernelGGL((dkdv_kernel<DT, DQK, DV, BMQ, NW, MB>), dim3(nkb * a.nbh), dim3(NW * 64), 0, s, a);
+    hipLaunchKernelGGL((dkdv_kernel<DT, DQK, DV, BMQ, NW>), dim3(nkb * a.nbh), dim3(NW * 64), 0, s, a);
   } else {
     const int nqb = (a.Sq + NW * 32 - 1) / (NW * 32);
-    hipLaunchKernelGGL((dq_kernel<DT, DQK, DV, BN, NW, MB>), dim3(nqb * a.nbh * (a.Hq / a.Hkv)), dim3(NW * 64), 0, s, a);
+    hipLaunchKernelGGL((dq_kernel<DT, DQK, DV, BN, NW>), dim3(nqb * a.nbh * (a.Hq / a.Hkv)), dim3(NW * 64), 0, s, a);
   }
   return hipGetLastError() == hipSuccess ? 0 : -7;
 }
@@ -1809,7 +1800,7 @@ static int run_bwd(int which, const CoreArgs& a, hipStream_t s) {
       return hipGetLastError() == hipSuccess ? 0 : -7;
     }
   } else {
-    if (a.mask) return run_bwd_generic<DT, DQK, DV, true>(which, a, s);
+    if (a.mask) return run_bwd_generic<DT, DQK, DV>(which, a, s);
   }
   if constexpr (DT != 1) {
     if (which == 0) {
@@ -1847,7 +1838,7 @@ static int run_bwd(int which, const CoreArgs& a, hipStream_t s) {
     }
     return hipGetLastError() == hipSuccess ? 0 : -7;
   } else {
-    return run_bwd_generic<DT, DQK, DV, false>(which, a, s);
+    return -4;  // fp32 without a mask: launch_bwd_split
   }
 }
 

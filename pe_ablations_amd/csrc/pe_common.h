@@ -128,6 +128,53 @@ __device__ __forceinline__ void store8(void* p, int64_t i, int dtype, const floa
   }
 }
 
+// An fp32 value as the sum of three bf16 ones, x = h + m + l: h = bf16(x), m = bf16(x - h), l = x - h - m.
+// Each step rounds to nearest, so both differences are exact in fp32 and l needs no more than the 8 bits
+// that bf16 has (24 = 8 + 8 + 8): the sum is x itself, as long as x does not round to a bf16 infinity
+// (|x| >= 2^128 (1 - 2^-9)) and l stays normal.  Two values at a time, packed as operand dwords.
+__device__ __forceinline__ void split_bf3(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+  h = pack_bf2(x0, x1);
+  x0 -= __builtin_bit_cast(float, h << 16);
+  x1 -= __builtin_bit_cast(float, h & 0xffff0000u);
+  m = pack_bf2(x0, x1);
+  x0 -= __builtin_bit_cast(float, m << 16);
+  x1 -= __builtin_bit_cast(float, m & 0xffff0000u);
+  l = pack_bf2(x0, x1);
+}
+
+// Operand rows (the prologue's output): row `row`, columns c .. c + 7 of rows of `width` elements.
+// dtype 3: three bf16 planes of `width` elements one after another in each row, holding h, m and l of
+// split_bf3 (the fp32 compute type's operands for the matrix cores)
+constexpr int DT_SPLIT = 3;  // DT_SPLIT_CODE on the host side
+__device__ __forceinline__ void row_store8(void* dst, int64_t row, int width, int c, int dtype, const float (&x)[8]) {
+  if (dtype == DT_SPLIT) {
+    uint16_t* p = (uint16_t*)dst + row * 3 * width + c;
+    u32x4 h, m, l;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint32_t a, b, d;
+      split_bf3(x[2 * e], x[2 * e + 1], a, b, d);
+      h[e] = a; m[e] = b; l[e] = d;
+    }
+    *(u32x4*)p = h;
+    *(u32x4*)(p + width) = m;
+    *(u32x4*)(p + 2 * width) = l;
+  } else {
+    store8(dst, row * width + c, dtype, x);
+  }
+}
+__device__ __forceinline__ void store_from_float(void* p, int64_t i, int dtype, float x);
+__device__ __forceinline__ void row_store(void* dst, int64_t row, int width, int c, int dtype, float x) {
+  if (dtype == DT_SPLIT) {
+    uint16_t* p = (uint16_t*)dst + row * 3 * width + c;
+    uint32_t h, m, l;
+    split_bf3(x, 0.f, h, m, l);
+    p[0] = (uint16_t)h; p[width] = (uint16_t)m; p[2 * width] = (uint16_t)l;
+  } else {
+    store_from_float(dst, row * width + c, dtype, x);
+  }
+}
+
 // 8 consecutive elements of type XT kept as loaded (16 or 32 bytes) until they are used
 template <int XT> struct Raw8 {
   u32x4 r[XT == 1 ? 2 : 1];

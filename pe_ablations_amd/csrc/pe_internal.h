@@ -6,6 +6,9 @@
 
 namespace pe {
 
+// PrepArgs::dst_dtype of operand rows held as three bf16 planes (pe_common.h, DT_SPLIT)
+constexpr int DT_SPLIT_CODE = 3;
+
 // Inverse PoPE transform fused into a gradient kernel's epilogue: the raw positional input x and
 // the view its gradient is written through, plus per-block partial sums of dphi and pos*dphi
 // (block = (b, h, tile) in that order; either pointer may be NULL).
@@ -113,6 +116,11 @@ struct CoreArgs {
 };
 
 int launch_fwd(int dt, int dqk, int dv, const CoreArgs& a, hipStream_t s);
+// fp32 compute on the bf16 matrix cores: q / k / v hold rows of three bf16 planes (DT_SPLIT)
+int launch_fwd_split(int dqk, int dv, const CoreArgs& a, hipStream_t s);
+// its backward, dq~ and dk~ / dV in one launch: dO in planes, L2 holding the
+// natural-unit lse (PreBwdArgs::nat), qsplit any number of ranges of each key block's query tiles
+int launch_bwd_split(int dqk, int dv, const CoreArgs& a, hipStream_t s);
 int launch_bwd_dkdv(int dt, int dqk, int dv, const CoreArgs& a, hipStream_t s);
 int launch_bwd_dq(int dt, int dqk, int dv, const CoreArgs& a, hipStream_t s);
 bool core_supported(int dqk, int dv);
@@ -237,6 +245,7 @@ struct PreBwdArgs {
   const void* out; int out_dtype; int64_t o_s[4];
   void* dO_op; int op_dtype; int width;
   const float* lse; float* Di; float* L2; int s_pad;
+  int nat;  // L2 holds lse itself (natural units) instead of lse * log2(e)
   int B, H, S, Dv;
 };
 int launch_prebwd(const PreBwdArgs& a, hipStream_t s);

@@ -135,9 +135,9 @@ __global__ __launch_bounds__(WPB * 64) void prep_pope_norm_kernel(PrepArgs a) {
           sv[e] = mul_nc(mu, sn);
         }
       }
-      const int64_t drow = ((int64_t)(b * a.H + h) * a.S + s) * a.width;
-      store8(a.dst, drow + a.Dc + t * 8, DDT, cv);
-      store8(a.dst, drow + a.Dc + a.Dr + t * 8, DDT, sv);
+      const int64_t drow = (int64_t)(b * a.H + h) * a.S + s;
+      row_store8(a.dst, drow, a.width, a.Dc + t * 8, DDT, cv);
+      row_store8(a.dst, drow, a.width, a.Dc + a.Dr + t * 8, DDT, sv);
     }
   }
   if (a.Dc > 0) {  // content part: converted copy
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(WPB * 64) void prep_pope_norm_kernel(PrepArgs a) {
       const int h = c / cpr, j = c - h * cpr;
       float v[8];
       load8(a.xc, b * a.xc_s[0] + h * a.xc_s[1] + (int64_t)s * a.xc_s[2] + j * 8, a.xc_dtype, v);
-      store8(a.dst, ((int64_t)(b * a.H + h) * a.S + s) * a.width + j * 8, DDT, v);
+      row_store8(a.dst, (int64_t)(b * a.H + h) * a.S + s, a.width, j * 8, DDT, v);
     }
   }
   const int used = a.Dc + 2 * a.Dr;
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(WPB * 64) void prep_pope_norm_kernel(PrepArgs a) {
   for (int c = lane; c < a.H * ppr; c += 64) {
     const int h = c / ppr, j = c - h * ppr;
     const float z[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    store8(a.dst, ((int64_t)(b * a.H + h) * a.S + s) * a.width + used + j * 8, DDT, z);
+    row_store8(a.dst, (int64_t)(b * a.H + h) * a.S + s, a.width, used + j * 8, DDT, z);
   }
 }
 
@@ -384,7 +384,7 @@ int launch_swiglu(const void* x, const void* gate, void* out, int64_t n, hipStre
 
 int launch_prep_norm(const PrepArgs& a, hipStream_t s) {
   if (a.mode != 0 || !a.norm_w || a.norm_w_dtype < 0 || a.norm_w_dtype > 2 || a.xr_dtype < 0 || a.xr_dtype > 2 ||
-      a.dst_dtype < 0 || a.dst_dtype > 2)
+      a.dst_dtype < 0 || a.dst_dtype > DT_SPLIT)
     return -4;
   if (a.dst_rows != 0 || a.dst_row0 != 0) return -2;  // writes contiguous (B, H, S, width) rows only
   if (a.Dr <= 0 || a.Dr % 8 != 0 || a.Dc % 8 != 0 || a.width % 8 != 0 || a.H * (a.Dr / 8) > 64 * MAXCPL) return -3;
@@ -399,7 +399,8 @@ int launch_prep_norm(const PrepArgs& a, hipStream_t s) {
     constexpr int C = decltype(c)::value;
     if (a.dst_dtype == 0) hipLaunchKernelGGL((prep_pope_norm_kernel<0, C>), grid, dim3(WPB * 64), 0, s, a);
     else if (a.dst_dtype == 2) hipLaunchKernelGGL((prep_pope_norm_kernel<2, C>), grid, dim3(WPB * 64), 0, s, a);
-    else hipLaunchKernelGGL((prep_pope_norm_kernel<1, C>), grid, dim3(WPB * 64), 0, s, a);
+    else if (a.dst_dtype == 1) hipLaunchKernelGGL((prep_pope_norm_kernel<1, C>), grid, dim3(WPB * 64), 0, s, a);
+    else hipLaunchKernelGGL((prep_pope_norm_kernel<DT_SPLIT, C>), grid, dim3(WPB * 64), 0, s, a);
   });
   return hipGetLastError() == hipSuccess ? 0 : -7;
 }

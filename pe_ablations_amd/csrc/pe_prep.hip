@@ -34,11 +34,11 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
   const int bh = (int)(row / a.S);
   const int h = bh % a.H, b = bh / a.H;
   const float pos = pe_pos(a.start_pos + s, a.pos_round);
-  const int64_t dbase = ((int64_t)bh * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s) * a.width;
+  const int64_t drow = (int64_t)bh * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s;
 
   for (int c = lane; c < a.Dc; c += 64) {
     const float x = load_as_float(a.xc, b * a.xc_s[0] + h * a.xc_s[1] + (int64_t)s * a.xc_s[2] + c * a.xc_s[3], a.xc_dtype);
-    store_from_float(a.dst, dbase + c, a.dst_dtype, x);
+    row_store(a.dst, drow, a.width, c, a.dst_dtype, x);
   }
   const int64_t xr0 = b * a.xr_s[0] + h * a.xr_s[1] + (int64_t)s * a.xr_s[2];
   int used = a.Dc;
@@ -50,8 +50,8 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
       if (a.is_key && a.delta) ph = add_nc(ph, a.delta[h * a.delta_hs + c]);
       float sn, cs;
       pe_sincos(ph, sn, cs);
-      store_from_float(a.dst, dbase + a.Dc + c, a.dst_dtype, mul_nc(mu, cs));
-      store_from_float(a.dst, dbase + a.Dc + a.Dr + c, a.dst_dtype, mul_nc(mu, sn));
+      row_store(a.dst, drow, a.width, a.Dc + c, a.dst_dtype, mul_nc(mu, cs));
+      row_store(a.dst, drow, a.width, a.Dc + a.Dr + c, a.dst_dtype, mul_nc(mu, sn));
     }
     used += 2 * a.Dr;
   } else {  // RoPE (mode 1) or plain (mode 2): values kept in registers for the optional L2 norm
@@ -79,14 +79,14 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
     for (int k = 0; k < MAX_PAIRS_PER_LANE; ++k) {
       const int i = 4 * lane + k;
       if (i < npairs) {
-        store_from_float(a.dst, dbase + a.Dc + 2 * i, a.dst_dtype, a.l2norm ? y0[k] / den : y0[k]);
+        row_store(a.dst, drow, a.width, a.Dc + 2 * i, a.dst_dtype, a.l2norm ? y0[k] / den : y0[k]);
         if (2 * i + 1 < a.Dr)
-          store_from_float(a.dst, dbase + a.Dc + 2 * i + 1, a.dst_dtype, a.l2norm ? y1[k] / den : y1[k]);
+          row_store(a.dst, drow, a.width, a.Dc + 2 * i + 1, a.dst_dtype, a.l2norm ? y1[k] / den : y1[k]);
       }
     }
     used += a.Dr;
   }
-  for (int c = used + lane; c < a.width; c += 64) store_from_float(a.dst, dbase + c, a.dst_dtype, 0.f);
+  for (int c = used + lane; c < a.width; c += 64) row_store(a.dst, drow, a.width, c, a.dst_dtype, 0.f);
 }
 
 // One wave per padded row (b, h, s < S_pad).  Rows s < S: dO repack, Di, L2 = lse*log2(e) (a row
@@ -114,13 +114,13 @@ __global__ __launch_bounds__(256) void prebwd_kernel(PreBwdArgs a) {
       d = load_as_float(a.dout, d0 + c * a.do_s[3], a.dout_dtype);
       acc += d * load_as_float(a.out, o0 + c * a.o_s[3], a.out_dtype);
     }
-    if (a.dO_op) store_from_float(a.dO_op, row * a.width + c, a.op_dtype, d);
+    if (a.dO_op) row_store(a.dO_op, row, a.width, c, a.op_dtype, d);
   }
   acc = wave_sum(acc);
   if (lane == 0) {
     a.Di[prow] = acc;
     const float lv = a.lse[row];
-    a.L2[prow] = lv == -INFINITY ? INFINITY : lv * LOG2E;
+    a.L2[prow] = lv == -INFINITY ? INFINITY : (a.nat ? lv : lv * LOG2E);
   }
 }
 
@@ -295,7 +295,7 @@ __device__ __forceinline__ void prep_pope_vec_body(const PrepArgs& a, int64_t gi
   const int bh = (int)(row / a.S);
   const int h = bh % a.H, b = bh / a.H;
   const float pos = pe_pos(a.start_pos + s, a.pos_round);
-  const int64_t drow = ((int64_t)bh * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s) * a.width;
+  const int64_t drow = (int64_t)bh * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s;
   float x[8];
   load8(a.xr, b * a.xr_s[0] + h * a.xr_s[1] + (int64_t)s * a.xr_s[2] + t * 8, XT, x);
   const f32x4 f0 = *(const f32x4*)(a.freqs + t * 8), f1 = *(const f32x4*)(a.freqs + t * 8 + 4);
@@ -332,18 +332,18 @@ __device__ __forceinline__ void prep_pope_vec_body(const PrepArgs& a, int64_t gi
       }
     }
   }
-  store8(a.dst, drow + a.Dc + t * 8, DT, cv);
-  store8(a.dst, drow + a.Dc + a.Dr + t * 8, DT, sv);
+  row_store8(a.dst, drow, a.width, a.Dc + t * 8, DT, cv);
+  row_store8(a.dst, drow, a.width, a.Dc + a.Dr + t * 8, DT, sv);
   if (a.Dc > 0) {
     const int64_t xc0 = b * a.xc_s[0] + h * a.xc_s[1] + (int64_t)s * a.xc_s[2];
     for (int j = t; j < a.Dc / 8; j += tpr) {
       float c[8];
       load8(a.xc, xc0 + j * 8, a.xc_dtype, c);
-      store8(a.dst, drow + j * 8, DT, c);
+      row_store8(a.dst, drow, a.width, j * 8, DT, c);
     }
   }
   const float zero[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int j = (a.Dc + 2 * a.Dr) / 8 + t; j < a.width / 8; j += tpr) store8(a.dst, drow + j * 8, DT, zero);
+  for (int j = (a.Dc + 2 * a.Dr) / 8 + t; j < a.width / 8; j += tpr) row_store8(a.dst, drow, a.width, j * 8, DT, zero);
   if (a.cdst) {  // the row's companion copy (KV-cache append: the value row), 16-bit elements
     const uint16_t* crow = (const uint16_t*)a.cv + b * a.cv_s[0] + h * a.cv_s[1] + (int64_t)s * a.cv_s[2];
     uint16_t* cd = (uint16_t*)a.cdst + ((int64_t)bh * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s) * a.cwidth;
@@ -400,8 +400,9 @@ template <int HT> __global__ __launch_bounds__(256) void prep_pope_small_kernel(
 }
 
 // one group of TPR = Dv / 8 lanes per padded row (TPR a power of two, groups never straddle a
-// wave); Di is the group's fixed-order butterfly sum.  XT: the element type of dO and out
-template <int XT> __global__ __launch_bounds__(256) void prebwd_vec_kernel(PreBwdArgs a, int lg_tpr) {
+// wave); Di is the group's fixed-order butterfly sum.  XT: the element type of dO and
+// out, OT that of the repacked rows
+template <int XT, int OT> __global__ __launch_bounds__(256) void prebwd_vec_kernel(PreBwdArgs a, int lg_tpr) {
   const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t prow = gid >> lg_tpr;
   const int t = (int)(gid & ((1 << lg_tpr) - 1));
@@ -417,7 +418,7 @@ template <int XT> __global__ __launch_bounds__(256) void prebwd_vec_kernel(PreBw
   float d[8], o[8];
   load8(a.dout, b * a.do_s[0] + h * a.do_s[1] + (int64_t)s * a.do_s[2] + t * 8, XT, d);
   load8(a.out, b * a.o_s[0] + h * a.o_s[1] + (int64_t)s * a.o_s[2] + t * 8, XT, o);
-  if (a.dO_op) store8(a.dO_op, row * a.width + t * 8, XT, d);
+  if (a.dO_op) row_store8(a.dO_op, row, a.width, t * 8, OT, d);
   float acc = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc += d[e] * o[e];
@@ -425,7 +426,7 @@ template <int XT> __global__ __launch_bounds__(256) void prebwd_vec_kernel(PreBw
   if (t == 0) {
     a.Di[prow] = acc;
     const float lv = a.lse[row];
-    a.L2[prow] = lv == -INFINITY ? INFINITY : lv * LOG2E;
+    a.L2[prow] = lv == -INFINITY ? INFINITY : (a.nat ? lv : lv * LOG2E);
   }
 }
 
@@ -445,7 +446,7 @@ __global__ __launch_bounds__(256) void prep_rope_vec_kernel(PrepArgs a, int lg_t
   const int bh = (int)(row / a.S);
   const int h = bh % a.H, b = bh / a.H;
   const float pos = pe_pos(a.start_pos + s, a.pos_round);
-  const int64_t drow = ((int64_t)bh * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s) * a.width;
+  const int64_t drow = (int64_t)bh * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s;
   float x[8], y[8];
   load8(a.xr, b * a.xr_s[0] + h * a.xr_s[1] + (int64_t)s * a.xr_s[2] + t * 8, a.xr_dtype, x);
   float ss = 0.f;
@@ -462,17 +463,17 @@ __global__ __launch_bounds__(256) void prep_rope_vec_kernel(PrepArgs a, int lg_t
 #pragma unroll
     for (int e = 0; e < 8; ++e) y[e] = y[e] / den;
   }
-  store8(a.dst, drow + a.Dc + t * 8, a.dst_dtype, y);
+  row_store8(a.dst, drow, a.width, a.Dc + t * 8, a.dst_dtype, y);
   if (a.Dc > 0) {
     const int64_t xc0 = b * a.xc_s[0] + h * a.xc_s[1] + (int64_t)s * a.xc_s[2];
     for (int j = t; j < a.Dc / 8; j += tpr) {
       float c[8];
       load8(a.xc, xc0 + j * 8, a.xc_dtype, c);
-      store8(a.dst, drow + j * 8, a.dst_dtype, c);
+      row_store8(a.dst, drow, a.width, j * 8, a.dst_dtype, c);
     }
   }
   const float zero[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int j = (a.Dc + a.Dr) / 8 + t; j < a.width / 8; j += tpr) store8(a.dst, drow + j * 8, a.dst_dtype, zero);
+  for (int j = (a.Dc + a.Dr) / 8 + t; j < a.width / 8; j += tpr) row_store8(a.dst, drow, a.width, j * 8, a.dst_dtype, zero);
 }
 
 __global__ __launch_bounds__(256) void inv_rope_vec_kernel(InvArgs a, int lg_tpr) {
@@ -541,10 +542,12 @@ static int inv_rope_vec_lg(const InvArgs& a) {
   return lg;
 }
 
-// element types the vectorised PoPE prologue is built for: raw rows and operands of one type, and fp32
-// rows (RMS-normed projections under autocast) into 16-bit operands; -1 for any other pair
+// element types the vectorised PoPE prologue is built for: raw rows and operands of one type, fp32 rows
+// (RMS-normed projections under autocast) into 16-bit operands and into fp32's three bf16 planes; -1 for
+// any other pair
 static int prep_vec_types(int xt, int dt) {
   if (xt == dt && dt >= 0 && dt <= 2) return dt;
+  if (xt == 1 && dt == DT_SPLIT) return 5;
   return xt == 1 ? (dt == 0 ? 3 : dt == 2 ? 4 : -1) : -1;
 }
 // calls f with the raw and operand element types of prep_vec_types' pair as compile-time constants
@@ -554,7 +557,8 @@ template <typename F> static void with_prep_types(int pair, F&& f) {
     case 1: f(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}); break;
     case 2: f(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{}); break;
     case 3: f(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{}); break;
-    default: f(std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{}); break;
+    case 4: f(std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{}); break;
+    default: f(std::integral_constant<int, 1>{}, std::integral_constant<int, DT_SPLIT>{}); break;
   }
 }
 static int prep_vec_types(const PrepArgs& a) { return prep_vec_types(a.xr_dtype, a.dst_dtype); }
@@ -567,7 +571,7 @@ static bool prep_vec_ok(const PrepArgs& a) {
 }
 
 bool prep_vec_copy_ok(const PrepArgs& a) {
-  return prep_vec_ok(a) && a.dst_dtype != 1 && a.cv && a.cdst && a.cv_s[3] == 1 && aligned16(a.cv, a.cv_s[0], a.cv_s[1], a.cv_s[2]) &&
+  return prep_vec_ok(a) && (a.dst_dtype == 0 || a.dst_dtype == 2) && a.cv && a.cdst && a.cv_s[3] == 1 && aligned16(a.cv, a.cv_s[0], a.cv_s[1], a.cv_s[2]) &&
          ((uintptr_t)a.cdst % 16) == 0 && a.cv_cols % 8 == 0 && a.cwidth % 8 == 0 && a.cv_cols <= a.cwidth;
 }
 
@@ -682,9 +686,9 @@ __device__ __forceinline__ void prep_pope_qheads_body(const PrepArgs& a, int64_t
       cv[e] = mul_nc(mu, cs[e]);
       sv[e] = mul_nc(mu, sn[e]);
     }
-    const int64_t drow = ((int64_t)(b * a.H + h) * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s) * a.width;
-    store8(a.dst, drow + t * 8, DT, cv);
-    store8(a.dst, drow + a.Dr + t * 8, DT, sv);
+    const int64_t drow = (int64_t)(b * a.H + h) * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s;
+    row_store8(a.dst, drow, a.width, t * 8, DT, cv);
+    row_store8(a.dst, drow, a.width, a.Dr + t * 8, DT, sv);
   }
 }
 
@@ -766,15 +770,16 @@ int launch_prebwd(const PreBwdArgs& a, hipStream_t s) {
   const int tpr = a.Dv / 8;
   const bool vec = a.dout_dtype == a.out_dtype && a.Dv % 8 == 0 && tpr <= 64 && (tpr & (tpr - 1)) == 0 &&
                    rows16(a.dout, a.dout_dtype, a.do_s) && rows16(a.out, a.out_dtype, a.o_s) &&
-                   (!a.dO_op || (a.op_dtype == a.dout_dtype && a.width == a.Dv && ((uintptr_t)a.dO_op % 16) == 0));
+                   (!a.dO_op || ((a.op_dtype == a.dout_dtype || (a.op_dtype == DT_SPLIT && a.dout_dtype == 1)) && a.width == a.Dv && ((uintptr_t)a.dO_op % 16) == 0));
   const int64_t nrows = (int64_t)a.B * a.H * a.s_pad;
   if (vec) {
     int lg = 0;
     while ((1 << lg) < tpr) ++lg;
     const dim3 grid((unsigned)((nrows * tpr + 255) / 256));
-    if (a.dout_dtype == 0) hipLaunchKernelGGL(prebwd_vec_kernel<0>, grid, dim3(256), 0, s, a, lg);
-    else if (a.dout_dtype == 2) hipLaunchKernelGGL(prebwd_vec_kernel<2>, grid, dim3(256), 0, s, a, lg);
-    else hipLaunchKernelGGL(prebwd_vec_kernel<1>, grid, dim3(256), 0, s, a, lg);
+    if (a.dout_dtype == 0) hipLaunchKernelGGL((prebwd_vec_kernel<0, 0>), grid, dim3(256), 0, s, a, lg);
+    else if (a.dout_dtype == 2) hipLaunchKernelGGL((prebwd_vec_kernel<2, 2>), grid, dim3(256), 0, s, a, lg);
+    else if (a.op_dtype != DT_SPLIT) hipLaunchKernelGGL((prebwd_vec_kernel<1, 1>), grid, dim3(256), 0, s, a, lg);
+    else hipLaunchKernelGGL((prebwd_vec_kernel<1, DT_SPLIT>), grid, dim3(256), 0, s, a, lg);
   } else {
     hipLaunchKernelGGL(prebwd_kernel, dim3((unsigned)((nrows + 3) / 4)), dim3(256), 0, s, a);
   }
