@@ -966,14 +966,13 @@ __global__ __launch_bounds__(512, 1) void dkdv_pair_kernel(CoreArgs a) {
   const bool l2w = __builtin_amdgcn_readfirstlane(w) == 0;  // the wave that loads each tile's L2 / Di
   const int nkb = (a.Sk + BNK - 1) / BNK;
   int kb, bh;
-  // QS (launched with a.qsplit > 1): workgroup jq of a key block takes query heads jq * hpw .. of
-  // its group and leaves fp32 partial dK~ / dV for dkdv_combine (run by the dQ launch).  A separate
-  // instantiation, so the unsplit kernel carries none of its registers.
+  // QS (launched with a.qsplit > 1): workgroup jq of a key block takes the jq-th range of its list of
+  // (query head, query tile) and leaves fp32 partial dK~ / dV for dkdv_combine (run by the dQ launch).  A
+  // separate instantiation, so the unsplit kernel carries none of its registers.
   const int nblk = nkb * a.nbh, jq = QS ? (int)blockIdx.x / nblk : 0;
   map_block(blockIdx.x - jq * nblk, nkb, a.nbh, false, kb, bh);
   bh += a.bh0;  // the head group's units
   const int b = bh / a.Hkv, hk = bh % a.Hkv, grp = a.Hq / a.Hkv;
-  const int hpw = QS ? grp / a.qsplit : grp, h_first = hk * grp + jq * hpw;
   const int k0 = kb * BNK, kw0 = k0 + pw * 32, myk = kw0 + l32;
   const int off = a.causal_off;
 
@@ -981,8 +980,12 @@ __global__ __launch_bounds__(512, 1) void dkdv_pair_kernel(CoreArgs a) {
   int qb0 = 0;
   if (a.causal) qb0 = max(0, k0 - off) / BMQ;
   if (qb0 > nqt) qb0 = nqt;
-  const int nper = nqt - qb0;
-  const int niter = nper * hpw;
+  const int nper = nqt - qb0, ntot = nper * grp;
+  // (ntot * qsplit < 2^31: at most 8 ranges; in scalar registers, as the tile addresses are)
+  const int it0 = QS ? __builtin_amdgcn_readfirstlane((uint32_t)(ntot * jq) / (uint32_t)a.qsplit) : 0;
+  const int niter = QS ? __builtin_amdgcn_readfirstlane((uint32_t)(ntot * (jq + 1)) / (uint32_t)a.qsplit) - it0 : ntot;
+  const int h_first = hk * grp + (QS && nper > 0 ? it0 / nper : 0);
+  const int qt_first = qb0 + (QS && nper > 0 ? it0 % nper : 0);
   const float sl2 = a.scale * LOG2E;
   const int64_t qrs = (int64_t)DQK * 2;
 
@@ -991,7 +994,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_pair_kernel(CoreArgs a) {
   const DmaPlan<BMQ, NCQ, NA, SZ> plan_q(pw, lane, (uint32_t)qrs);
   const DmaPlan<BMQ, NCO, NA, SZ> plan_o(pw, lane, (uint32_t)(a.do_ss * 2));
   const uint32_t smem_l = lds_addr(smem);
-  int iss_h = h_first, iss_qt = qb0;
+  int iss_h = h_first, iss_qt = qt_first;
   auto issue = [&](int it) {
     char* st = smem + (it % NSTG) * STAGE;
     const uint32_t stl = smem_l + (uint32_t)((it % NSTG) * STAGE);
@@ -1134,7 +1137,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_pair_kernel(CoreArgs a) {
 #pragma unroll
     for (int i = 0; i < 2 * QT; ++i) pa0[i] = pa1[i] = u32x4{0u, 0u, 0u, 0u};
     f32x16 s[QT];
-    int cur_qt = qb0;  // query tile of step t
+    int cur_qt = qt_first;  // query tile of step t
     // step t: S of tile t (products right after the barrier), the loads of tile t + 2, P of tile t,
     // then dV of tile t - 1 from the other P buffer
     auto astep = [&](int t, u32x4 (&pn)[2 * QT], u32x4 (&pp)[2 * QT]) {
@@ -1291,7 +1294,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_pair_kernel(CoreArgs a) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) dk[t][j] = 0.f;
     f32x16 dp[QT];
-    int prev_h = h_first, prev_qt = qb0;  // head and query tile of step t - 1
+    int prev_h = h_first, prev_qt = qt_first;  // head and query tile of step t - 1
     // the wave's key row in the packed dS (pe_internal.h), less its first stored 64-query block
     const int64_t ds_row = ds_row_base(kw0 >> 5, a.ds_e, a.ds_nqt, a.causal) - ds_first(kb, a.ds_e, a.causal);
     // role B's instructions go first when both waves of a SIMD are ready to issue, except while
@@ -1367,8 +1370,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_pair_kernel(CoreArgs a) {
   if constexpr (!QS) dk_epilogue<HT, DQK>(a, st_epi, tid, b, hk, kb, bh, nkb);
 }
 
-// The query-head split of the pair kernel (a.qsplit > 1, grids with fewer key blocks than compute
-// units): one workgroup of 512 threads per key block of (b, hk) adds the qsplit fp32 partials of
+// The query split of the pair kernel (a.qsplit > 1, see key_split in pe_api.cpp): one workgroup of 512 threads per key block of (b, hk) adds the qsplit fp32 partials of
 // dV and dK~ in slice order, stores dV in dv's dtype, and either runs the dK~ epilogue
 // (a.fuse_inv) or leaves the sum in slice 0 of dk_t for the stand-alone inverse-transform kernels.
 // Both paths see the same sums, so the fused and unfused gradients stay bitwise equal.  It runs as
