@@ -40,7 +40,7 @@ struct Layout {
   int dqk, dv;
   bool split;  // fp32 compute with its operands as three bf16 planes (pe_split.hip)
   size_t q_off, k_off, v_off, tab_off, fwd_total;
-  size_t do_off, di_off, l2_off, dq_off, dk_off, pq_off, pk_off, pkd_off, dvp_off, ds_off, bwd_total;
+  size_t do_off, di_off, l2_off, dq_off, dk_off, pq_off, pk_off, pkd_off, dvp_off, rtab_off, ds_off, bwd_total;
   int ksplit;    // query-head split of the dK/dV pair kernel (pe::CoreArgs::qsplit)
   int sq_pad;
   int ds_nqt, ds_rows, ds_e;
@@ -66,8 +66,8 @@ constexpr int kSplitCus = 256;
 
 // dK/dV pair kernel (16-bit, transformed width 128 / 256, value width 64 / 128): workgroups per key block.
 // A causal block's work falls with its key position, from every query tile to one, so a grid of one
-// workgroup per compute unit waits for its first blocks; two a unit, issued longest first, even out.  Below
-// that many blocks the query heads of the GQA group are shared out (a power of two dividing it) and, past
+// workgroup per compute unit waits for its first blocks; from one and a half a unit on, issued longest
+// first, they even out (384 blocks: as fast whole as halved).  Below that the query heads of the GQA group are shared out (a power of two dividing it) and, past
 // 512 queries, their query tiles, as long as a range keeps four 64-query tiles (up to 512 the workspace
 // keeps the size it had).  Forward and backward on one GPU, without against with: 16 -> 4 heads of 128, RoPE,
 // 4 x 2048 rows 502 / 433 us; 16 heads of 128, 1024 rows 157 / 147; 4 heads of 128, 4096 rows 403 / 333,
@@ -76,10 +76,10 @@ int key_split(const pe_attn_params* p, int dqk, int dv) {
   if (!half_dt(p->dtype) || !((dqk == 128 || dqk == 256) && (dv == 64 || dv == 128))) return 1;
   const int grp = p->Hq / p->Hkv;
   const int64_t blocks = (int64_t)p->B * p->Hkv * ((p->Sk + 127) / 128);
-  const int64_t want = p->causal != PE_CAUSAL_NONE ? 2 * kSplitCus : kSplitCus;
+  const int64_t even = p->causal != PE_CAUSAL_NONE ? kSplitCus * 3 / 2 : kSplitCus;
   const int tiles = grp * ((p->Sq + 63) / 64);
   int ks = 1;
-  while (ks < 8 && blocks * ks < want && (grp % (2 * ks) == 0 || (p->Sq > 512 && tiles / (2 * ks) >= 4))) ks *= 2;
+  while (ks < 8 && blocks * ks < (ks == 1 ? even : kSplitCus) && (grp % (2 * ks) == 0 || (p->Sq > 512 && tiles / (2 * ks) >= 4))) ks *= 2;
   return ks;
 }
 
@@ -164,7 +164,9 @@ Layout layout(const pe_attn_params* p, bool masked = false, bool unit = false) {
   L.pk_off = L.pq_off + align_up((size_t)L.nq_blocks * p->Dr * 4);
   L.pkd_off = L.pk_off + align_up((size_t)L.nk_blocks * p->Dr * 4);
   L.dvp_off = L.pkd_off + align_up((size_t)L.nk_blocks * p->Dr * 4);
-  L.ds_off = L.dvp_off + (slices > 1 ? align_up(nk * L.dv * 4 * slices) : 0);
+  L.rtab_off = L.dvp_off + (slices > 1 ? align_up(nk * L.dv * 4 * slices) : 0);
+  // the fused RoPE gradient's angles (cos / sin, fp32 [Sq][2][Dr / 2]), written by the backward's dO pass
+  L.ds_off = L.rtab_off + (half_dt(p->dtype) && p->mode == PE_MODE_ROPE ? align_up((size_t)p->Sq * p->Dr * 4) : 0);
   // bf16 path: dS in fragment order, 4 KiB blocks packed per (b, h) to the blocks the causal
   // dK/dV kernel stores (pe::ds_row_base), written by it for the dQ GEMM.  The dQ GEMM's masked
   // edge steps also load up to four blocks before a key row's first stored one; those lie in the
@@ -498,7 +500,7 @@ static int fwd_impl(const pe_attn_params* p, const pe_norm_params* nrm, const pe
     pe::PrepArgs aq;
     fill_prep(aq, p, 0, qc, qr, freqs, nullptr, ws + L.q_off, L.dqk);
     a.dst_dtype = aq.dst_dtype = opd;
-    rc = qtab ? pe::launch_prep_qk(a, aq, qtab, s) : 1;
+    rc = qtab ? pe::launch_prep_qk(a, aq, qtab, s) : p->mode != PE_MODE_POPE ? pe::launch_prep_rope_qk(a, aq, s) : 1;
     if (rc == 1 && qtab) rc = pe::launch_prep_k_qheads(a, aq, qtab, s);
     if (rc == 1) {
       if (qtab) rc = pe::launch_prep_and_table(a, freqs, p->start_pos_q, p->Sq, p->Dr, p->position_rounding, qtab, s);
@@ -865,14 +867,19 @@ static int bwd_impl(const pe_attn_params* p, const pe_tensor_t* qc, const pe_ten
   const bool gm = generic_masked(p, masked);
   const bool do_direct = half_dt(dt) && !gm && v_direct(p, dout, L.dv);
   pb.dO_op = do_direct ? nullptr : bws + L.do_off; pb.op_dtype = L.split ? pe::DT_SPLIT_CODE : p->dtype; pb.width = L.dv;
-  pb.nat = L.split;
   pb.Di = (float*)(bws + L.di_off);
   pb.L2 = (float*)(bws + L.l2_off);
   pb.lse = lse;
   pb.s_pad = L.sq_pad;
   pb.B = p->B; pb.H = p->Hq; pb.S = p->Sq; pb.Dv = p->Dv;
+  // RoPE / no-PE (QKNorm included) at head widths 64 and 128 with vector views: the dQ GEMM and the dK/dV
+  // kernel apply the gradient in their epilogues instead of the stand-alone kernels below (the workspace
+  // still reserves dq~ / dk~: alignment is a call-time fact)
+  const bool rfuse = !gm && half_dt(dt) && (p->mode == PE_MODE_ROPE || p->mode == PE_MODE_NONE) && p->Dc == 0 &&
+                     (p->Dr == 64 || p->Dr == 128) && L.dqk == p->Dr && vec16(qr) && vec16(kr) && vec16(dqr) && vec16(dkr);
+  float* rtab = rfuse && p->mode == PE_MODE_ROPE && p->Dr > 0 ? (float*)(bws + L.rtab_off) : nullptr;
   stage_mark(PE_STAGE_BWD_PRE, 0, s);
-  if ((rc = pe::launch_prebwd(pb, s))) return rc;
+  if ((rc = pe::launch_prebwd(pb, {freqs, rtab, p->Sq, p->Dr / 2, p->start_pos_q, p->position_rounding}, s))) return rc;
   stage_mark(PE_STAGE_BWD_PRE, 1, s);
 
   pe::CoreArgs c = core_args(p, L, fws, v);
@@ -903,11 +910,6 @@ static int bwd_impl(const pe_attn_params* p, const pe_tensor_t* qc, const pe_ten
   // inverse PoPE transform in their epilogues
   const bool split = !gm && fused_split_bwd(p, qr, kr, dqc, dqr, dkc, dkr);
   const bool fuse = (!gm && fused_bwd(p)) || split;
-  // RoPE / no-PE (QKNorm included) at transformed width 64, the reference's head width, with vector
-  // views: the dQ GEMM and the dK/dV kernel apply the gradient in their epilogues instead of the
-  // stand-alone kernels below (the workspace still reserves dq~ / dk~: alignment is a call-time fact)
-  const bool rfuse = !gm && half_dt(dt) && (p->mode == PE_MODE_ROPE || p->mode == PE_MODE_NONE) && p->Dc == 0 &&
-                     p->Dr == 64 && L.dqk == 64 && vec16(qr) && vec16(kr) && vec16(dqr) && vec16(dkr);
   const int nqg = (p->Sq + 255) / 256, nkg = (p->Sk + 127) / 128;
   auto view = [p](pe::EpiPoPE& e, const pe_tensor_t* x, const pe_tensor_t* dx, int start) {
     e.x = x->data; e.x_dtype = x->dtype;
@@ -924,6 +926,8 @@ static int bwd_impl(const pe_attn_params* p, const pe_tensor_t* qc, const pe_ten
     c.freqs = freqs;
     view(c.eq, qr, dqr, p->start_pos_q);
     view(c.ek, kr, dkr, p->start_pos_k);
+    c.eq.tab = rtab;
+    c.ek.tab = p->start_pos_k == p->start_pos_q && p->Sk <= p->Sq ? rtab : nullptr;
   }
   if (fuse) {
     c.fuse_inv = 1;

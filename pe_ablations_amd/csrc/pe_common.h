@@ -186,6 +186,14 @@ template <int XT> struct Raw8 {
       r[0] = *(const u32x4*)((const uint16_t*)p + i);
     }
   }
+  __device__ __forceinline__ void store(void* p, int64_t i) const {
+    if constexpr (XT == 1) {
+      *(u32x4*)((float*)p + i) = r[0];
+      *(u32x4*)((float*)p + i + 4) = r[1];
+    } else {
+      *(u32x4*)((uint16_t*)p + i) = r[0];
+    }
+  }
   __device__ __forceinline__ void get(float (&x)[8]) const {
     if constexpr (XT == 0) unpack8(r[0], x);
     else if constexpr (XT == 2) unpack8_h(r[0], x);
@@ -783,16 +791,23 @@ __device__ __forceinline__ float inv_pope_elem(float x, float pos, float freq, f
 // RoPE (mode 1) or no-PE (mode 2) forward of one pair (x0, x1) of a row, src/model/rope.py:35-57:
 // y = mscale * (x0 cos - x1 sin, x0 sin + x1 cos) at angle fl(pos * inv_freq), or y = x; each product
 // and sum rounded on its own, as torch's ops round them.  cs / sn are kept for the gradient.
+__device__ __forceinline__ void rope_pair_cs(int mode, float x0, float x1, float sn, float cs, float ms, float& y0,
+                                             float& y1) {
+  if (mode == 1) {
+    y0 = sub_nc(mul_nc(x0, cs), mul_nc(x1, sn)) * ms;
+    y1 = add_nc(mul_nc(x0, sn), mul_nc(x1, cs)) * ms;
+  } else {
+    y0 = x0; y1 = x1;
+  }
+}
 __device__ __forceinline__ void rope_pair(int mode, float x0, float x1, float pos, float fr, float ms, float& y0,
                                           float& y1, float& sn, float& cs) {
   if (mode == 1) {
     pe_sincos(mul_nc(pos, fr), sn, cs);
-    y0 = sub_nc(mul_nc(x0, cs), mul_nc(x1, sn)) * ms;
-    y1 = add_nc(mul_nc(x0, sn), mul_nc(x1, cs)) * ms;
   } else {
     sn = 0.f; cs = 1.f;
-    y0 = x0; y1 = x1;
   }
+  rope_pair_cs(mode, x0, x1, sn, cs, ms, y0, y1);
 }
 __device__ __forceinline__ float sq2(float a, float b) { return add_nc(mul_nc(a, a), mul_nc(b, b)); }
 __device__ __forceinline__ float dot2(float a0, float a1, float b0, float b1) {
@@ -826,16 +841,16 @@ __device__ __forceinline__ void l2_coefs(float ss, float zd, float& c1, float& c
 }
 
 // The gradient of one 8-element chunk (pairs 4t .. 4t + 3) of a RoPE / no-PE row through QKNorm: x
-// the raw inputs, g the gradient of the transformed chunk, fr4 the chunk's 4 inverse frequencies
-// (RoPE), tpr threads per row, adjacent and aligned in the wave (QKNorm's row sums by an xor
+// the raw inputs, g the gradient of the transformed chunk, sn / cs the sine and cosine of the pairs' angles
+// (0 and 1 without PE), tpr threads per row, adjacent and aligned in the wave (QKNorm's row sums by an xor
 // butterfly over them).  Every thread of a row group must call it together.
-__device__ __forceinline__ void inv_rope_chunk(int mode, bool l2, const float (&fr4)[4], float pos, float ms, int tpr,
-                                               const float (&x)[8], const float (&g)[8], float (&dx)[8]) {
-  float z[8], sn[4], cs[4];
+__device__ __forceinline__ void inv_rope_chunk(int mode, bool l2, const float (&sn)[4], const float (&cs)[4], float ms,
+                                               int tpr, const float (&x)[8], const float (&g)[8], float (&dx)[8]) {
+  float z[8];
   float ss = 0.f, zd = 0.f;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    rope_pair(mode, x[2 * k], x[2 * k + 1], pos, fr4[k], ms, z[2 * k], z[2 * k + 1], sn[k], cs[k]);
+    rope_pair_cs(mode, x[2 * k], x[2 * k + 1], sn[k], cs[k], ms, z[2 * k], z[2 * k + 1]);
     ss = add_nc(ss, sq2(z[2 * k], z[2 * k + 1]));
     zd = add_nc(zd, dot2(z[2 * k], z[2 * k + 1], g[2 * k], g[2 * k + 1]));
   }
@@ -851,6 +866,14 @@ __device__ __forceinline__ void inv_rope_chunk(int mode, bool l2, const float (&
   for (int k = 0; k < 4; ++k)
     rope_pair_grad(mode, l2, g[2 * k], g[2 * k + 1], z[2 * k], z[2 * k + 1], c1, c2, cs[k], sn[k], ms, dx[2 * k],
                    dx[2 * k + 1]);
+}
+// sine and cosine of the angles fl(pos * freqs[4t + k]), k < 4 (mode 2, no PE: 0 and 1)
+__device__ __forceinline__ void rope_angles4(int mode, const float* freqs, int t, float pos, float (&sn)[4], float (&cs)[4]) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    sn[k] = 0.f; cs[k] = 1.f;
+    if (mode == 1) pe_sincos(mul_nc(pos, freqs[4 * t + k]), sn[k], cs[k]);
+  }
 }
 
 // Launch-order remap.  Blocks are issued heaviest first (LPT for the causal triangle) and, when the

@@ -18,6 +18,7 @@ struct EpiPoPE {
   void* dxc; int dxc_dtype; int64_t dxc_s[4];  // content-part gradient (split form, Dc > 0)
   int start_pos;
   int pos_round;  // PE_POS_* rounding of positions
+  const float* tab;  // fused RoPE gradient: cos / sin of the rows' angles, [S][2][Dr / 2], or null
   float* part_delta;
   float* part_freq;
 };
@@ -80,7 +81,7 @@ struct CoreArgs {
   int fuse_inv; int Dr; int Dc;
   const float* freqs; const float* delta; int64_t delta_hs;
   EpiPoPE eq, ek;
-  // fused RoPE / no-PE gradient (16-bit compute, transformed width 64, no content part, vector views):
+  // fused RoPE / no-PE gradient (16-bit compute, transformed width 64 or 128, no content part, vector views):
   // the dQ GEMM and the dK/dV kernel apply the QKNorm and rotation backward of their staged dq~ / dk~
   // rows and write dq / dk through eq / ek (x, dx, start_pos, pos_round); freqs holds the inverse
   // frequencies.  rope_mode 1 = RoPE, 2 = no PE; rope_l2 = QKNorm; rope_ms = mscale
@@ -119,7 +120,7 @@ int launch_fwd(int dt, int dqk, int dv, const CoreArgs& a, hipStream_t s);
 // fp32 compute on the bf16 matrix cores: q / k / v hold rows of three bf16 planes (DT_SPLIT)
 int launch_fwd_split(int dqk, int dv, const CoreArgs& a, hipStream_t s);
 // its backward, dq~ and dk~ / dV in one launch: dO in planes, L2 holding the
-// natural-unit lse (PreBwdArgs::nat), qsplit any number of ranges of each key block's query tiles
+// natural-unit lse (PreBwdArgs), qsplit any number of ranges of each key block's query tiles
 int launch_bwd_split(int dqk, int dv, const CoreArgs& a, hipStream_t s);
 int launch_bwd_dkdv(int dt, int dqk, int dv, const CoreArgs& a, hipStream_t s);
 int launch_bwd_dq(int dt, int dqk, int dv, const CoreArgs& a, hipStream_t s);
@@ -175,6 +176,9 @@ int launch_prep_qk(const PrepArgs& ak, const PrepArgs& aq, float* tab, hipStream
 // content part or padding, aq.tab null): query threads evaluate each phase once for several heads
 // and the rows of b = 0 write tab; returns 1 without launching when the layout does not qualify
 int launch_prep_k_qheads(const PrepArgs& ak, const PrepArgs& aq, float* tab, hipStream_t s);
+// both sides of a 16-bit RoPE / no-PE prologue (no content part, no padding, vector rows) in one launch that
+// evaluates each angle once for several heads; returns 1 without launching when the layout does not qualify
+int launch_prep_rope_qk(const PrepArgs& ak, const PrepArgs& aq, hipStream_t s);
 // PoPE prologue with the RMSNorm fused in: one workgroup per token (all heads)
 int launch_prep_norm(const PrepArgs& a, hipStream_t s);
 
@@ -239,16 +243,19 @@ int launch_rmsnorm_bwd(NormBwdArgs a, int n_cu, hipStream_t s);
 int launch_swiglu(const void* x, const void* gate, void* out, int64_t n, hipStream_t s);
 
 // dO repack (to compute dtype, width DV, contiguous), Di = rowsum(dO * O) and the log2-scaled
-// lse, both into (B, H, S_pad) arrays whose padding rows hold Di = 0, L2 = +inf.
+// lse, both into (B, H, S_pad) arrays whose padding rows hold Di = 0, L2 = +inf.  With dO_op in planes
+// (op_dtype DT_SPLIT) L2 is the lse itself, in natural units.
 struct PreBwdArgs {
   const void* dout; int dout_dtype; int64_t do_s[4];
   const void* out; int out_dtype; int64_t o_s[4];
   void* dO_op; int op_dtype; int width;
   const float* lse; float* Di; float* L2; int s_pad;
-  int nat;  // L2 holds lse itself (natural units) instead of lse * log2(e)
   int B, H, S, Dv;
 };
-int launch_prebwd(const PreBwdArgs& a, hipStream_t s);
+// a phase table to write beside it: cos / sin of fl(pe_pos(start + s) * freqs[c]) for s < S, c < D into
+// tab [S][2][D]; tab null for none
+struct TabArgs { const float* freqs; float* tab; int S, D, start, pos_round; };
+int launch_prebwd(const PreBwdArgs& a, const TabArgs& t, hipStream_t s);
 
 // Inverse transform: dx~ (fp32, (B,H,S,width)) -> dxc, dxr, plus per-block partial sums of the
 // phase gradient for the key phase bias and for the frequencies.

@@ -89,6 +89,16 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
   for (int c = used + lane; c < a.width; c += 64) row_store(a.dst, drow, a.width, c, a.dst_dtype, 0.f);
 }
 
+__device__ __forceinline__ void phase_table_body(const float* freqs, int start, int S, int Dr, int pos_round,
+                                                 float* tab, int64_t gid) {
+  if (gid >= (int64_t)S * Dr) return;
+  const int s = (int)(gid / Dr), c = (int)(gid % Dr);
+  float sn, cs;
+  pe_sincos(mul_nc(pe_pos(start + s, pos_round), freqs[c]), sn, cs);
+  tab[(int64_t)s * 2 * Dr + c] = cs;
+  tab[(int64_t)s * 2 * Dr + Dr + c] = sn;
+}
+
 // One wave per padded row (b, h, s < S_pad).  Rows s < S: dO repack, Di, L2 = lse*log2(e) (a row
 // without visible keys, lse = -inf, gets +inf so that its probabilities are 0).  Padding rows:
 // Di = 0, L2 = +inf.
@@ -120,7 +130,7 @@ __global__ __launch_bounds__(256) void prebwd_kernel(PreBwdArgs a) {
   if (lane == 0) {
     a.Di[prow] = acc;
     const float lv = a.lse[row];
-    a.L2[prow] = lv == -INFINITY ? INFINITY : (a.nat ? lv : lv * LOG2E);
+    a.L2[prow] = lv == -INFINITY ? INFINITY : (a.op_dtype == DT_SPLIT ? lv : lv * LOG2E);
   }
 }
 
@@ -336,10 +346,18 @@ __device__ __forceinline__ void prep_pope_vec_body(const PrepArgs& a, int64_t gi
   row_store8(a.dst, drow, a.width, a.Dc + a.Dr + t * 8, DT, sv);
   if (a.Dc > 0) {
     const int64_t xc0 = b * a.xc_s[0] + h * a.xc_s[1] + (int64_t)s * a.xc_s[2];
-    for (int j = t; j < a.Dc / 8; j += tpr) {
-      float c[8];
-      load8(a.xc, xc0 + j * 8, a.xc_dtype, c);
-      row_store8(a.dst, drow, a.width, j * 8, DT, c);
+    if (DT != DT_SPLIT && a.xc_dtype == DT) {
+      for (int j = t; j < a.Dc / 8; j += tpr) {
+        Raw8<DT == DT_SPLIT ? 1 : DT> c;
+        c.load(a.xc, xc0 + j * 8);
+        c.store(a.dst, drow * a.width + j * 8);
+      }
+    } else {
+      for (int j = t; j < a.Dc / 8; j += tpr) {
+        float c[8];
+        load8(a.xc, xc0 + j * 8, a.xc_dtype, c);
+        row_store8(a.dst, drow, a.width, j * 8, DT, c);
+      }
     }
   }
   const float zero[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -402,8 +420,7 @@ template <int HT> __global__ __launch_bounds__(256) void prep_pope_small_kernel(
 // one group of TPR = Dv / 8 lanes per padded row (TPR a power of two, groups never straddle a
 // wave); Di is the group's fixed-order butterfly sum.  XT: the element type of dO and
 // out, OT that of the repacked rows
-template <int XT, int OT> __global__ __launch_bounds__(256) void prebwd_vec_kernel(PreBwdArgs a, int lg_tpr) {
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
+template <int XT, int OT> __device__ __forceinline__ void prebwd_vec_body(const PreBwdArgs& a, int lg_tpr, int64_t gid) {
   const int64_t prow = gid >> lg_tpr;
   const int t = (int)(gid & ((1 << lg_tpr) - 1));
   if (prow >= (int64_t)a.B * a.H * a.s_pad) return;
@@ -416,9 +433,15 @@ template <int XT, int OT> __global__ __launch_bounds__(256) void prebwd_vec_kern
   const int h = bh % a.H, b = bh / a.H;
   const int64_t row = (int64_t)bh * a.S + s;
   float d[8], o[8];
-  load8(a.dout, b * a.do_s[0] + h * a.do_s[1] + (int64_t)s * a.do_s[2] + t * 8, XT, d);
-  load8(a.out, b * a.o_s[0] + h * a.o_s[1] + (int64_t)s * a.o_s[2] + t * 8, XT, o);
-  if (a.dO_op) row_store8(a.dO_op, row, a.width, t * 8, OT, d);
+  Raw8<XT> rd, ro;
+  rd.load(a.dout, b * a.do_s[0] + h * a.do_s[1] + (int64_t)s * a.do_s[2] + t * 8);
+  ro.load(a.out, b * a.o_s[0] + h * a.o_s[1] + (int64_t)s * a.o_s[2] + t * 8);
+  rd.get(d);
+  ro.get(o);
+  if (a.dO_op) {
+    if constexpr (OT == XT) rd.store(a.dO_op, row * a.width + t * 8);
+    else row_store8(a.dO_op, row, a.width, t * 8, OT, d);
+  }
   float acc = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc += d[e] * o[e];
@@ -426,8 +449,17 @@ template <int XT, int OT> __global__ __launch_bounds__(256) void prebwd_vec_kern
   if (t == 0) {
     a.Di[prow] = acc;
     const float lv = a.lse[row];
-    a.L2[prow] = lv == -INFINITY ? INFINITY : (a.nat ? lv : lv * LOG2E);
+    a.L2[prow] = lv == -INFINITY ? INFINITY : (OT == DT_SPLIT ? lv : lv * LOG2E);
   }
+}
+
+template <int XT, int OT> __global__ __launch_bounds__(256) void prebwd_vec_kernel(PreBwdArgs a, int lg_tpr) {
+  prebwd_vec_body<XT, OT>(a, lg_tpr, (int64_t)blockIdx.x * 256 + threadIdx.x);
+}
+// ... and the phase table, in the blocks from nblk on (16-bit rows, where the fused RoPE gradient reads it)
+template <int HT> __global__ __launch_bounds__(256) void prebwd_tab_kernel(PreBwdArgs a, int lg_tpr, unsigned nblk, TabArgs t) {
+  if (blockIdx.x < nblk) prebwd_vec_body<HT, HT>(a, lg_tpr, (int64_t)blockIdx.x * 256 + threadIdx.x);
+  else phase_table_body(t.freqs, t.start, t.S, t.D, t.pos_round, t.tab, (int64_t)(blockIdx.x - nblk) * 256 + threadIdx.x);
 }
 
 // RoPE / no-PE prologue and its gradient, vector form: thread t of a row owns elements 8t .. 8t + 7
@@ -476,6 +508,52 @@ __global__ __launch_bounds__(256) void prep_rope_vec_kernel(PrepArgs a, int lg_t
   for (int j = (a.Dc + a.Dr) / 8 + t; j < a.width / 8; j += tpr) row_store8(a.dst, drow, a.width, j * 8, a.dst_dtype, zero);
 }
 
+// Both sides of a RoPE / no-PE prologue without a content part in one launch, RHG heads per thread: thread
+// (b, head group, s, chunk t) loads its chunk of the group's heads, evaluates the sine and cosine of its 4
+// angles once and transforms them all.  Blocks below nkblk take key rows.  Per element, and in QKNorm's
+// sums, the arithmetic is prep_rope_vec_kernel's: bitwise equal rows.  4 x 2048 rows of 16 -> 4 heads of
+// 128: 41 us in two launches that evaluate every angle per head, 29 in this one.
+constexpr int RHG = 4;
+template <int DT> __device__ __forceinline__ void prep_rope_heads_body(const PrepArgs& a, int lg_tpr, int64_t gid) {
+  const int tpr = 1 << lg_tpr, t = (int)(gid & (tpr - 1)), ngrp = (a.H + RHG - 1) / RHG;
+  const int64_t unit = gid >> lg_tpr;
+  if (unit >= (int64_t)a.B * ngrp * a.S) return;  // whole row groups
+  const int s = (int)(unit % a.S), bg = (int)(unit / a.S);
+  const int h0 = bg % ngrp * RHG, b = bg / ngrp;
+  const int64_t xb = b * a.xr_s[0] + (int64_t)s * a.xr_s[2] + t * 8;
+  Raw8<DT> xv[RHG];
+#pragma unroll
+  for (int j = 0; j < RHG; ++j)
+    if (h0 + j < a.H) xv[j].load(a.xr, xb + (int64_t)(h0 + j) * a.xr_s[1]);
+  float sn[4], cs[4];
+  rope_angles4(a.mode, a.freqs, t, pe_pos(a.start_pos + s, a.pos_round), sn, cs);
+#pragma unroll
+  for (int j = 0; j < RHG; ++j) {
+    const int h = h0 + j;
+    if (h >= a.H) break;  // the same for the row's threads
+    float x[8], y[8];
+    xv[j].get(x);
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      rope_pair_cs(a.mode, x[2 * k], x[2 * k + 1], sn[k], cs[k], a.mscale, y[2 * k], y[2 * k + 1]);
+      ss = add_nc(ss, sq2(y[2 * k], y[2 * k + 1]));
+    }
+    if (a.l2norm) {
+      for (int m = tpr >> 1; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+      const float den = sqrtf(ss) + 1e-6f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = y[e] / den;
+    }
+    store8(a.dst, ((int64_t)(b * a.H + h) * a.S + s) * a.width + t * 8, DT, y);
+  }
+}
+template <int DT>
+__global__ __launch_bounds__(256) void prep_rope_qk_kernel(PrepArgs ak, PrepArgs aq, unsigned nkblk, int lg_tpr) {
+  if (blockIdx.x < nkblk) prep_rope_heads_body<DT>(ak, lg_tpr, (int64_t)blockIdx.x * 256 + threadIdx.x);
+  else prep_rope_heads_body<DT>(aq, lg_tpr, (int64_t)(blockIdx.x - nkblk) * 256 + threadIdx.x);
+}
+
 __global__ __launch_bounds__(256) void inv_rope_vec_kernel(InvArgs a, int lg_tpr) {
   const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int tpr = 1 << lg_tpr;
@@ -495,12 +573,11 @@ __global__ __launch_bounds__(256) void inv_rope_vec_kernel(InvArgs a, int lg_tpr
       store8(a.dxc, dc0 + j * 8, a.dxc_dtype, c);
     }
   }
-  float x[8], gv[8], dx[8], fr4[4];
+  float x[8], gv[8], dx[8], sn[4], cs[4];
   load8(a.xr, b * a.xr_s[0] + h * a.xr_s[1] + (int64_t)s * a.xr_s[2] + t * 8, a.xr_dtype, x);
   load8(grow, a.Dc + t * 8, 1, gv);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) fr4[k] = a.mode == 1 ? a.freqs[4 * t + k] : 0.f;
-  inv_rope_chunk(a.mode, a.l2norm != 0, fr4, pos, a.mscale, tpr, x, gv, dx);
+  rope_angles4(a.mode, a.freqs, t, pos, sn, cs);
+  inv_rope_chunk(a.mode, a.l2norm != 0, sn, cs, a.mscale, tpr, x, gv, dx);
   store8(a.dxr, b * a.dxr_s[0] + h * a.dxr_s[1] + (int64_t)s * a.dxr_s[2] + t * 8, a.dxr_dtype, dx);
 }
 
@@ -604,16 +681,6 @@ int launch_prep(const PrepArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(prep_kernel, dim3((unsigned)((nrows + 3) / 4)), dim3(256), 0, s, a);
   }
   return hipGetLastError() == hipSuccess ? 0 : -7;
-}
-
-__device__ __forceinline__ void phase_table_body(const float* freqs, int start, int S, int Dr, int pos_round,
-                                                 float* tab, int64_t gid) {
-  if (gid >= (int64_t)S * Dr) return;
-  const int s = (int)(gid / Dr), c = (int)(gid % Dr);
-  float sn, cs;
-  pe_sincos(mul_nc(pe_pos(start + s, pos_round), freqs[c]), sn, cs);
-  tab[(int64_t)s * 2 * Dr + c] = cs;
-  tab[(int64_t)s * 2 * Dr + Dr + c] = sn;
 }
 
 __global__ __launch_bounds__(256) void phase_table_kernel(const float* freqs, int start, int S, int Dr, int pos_round,
@@ -727,6 +794,23 @@ int launch_prep_k_qheads(const PrepArgs& ak, const PrepArgs& aq, float* tab, hip
   return hipGetLastError() == hipSuccess ? 0 : -7;
 }
 
+int launch_prep_rope_qk(const PrepArgs& ak, const PrepArgs& aq, hipStream_t s) {
+  const int lg = prep_rope_vec_lg(ak);
+  auto ok = [](const PrepArgs& a) {
+    return a.Dc == 0 && a.width == a.Dr && a.dst_rows == 0 && a.dst_row0 == 0 && a.xr_dtype == a.dst_dtype &&
+           (a.dst_dtype == 0 || a.dst_dtype == 2);
+  };
+  if (lg < 0 || prep_rope_vec_lg(aq) != lg || !ok(ak) || !ok(aq) || ak.dst_dtype != aq.dst_dtype) return 1;
+  auto blocks = [lg](const PrepArgs& a) { return ((((int64_t)a.B * ((a.H + RHG - 1) / RHG) * a.S) << lg) + 255) / 256; };
+  const int64_t nk = blocks(ak), nq = blocks(aq);
+  if (nk == 0 || nq == 0) return 1;
+  if (nk + nq > 0x7fffffff) return -2;
+  const dim3 grid((unsigned)(nk + nq));
+  if (ak.dst_dtype == 0) hipLaunchKernelGGL(prep_rope_qk_kernel<0>, grid, dim3(256), 0, s, ak, aq, (unsigned)nk, lg);
+  else hipLaunchKernelGGL(prep_rope_qk_kernel<2>, grid, dim3(256), 0, s, ak, aq, (unsigned)nk, lg);
+  return hipGetLastError() == hipSuccess ? 0 : -7;
+}
+
 int launch_prep_qk(const PrepArgs& ak, const PrepArgs& aq, float* tab, hipStream_t s) {
   if (!prep_vec_ok(ak) || !prep_vec_ok(aq) || prep_vec_types(ak) != prep_vec_types(aq) || ak.cdst || aq.cdst ||
       aq.tab || !ak.is_key || aq.is_key || aq.Dr != ak.Dr)
@@ -766,7 +850,7 @@ int launch_phase_table(const float* freqs, int start, int S, int Dr, int pos_rou
   return hipGetLastError() == hipSuccess ? 0 : -7;
 }
 
-int launch_prebwd(const PreBwdArgs& a, hipStream_t s) {
+int launch_prebwd(const PreBwdArgs& a, const TabArgs& t, hipStream_t s) {
   const int tpr = a.Dv / 8;
   const bool vec = a.dout_dtype == a.out_dtype && a.Dv % 8 == 0 && tpr <= 64 && (tpr & (tpr - 1)) == 0 &&
                    rows16(a.dout, a.dout_dtype, a.do_s) && rows16(a.out, a.out_dtype, a.o_s) &&
@@ -775,7 +859,16 @@ int launch_prebwd(const PreBwdArgs& a, hipStream_t s) {
   if (vec) {
     int lg = 0;
     while ((1 << lg) < tpr) ++lg;
-    const dim3 grid((unsigned)((nrows * tpr + 255) / 256));
+    const unsigned nblk = (unsigned)((nrows * tpr + 255) / 256);
+    const dim3 grid(nblk), tgrid(nblk + (unsigned)(((int64_t)t.S * t.D + 255) / 256));
+    if (t.tab && a.dout_dtype == 0) {
+      hipLaunchKernelGGL(prebwd_tab_kernel<0>, tgrid, dim3(256), 0, s, a, lg, nblk, t);
+      return hipGetLastError() == hipSuccess ? 0 : -7;
+    }
+    if (t.tab && a.dout_dtype == 2) {
+      hipLaunchKernelGGL(prebwd_tab_kernel<2>, tgrid, dim3(256), 0, s, a, lg, nblk, t);
+      return hipGetLastError() == hipSuccess ? 0 : -7;
+    }
     if (a.dout_dtype == 0) hipLaunchKernelGGL((prebwd_vec_kernel<0, 0>), grid, dim3(256), 0, s, a, lg);
     else if (a.dout_dtype == 2) hipLaunchKernelGGL((prebwd_vec_kernel<2, 2>), grid, dim3(256), 0, s, a, lg);
     else if (a.op_dtype != DT_SPLIT) hipLaunchKernelGGL((prebwd_vec_kernel<1, 1>), grid, dim3(256), 0, s, a, lg);
@@ -783,6 +876,7 @@ int launch_prebwd(const PreBwdArgs& a, hipStream_t s) {
   } else {
     hipLaunchKernelGGL(prebwd_kernel, dim3((unsigned)((nrows + 3) / 4)), dim3(256), 0, s, a);
   }
+  if (t.tab) return launch_phase_table(t.freqs, t.start, t.S, t.D, t.pos_round, t.tab, s);
   return hipGetLastError() == hipSuccess ? 0 : -7;
 }
 
