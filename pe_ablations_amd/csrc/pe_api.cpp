@@ -872,11 +872,11 @@ static int bwd_impl(const pe_attn_params* p, const pe_tensor_t* qc, const pe_ten
   pb.lse = lse;
   pb.s_pad = L.sq_pad;
   pb.B = p->B; pb.H = p->Hq; pb.S = p->Sq; pb.Dv = p->Dv;
-  // RoPE / no-PE (QKNorm included) at head widths 64 and 128 with vector views: the dQ GEMM and the dK/dV
+  // RoPE / no-PE (QKNorm included) at head widths 64 and, with values as wide, 128 and vector views: the dQ GEMM and the dK/dV
   // kernel apply the gradient in their epilogues instead of the stand-alone kernels below (the workspace
   // still reserves dq~ / dk~: alignment is a call-time fact)
   const bool rfuse = !gm && half_dt(dt) && (p->mode == PE_MODE_ROPE || p->mode == PE_MODE_NONE) && p->Dc == 0 &&
-                     (p->Dr == 64 || p->Dr == 128) && L.dqk == p->Dr && vec16(qr) && vec16(kr) && vec16(dqr) && vec16(dkr);
+                     (p->Dr == 64 || (p->Dr == 128 && L.dv == 128)) && L.dqk == p->Dr && vec16(qr) && vec16(kr) && vec16(dqr) && vec16(dkr);
   float* rtab = rfuse && p->mode == PE_MODE_ROPE && p->Dr > 0 ? (float*)(bws + L.rtab_off) : nullptr;
   stage_mark(PE_STAGE_BWD_PRE, 0, s);
   if ((rc = pe::launch_prebwd(pb, {freqs, rtab, p->Sq, p->Dr / 2, p->start_pos_q, p->position_rounding}, s))) return rc;

@@ -822,7 +822,7 @@ __device__ __forceinline__ void content_rows(const EpiPoPE& e, const float* st, 
 // transform of the staged rows st_epi[128 keys][DQK] (fp32, scaled) of key block kb of (b, hk)
 // into dk (and the content part's copy into dk_c), plus the block's phase-gradient partials at
 // index bh * nkb + kb; or the RoPE gradient of those rows.  Only with a.fuse_inv or a.rope_fuse set.
-template <int HT, int DQK>
+template <int HT, int DQK, int DV>
 __device__ __forceinline__ void dk_epilogue(const CoreArgs& a, float* st_epi, int tid, int b, int hk, int kb,
                                             int bh, int nkb) {
   constexpr int NW = 8, BNK = 128;
@@ -867,8 +867,9 @@ __device__ __forceinline__ void dk_epilogue(const CoreArgs& a, float* st_epi, in
       }
     }
   };
-  if (DQK == 128 && a.rope_fuse) {  // RoPE / no-PE at head width 128
-    if constexpr (DQK == 128)
+  constexpr bool RP = DQK == 128 && DV == 128;
+  if (RP && a.rope_fuse) {  // RoPE / no-PE at head width 128
+    if constexpr (RP)
       rope_epi_rows<HT, DQK, NW * 64, BNK>(a, a.ek, st_epi, tid, k0, a.Sk, b, hk, [] { __syncthreads(); });
   } else if (DQK == 128 && a.fuse_inv && a.Dc == DQK / 2) {  // split form: fused only at width 128, vector views
     if constexpr (DQK == 128) epi_vec(std::integral_constant<int, DQK / 2>{});
@@ -1368,7 +1369,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_pair_kernel(CoreArgs a) {
       if (t < niter) scores_dp(smem + (t % NSTG) * STAGE + SQ_BYTES + rro, vf, dp);
       __syncthreads();  // role A waited for tile t + 1's loads before this barrier
     }
-    if ((a.fuse_inv || a.rope_fuse) && !QS) {
+    if ((a.fuse_inv || (DQK == 128 && DV == 128 && a.rope_fuse)) && !QS) {
 #pragma unroll
       for (int t = 0; t < NDK; ++t)
 #pragma unroll
@@ -1385,7 +1386,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_pair_kernel(CoreArgs a) {
     }
   }
 
-  if constexpr (!QS) dk_epilogue<HT, DQK>(a, st_epi, tid, b, hk, kb, bh, nkb);
+  if constexpr (!QS) dk_epilogue<HT, DQK, DV>(a, st_epi, tid, b, hk, kb, bh, nkb);
 }
 
 // The query split of the pair kernel (a.qsplit > 1, see key_split in pe_api.cpp): one workgroup of 512 threads per key block of (b, hk) adds the qsplit fp32 partials of
@@ -1404,7 +1405,7 @@ __device__ __forceinline__ void dkdv_combine(const CoreArgs& a, int blk_id, floa
   bh += a.bh0;
   const int b = bh / a.Hkv, hk = bh % a.Hkv, k0 = kb * BNK;
   const int64_t units = (int64_t)a.B * a.Hkv;
-  const bool fuse = a.fuse_inv || a.rope_fuse;
+  const bool fuse = a.fuse_inv || (DQK == 128 && DV == 128 && a.rope_fuse);
   for (int i = tid; i < BNK * (DV / 4); i += NT) {
     const int r = i / (DV / 4), c = (i % (DV / 4)) * 4, key = k0 + r;
     if (key >= a.Sk) continue;
@@ -1426,7 +1427,7 @@ __device__ __forceinline__ void dkdv_combine(const CoreArgs& a, int blk_id, floa
     }
     if (fuse) *(f32x4*)(st_epi + r * DQK + c) = sum;
   }
-  if (fuse) dk_epilogue<HT, DQK>(a, st_epi, tid, b, hk, kb, bh, nkb);
+  if (fuse) dk_epilogue<HT, DQK, DV>(a, st_epi, tid, b, hk, kb, bh, nkb);
 }
 
 // dQ~ = dS k~ as a GEMM over the dS^T rows the dK/dV kernel stored (no score recompute).  A

@@ -294,7 +294,7 @@ __global__ __launch_bounds__(RW * 64) void reduce_kernel(ReduceArgs a) {
 // ... and zero padding chunks the same way; TPR = Dr / 8
 // tab_out (query side, phases evaluated here): the rows of (b, h) = (0, 0) also write their cos /
 // sin to the [S][2][Dr] phase table, the values launch_phase_table would write.  XT / DT: element types
-// of the raw positional rows and of the operand rows (the content rows' type is read at run time)
+// of the raw positional rows and of the operand rows (content rows: the same type, or read at run time)
 template <int XT, int DT>
 __device__ __forceinline__ void prep_pope_vec_body(const PrepArgs& a, int64_t gid, float* tab_out = nullptr) {
   const int tpr = a.Dr >> 3;
@@ -346,9 +346,9 @@ __device__ __forceinline__ void prep_pope_vec_body(const PrepArgs& a, int64_t gi
   row_store8(a.dst, drow, a.width, a.Dc + a.Dr + t * 8, DT, sv);
   if (a.Dc > 0) {
     const int64_t xc0 = b * a.xc_s[0] + h * a.xc_s[1] + (int64_t)s * a.xc_s[2];
-    if (DT != DT_SPLIT && a.xc_dtype == DT) {
+    if constexpr (XT == DT) {  // content rows of the same type (prep_vec_ok)
       for (int j = t; j < a.Dc / 8; j += tpr) {
-        Raw8<DT == DT_SPLIT ? 1 : DT> c;
+        Raw8<XT> c;
         c.load(a.xc, xc0 + j * 8);
         c.store(a.dst, drow * a.width + j * 8);
       }
@@ -644,7 +644,7 @@ static bool prep_vec_ok(const PrepArgs& a) {
   return a.mode == 0 && prep_vec_types(a) >= 0 && a.Dr > 0 && a.Dr % 8 == 0 && a.Dc % 8 == 0 && a.width % 8 == 0 &&
          rows16(a.xr, a.xr_dtype, a.xr_s) && ((uintptr_t)a.dst % 16) == 0 && ((uintptr_t)a.freqs % 16) == 0 &&
          (!a.is_key || !a.delta || (((uintptr_t)a.delta % 16) == 0 && a.delta_hs % 4 == 0)) &&
-         (a.Dc == 0 || rows16(a.xc, a.xc_dtype, a.xc_s));
+         (a.Dc == 0 || (rows16(a.xc, a.xc_dtype, a.xc_s) && (a.xr_dtype != a.dst_dtype || a.xc_dtype == a.dst_dtype)));
 }
 
 bool prep_vec_copy_ok(const PrepArgs& a) {
