@@ -296,6 +296,9 @@ int pe_rmsnorm_bwd(const void* x, int32_t x_dtype, int64_t x_row_stride, int64_t
  * aligned pointers (out may alias x or gate).  Forward only: the module calls it when no gradient
  * is needed. */
 int pe_swiglu_fwd(const void* x, const void* gate, void* out, int64_t n, void* stream);
+/* Its gradients for the output gradient dy, as autograd computes them through the two torch ops:
+ * dx = dy * silu(gate), dgate = (dy * x) * silu'(gate); same layout and alignment. */
+int pe_swiglu_bwd(const void* x, const void* gate, const void* dy, void* dx, void* dgate, int64_t n, void* stream);
 
 /* Elementwise positional prologue on its own (the HBM-bound half of the forward): writes the
  * transformed rows [content | transform | zero pad] of x into dst (B,H,S,width) contiguous in

@@ -32,7 +32,7 @@ EXPORTED = [
     "pe_attn_set_stage_events", "pe_attn_transform_bwd_workspace_bytes", "pe_attn_transform_bwd",
     "pe_attn_fwd_normed", "pe_rmsnorm_fwd", "pe_attn_fwd_noalloc", "pe_attn_noalloc_scratch_bytes",
     "pe_attn_value_width", "pe_attn_cache_append", "pe_attn_decode_workspace_bytes", "pe_attn_decode",
-    "pe_swiglu_fwd", "pe_rmsnorm_bwd_workspace_bytes", "pe_rmsnorm_bwd", "pe_attn_fwd_masked",
+    "pe_swiglu_fwd", "pe_swiglu_bwd", "pe_rmsnorm_bwd_workspace_bytes", "pe_rmsnorm_bwd", "pe_attn_fwd_masked",
     "pe_attn_bwd_masked", "pe_attn_bwd_masked_workspace_bytes",
 ]
 
@@ -133,6 +133,8 @@ def lib():
             L.pe_rmsnorm_bwd.restype = ctypes.c_int
             L.pe_swiglu_fwd.argtypes = [vp, vp, vp, i64, vp]
             L.pe_swiglu_fwd.restype = ctypes.c_int
+            L.pe_swiglu_bwd.argtypes = [vp, vp, vp, vp, vp, i64, vp]
+            L.pe_swiglu_bwd.restype = ctypes.c_int
             L.pe_attn_fwd_noalloc.argtypes = [P, T, T, T, T, T, vp, vp, T, vp, vp]
             L.pe_attn_fwd_noalloc.restype = ctypes.c_int
             L.pe_attn_noalloc_scratch_bytes.argtypes = []

@@ -822,6 +822,15 @@ int pe_swiglu_fwd(const void* x, const void* gate, void* out, int64_t n, void* s
   return pe::launch_swiglu(x, gate, out, n, (hipStream_t)stream);
 }
 
+int pe_swiglu_bwd(const void* x, const void* gate, const void* dy, void* dx, void* dgate, int64_t n, void* stream) {
+  if (!x || !gate || !dy || !dx || !dgate) return PE_ERR_NULL;
+  if (n < 0 || n % 8 != 0) return PE_ERR_SHAPE;
+  if (((uintptr_t)x | (uintptr_t)gate | (uintptr_t)dy | (uintptr_t)dx | (uintptr_t)dgate) % 16) return PE_ERR_STRIDE;
+  const int rc = device_ok();
+  if (rc) return rc;
+  return pe::launch_swiglu_bwd(x, gate, dy, dx, dgate, n, (hipStream_t)stream);
+}
+
 }  // extern "C"
 
 static int bwd_impl(const pe_attn_params* p, const pe_tensor_t* qc, const pe_tensor_t* qr,

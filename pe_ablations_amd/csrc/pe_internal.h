@@ -240,6 +240,8 @@ struct NormBwdArgs {
 int64_t rmsnorm_bwd_part_floats(int64_t rows, int n, int n_cu);
 int launch_rmsnorm_bwd(NormBwdArgs a, int n_cu, hipStream_t s);
 // silu(gate) * x over n bf16 elements (n % 8 == 0, 16-byte aligned pointers)
+// and its gradients: dx = dy silu(gate), dgate = (dy x) silu'(gate)
+int launch_swiglu_bwd(const void* x, const void* gate, const void* dy, void* dx, void* dgate, int64_t n, hipStream_t s);
 int launch_swiglu(const void* x, const void* gate, void* out, int64_t n, hipStream_t s);
 
 // dO repack (to compute dtype, width DV, contiguous), Di = rowsum(dO * O) and the log2-scaled

@@ -654,6 +654,71 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.
     return y.view(*x.shape[:-1], n)
 
 
+def plain_autograd(*tensors: torch.Tensor) -> bool:
+    """Whether ordinary eager autograd is all that looks at these tensors, so that one fused Function may
+    stand for a chain of torch ops: plain CUDA tensors, no functorch transform (vmap, jvp, grad), no
+    forward-mode level, no tracing or compiling, and no dispatch or function mode that would see the ops."""
+    return (all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing())
+
+
+def rms_norm_expression(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """The reference module's torch expression (src/model/normalization.py:22-27)."""
+    xf = x.float()
+    return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps)).type_as(x) * weight
+
+
+class RMSNormFn(torch.autograd.Function):
+    """rms_norm with pe_rmsnorm_bwd as its backward (one launch forward, two backward, in place of the
+    expression's six and about twelve).  Under create_graph the backward differentiates the torch
+    expression instead, so higher derivatives are those of the expression."""
+
+    @staticmethod
+    def forward(ctx, x, weight, eps):
+        ctx.save_for_backward(x, weight)
+        ctx.eps = eps
+        return rms_norm(x, weight, eps)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            y = rms_norm_expression(x, weight, ctx.eps)
+            need = [t for t, n in zip((x, weight), ctx.needs_input_grad) if n]
+            grads = iter(torch.autograd.grad(y, need, dy, create_graph=True))
+            return tuple(next(grads) if n else None for n in ctx.needs_input_grad[:2]) + (None,)
+        return rms_norm_backward(x, weight, dy, ctx.eps) + (None,)
+
+
+class SwiGLUFn(torch.autograd.Function):
+    """swiglu (bf16) with pe_swiglu_bwd as its backward; under create_graph the backward differentiates
+    F.silu(gate) * x."""
+
+    @staticmethod
+    def forward(ctx, x, gate):
+        ctx.save_for_backward(x, gate)
+        return swiglu(x, gate)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, gate = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            need = [t for t, n in zip((x, gate), ctx.needs_input_grad) if n]
+            grads = iter(torch.autograd.grad(torch.nn.functional.silu(gate) * x, need, dy, create_graph=True))
+            return tuple(next(grads) if n else None for n in ctx.needs_input_grad)
+        xc, gc, dc = x.contiguous(), gate.contiguous(), dy.contiguous()
+        if any(t.data_ptr() % 16 for t in (xc, gc, dc)):
+            xc, gc, dc = (t.clone(memory_format=torch.contiguous_format) for t in (xc, gc, dc))
+        dx, dg = torch.empty_like(xc), torch.empty_like(xc)
+        with _on(x.device):
+            _lib.check(_lib.lib().pe_swiglu_bwd(xc.data_ptr(), gc.data_ptr(), dc.data_ptr(), dx.data_ptr(), dg.data_ptr(),
+                                                xc.numel(), _stream(x.device)))
+        return dx, dg
+
+
 def swiglu(x: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     """F.silu(gate) * x over bf16 through pe_swiglu_fwd (src/model/ffn.py:17-27), bitwise torch's
     result for the two bf16 ops, in one pass.  Both tensors bf16, same shape, on the GPU.  No

@@ -2,9 +2,9 @@
 
 RMSNorm: x * rsqrt(mean(x^2) + eps) in fp32, cast back to x's dtype, times the weight (which
 promotes the result to fp32 when the weight is fp32, the precision the PoPE transform then sees).
-When no gradient is needed and the tensor is on the GPU it runs the library's one-pass HIP kernel
-(pe_rmsnorm_fwd); in training it is the reference's torch expression, whose autograd gives the
-backward.  On the position projections of the PoPE attention, inference skips the module
+On the GPU it runs the library's one-pass HIP kernel (pe_rmsnorm_fwd), in training with
+pe_rmsnorm_bwd as its backward (RMSNormFn); elsewhere, and where something other than plain autograd
+looks at the ops (functorch, forward mode, tracing), it is the reference's torch expression.  On the position projections of the PoPE attention, inference skips the module
 altogether: the norm is fused into the attention's transform kernel.  QKNorm is fused into the
 attention kernel for the RoPE / no-PE modules (qk_l2norm); the module form here serves direct
 callers.
@@ -13,6 +13,7 @@ callers.
 import torch
 import torch.nn as nn
 
+from .functional import RMSNormFn, plain_autograd
 from .functional import rms_norm as _hip_rms_norm
 
 _HIP_NORM_MAX = 8192
@@ -29,10 +30,12 @@ class RMSNorm(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         n = x.shape[-1]
-        if (x.is_cuda and not torch.is_grad_enabled() and n % 8 == 0 and n <= _HIP_NORM_MAX
-                and x.dtype in (torch.bfloat16, torch.float32)
+        if (x.is_cuda and n % 8 == 0 and n <= _HIP_NORM_MAX and x.dtype in (torch.bfloat16, torch.float32)
                 and self.weight.dtype in (torch.bfloat16, torch.float32)):
-            return _hip_rms_norm(x, self.weight, self.eps)
+            if not torch.is_grad_enabled():
+                return _hip_rms_norm(x, self.weight, self.eps)
+            if self.weight.shape == (n,) and self.weight.device == x.device and plain_autograd(x, self.weight):
+                return RMSNormFn.apply(x, self.weight, self.eps)
         return self._norm(x.float()).type_as(x) * self.weight
 
 
