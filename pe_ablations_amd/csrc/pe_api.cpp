@@ -481,17 +481,16 @@ static int fwd_impl(const pe_attn_params* p, const pe_norm_params* nrm, const pe
   stage_mark(PE_STAGE_FWD_PREP, 0, s);
   float* qtab = use_qtab(p) ? (float*)(ws + L.tab_off) : nullptr;
   if (nrm) {
-    if (qtab && (rc = pe::launch_phase_table(freqs, p->start_pos_q, p->Sq, p->Dr, p->position_rounding, qtab, s)))
-      return rc;
-    fill_prep(a, p, 0, qc, qr, freqs, nullptr, ws + L.q_off, L.dqk);
-    a.dst_dtype = opd;
-    a.tab = qtab;
-    a.norm_w = nrm->q_weight; a.norm_w_dtype = nrm->weight_dtype; a.norm_eps = nrm->eps;
-    if ((rc = pe::launch_prep_norm(a, s))) return rc;
+    pe::PrepArgs aq;
+    fill_prep(aq, p, 0, qc, qr, freqs, nullptr, ws + L.q_off, L.dqk);
+    aq.norm_w = nrm->q_weight;
     fill_prep(a, p, 1, kc, kr, freqs, delta, ws + L.k_off, L.dqk);
-    a.dst_dtype = opd;
-    a.norm_w = nrm->k_weight; a.norm_w_dtype = nrm->weight_dtype; a.norm_eps = nrm->eps;
-    if ((rc = pe::launch_prep_norm(a, s))) return rc;
+    a.norm_w = nrm->k_weight;
+    for (pe::PrepArgs* x : {&aq, &a}) {
+      x->dst_dtype = opd;
+      x->norm_w_dtype = nrm->weight_dtype; x->norm_eps = nrm->eps;
+    }
+    if ((rc = pe::launch_prep_norm(aq, a, qtab, s))) return rc;
   } else {
     // small shapes: both sides in one launch; larger ones without a content part: both sides in
     // one launch with each query phase evaluated once for several heads; else keys first, with the

@@ -179,8 +179,9 @@ int launch_prep_k_qheads(const PrepArgs& ak, const PrepArgs& aq, float* tab, hip
 // both sides of a 16-bit RoPE / no-PE prologue (no content part, no padding, vector rows) in one launch that
 // evaluates each angle once for several heads; returns 1 without launching when the layout does not qualify
 int launch_prep_rope_qk(const PrepArgs& ak, const PrepArgs& aq, hipStream_t s);
-// PoPE prologue with the RMSNorm fused in: one workgroup per token (all heads)
-int launch_prep_norm(const PrepArgs& a, hipStream_t s);
+// both sides of the PoPE prologue with the RMSNorm fused in, one wave per token (all heads), and the query
+// phase table (tab, may be null)
+int launch_prep_norm(const PrepArgs& aq, const PrepArgs& ak, float* tab, hipStream_t s);
 
 // Attention of Sq new query rows (transformed, (B, Hq, Sq, DQK) contiguous) against the first L
 // rows of a cache of transformed keys (B, Hkv, cap, DQK) and values (B, Hkv, cap, DV), split over

@@ -15,6 +15,8 @@
 // squares is reduced by the wave's xor butterfly, which leaves the same value in every lane and
 // depends on nothing but the row, so no LDS and no barrier are involved and the waves of a
 // workgroup (rows of their own) never wait for each other.
+#include <algorithm>
+
 #include "pe_common.h"
 #include "pe_internal.h"
 
@@ -77,10 +79,12 @@ __global__ __launch_bounds__(WPB * 64) void rmsnorm_kernel(NormArgs a) {
   }
 }
 
+// tab_out (query side): the first batch entry's tokens also write their first head's cos / sin to the
+// [S][2][Dr] phase table
 template <int DDT, int CPL>
-__global__ __launch_bounds__(WPB * 64) void prep_pope_norm_kernel(PrepArgs a) {
+__device__ __forceinline__ void prep_pope_norm_body(const PrepArgs& a, int blk, float* tab_out) {
   const int lane = threadIdx.x & 63;
-  const int tok = blockIdx.x * WPB + (threadIdx.x >> 6);
+  const int tok = blk * WPB + (threadIdx.x >> 6);
   if (tok >= a.B * a.S) return;  // whole waves: the kernel has no barrier
   const int tpr = a.Dr >> 3;
   const int nch = a.H * tpr;
@@ -100,40 +104,42 @@ __global__ __launch_bounds__(WPB * 64) void prep_pope_norm_kernel(PrepArgs a) {
   }
   const float r = rsqrtf(wave_sum(ss) * (1.0f / (float)(a.H * a.Dr)) + a.norm_eps);
   const bool add = a.is_key && a.delta;
+  float cs8[8], sn8[8];
+  auto phases = [&](int h, int t) {  // of the 8 dims of chunk t of head h
+    const f32x4 f0 = *(const f32x4*)(a.freqs + t * 8), f1 = *(const f32x4*)(a.freqs + t * 8 + 4);
+    f32x4 d0 = {0.f, 0.f, 0.f, 0.f}, d1 = d0;
+    if (add) {
+      d0 = *(const f32x4*)(a.delta + h * a.delta_hs + t * 8);
+      d1 = *(const f32x4*)(a.delta + h * a.delta_hs + t * 8 + 4);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float ph = mul_nc(pos, e < 4 ? f0[e] : f1[e - 4]);
+      if (add) ph = add_nc(ph, e < 4 ? d0[e] : d1[e - 4]);
+      pe_sincos(ph, sn8[e], cs8[e]);
+    }
+  };
+  // Dr / 8 divides 64: a lane's chunks all sit at the same place of their heads, and without a phase bias per
+  // head they share their phases
+  const bool once = 64 % tpr == 0 && (!add || a.delta_hs == 0);
+  if (once) phases(0, lane % tpr);
 #pragma unroll
   for (int k = 0; k < CPL; ++k) {
     const int c = lane + k * 64;
     if (c < nch) {
       const int h = c / tpr, t = c - h * tpr;
       norm_chunk(x[k], r, a.xr_dtype, a.norm_w, a.norm_w_dtype, c * 8);
-      const f32x4 f0 = *(const f32x4*)(a.freqs + t * 8), f1 = *(const f32x4*)(a.freqs + t * 8 + 4);
-      f32x4 d0 = {0.f, 0.f, 0.f, 0.f}, d1 = d0;
-      if (add) {
-        d0 = *(const f32x4*)(a.delta + h * a.delta_hs + t * 8);
-        d1 = *(const f32x4*)(a.delta + h * a.delta_hs + t * 8 + 4);
-      }
+      if (!once) phases(h, t);
       float cv[8], sv[8];
-      if (a.tab && !a.is_key) {  // query phases from the table (the same values pe_sincos gives)
-        const float* tr = a.tab + (int64_t)s * 2 * a.Dr + t * 8;
-        const f32x4 c0 = *(const f32x4*)tr, c1 = *(const f32x4*)(tr + 4);
-        const f32x4 s0 = *(const f32x4*)(tr + a.Dr), s1 = *(const f32x4*)(tr + a.Dr + 4);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float mu = softplus_f(x[k][e]);
-          cv[e] = mul_nc(mu, e < 4 ? c0[e] : c1[e - 4]);
-          sv[e] = mul_nc(mu, e < 4 ? s0[e] : s1[e - 4]);
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float mu = softplus_f(x[k][e]);
-          float ph = mul_nc(pos, e < 4 ? f0[e] : f1[e - 4]);
-          if (add) ph = add_nc(ph, e < 4 ? d0[e] : d1[e - 4]);
-          float sn, cs;
-          pe_sincos(ph, sn, cs);
-          cv[e] = mul_nc(mu, cs);
-          sv[e] = mul_nc(mu, sn);
-        }
+      for (int e = 0; e < 8; ++e) {
+        const float mu = softplus_f(x[k][e]);
+        cv[e] = mul_nc(mu, cs8[e]);
+        sv[e] = mul_nc(mu, sn8[e]);
+      }
+      if (tab_out && b == 0 && h == 0) {
+        store8(tab_out, (int64_t)s * 2 * a.Dr + t * 8, 1, cs8);
+        store8(tab_out, (int64_t)s * 2 * a.Dr + a.Dr + t * 8, 1, sn8);
       }
       const int64_t drow = (int64_t)(b * a.H + h) * a.S + s;
       row_store8(a.dst, drow, a.width, a.Dc + t * 8, DDT, cv);
@@ -156,6 +162,15 @@ __global__ __launch_bounds__(WPB * 64) void prep_pope_norm_kernel(PrepArgs a) {
     const float z[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     row_store8(a.dst, (int64_t)(b * a.H + h) * a.S + s, a.width, used + j * 8, DDT, z);
   }
+}
+
+// Both sides in one launch: blocks below nqblk take query tokens and write the phase table (tab, may be
+// null), the rest key tokens.  One launch instead of the table's and one a side: at the trainer's size (8 x
+// 512 tokens, 8 -> 4 heads of 32) each is a few microseconds, about what a launch costs.
+template <int DDT, int CPL>
+__global__ __launch_bounds__(WPB * 64) void prep_pope_norm_kernel(PrepArgs aq, PrepArgs ak, unsigned nqblk, float* tab) {
+  if (blockIdx.x < nqblk) prep_pope_norm_body<DDT, CPL>(aq, (int)blockIdx.x, tab);
+  else prep_pope_norm_body<DDT, CPL>(ak, (int)(blockIdx.x - nqblk), nullptr);
 }
 
 // chunks per lane for a row of nch 8-element chunks: the smallest instantiated count that covers it
@@ -415,7 +430,7 @@ int launch_swiglu_bwd(const void* x, const void* gate, const void* dy, void* dx,
   return hipGetLastError() == hipSuccess ? 0 : -7;
 }
 
-int launch_prep_norm(const PrepArgs& a, hipStream_t s) {
+static int prep_norm_check(const PrepArgs& a) {
   if (a.mode != 0 || !a.norm_w || a.norm_w_dtype < 0 || a.norm_w_dtype > 2 || a.xr_dtype < 0 || a.xr_dtype > 2 ||
       a.dst_dtype < 0 || a.dst_dtype > DT_SPLIT)
     return -4;
@@ -426,14 +441,23 @@ int launch_prep_norm(const PrepArgs& a, hipStream_t s) {
                   ((uintptr_t)a.dst % 16) == 0 && ((uintptr_t)a.freqs % 16) == 0 && ((uintptr_t)a.norm_w % 16) == 0 &&
                   (!a.is_key || !a.delta || (((uintptr_t)a.delta % 16) == 0 && a.delta_hs % 4 == 0)) &&
                   (a.Dc == 0 || (a.xc_s[3] == 1 && rows_aligned(a.xc, a.xc_dtype, a.xc_s[0], a.xc_s[1], a.xc_s[2])));
-  if (!ok) return -5;
-  const dim3 grid((unsigned)(((int64_t)a.B * a.S + WPB - 1) / WPB));
-  with_cpl(chunks_per_lane(a.H * (a.Dr / 8)), [&](auto c) {
+  return ok ? 0 : -5;
+}
+
+int launch_prep_norm(const PrepArgs& aq, const PrepArgs& ak, float* tab, hipStream_t s) {
+  int rc = prep_norm_check(aq);
+  if (rc || (rc = prep_norm_check(ak))) return rc;
+  if (aq.dst_dtype != ak.dst_dtype || aq.Dr != ak.Dr) return -4;
+  const int64_t nq = ((int64_t)aq.B * aq.S + WPB - 1) / WPB, nk = ((int64_t)ak.B * ak.S + WPB - 1) / WPB;
+  if (nq + nk > 0x7fffffff) return -2;
+  const dim3 grid((unsigned)(nq + nk));
+  with_cpl(chunks_per_lane(std::max(aq.H, ak.H) * (aq.Dr / 8)), [&](auto c) {
     constexpr int C = decltype(c)::value;
-    if (a.dst_dtype == 0) hipLaunchKernelGGL((prep_pope_norm_kernel<0, C>), grid, dim3(WPB * 64), 0, s, a);
-    else if (a.dst_dtype == 2) hipLaunchKernelGGL((prep_pope_norm_kernel<2, C>), grid, dim3(WPB * 64), 0, s, a);
-    else if (a.dst_dtype == 1) hipLaunchKernelGGL((prep_pope_norm_kernel<1, C>), grid, dim3(WPB * 64), 0, s, a);
-    else hipLaunchKernelGGL((prep_pope_norm_kernel<DT_SPLIT, C>), grid, dim3(WPB * 64), 0, s, a);
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(WPB * 64), 0, s, aq, ak, (unsigned)nq, tab); };
+    if (aq.dst_dtype == 0) go(prep_pope_norm_kernel<0, C>);
+    else if (aq.dst_dtype == 2) go(prep_pope_norm_kernel<2, C>);
+    else if (aq.dst_dtype == 1) go(prep_pope_norm_kernel<1, C>);
+    else go(prep_pope_norm_kernel<DT_SPLIT, C>);
   });
   return hipGetLastError() == hipSuccess ? 0 : -7;
 }

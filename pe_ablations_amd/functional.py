@@ -532,21 +532,22 @@ def _launch_normed(qr, kr, v, qc, kc, freqs, delta, cfg, wq, wk, eps):
     L = _lib.lib()
     dev = qr.device
     wq, wk = wq.contiguous(), wk.contiguous()
-    p = _params(cfg, qr, kr, v, qc, delta)
-    _lib.check(L.pe_attn_check(ctypes_ref(p)))
+    key = ("normed", cfg["key"], _sig(qr), _sig(kr), _sig(v), _sig(qc), _sig(kc), None if delta is None else delta.dim())
+    plans = _plans()
+    fp = plans.get(key)
+    if fp is None:
+        fp = plans[key] = _FwdPlan(cfg, qr, kr, v, qc, kc, delta)
     n = _lib.PeNormParams()
     n.q_weight, n.k_weight = wq.data_ptr(), wk.data_ptr()
     n.weight_dtype, n.eps = _dtype_code(wq.dtype), float(eps)
-    cdt = _TORCH_DTYPE[cfg["dtype"]]
-    B, Hq, Sq, Dv = qr.shape[0], qr.shape[1], qr.shape[2], v.shape[3]
-    ws_bytes = L.pe_attn_fwd_workspace_bytes(ctypes_ref(p))
-    fws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    out = torch.empty((B, Sq, Hq, Dv), dtype=cdt, device=dev).transpose(1, 2)
-    lse = torch.empty((B, Hq, Sq), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        rc = L.pe_attn_fwd_normed(ctypes_ref(p), ctypes_ref(n), ref(_tensor(qc)), ref(_tensor(qr)),
-                                  ref(_tensor(kc)), ref(_tensor(kr)), ref(_tensor(v)), _ptr(freqs), _ptr(delta),
-                                  ref(_tensor(out)), lse.data_ptr(), fws.data_ptr(), ws_bytes, _stream(dev))
+    fws = torch.empty(fp.ws, dtype=torch.uint8, device=dev)
+    out = torch.empty(fp.out_shape, dtype=fp.cdt, device=dev).transpose(1, 2)
+    lse = torch.empty((fp.out_shape[0], fp.out_shape[2], fp.out_shape[1]), dtype=torch.float32, device=dev)
+    d = fp.d
+    with _on(dev):
+        rc = L.pe_attn_fwd_normed(fp.pref, ctypes.byref(n), d[0].bind(qc), d[1].bind(qr), d[2].bind(kc), d[3].bind(kr),
+                                  d[4].bind(v), _ptr(freqs), _ptr(delta), d[5].bind(out), lse.data_ptr(),
+                                  fws.data_ptr(), fp.ws, _stream(dev))
     _lib.check(rc)
     return out, lse, fws
 
