@@ -635,6 +635,10 @@ DecodePlan decode_plan(const pe_attn_params* p) {
   // count, not the device's: the workspace query and the call must size the partials alike.
   int64_t nu = (1024 + tiles - 1) / tiles;
   nu = std::min<int64_t>(nu, (nkb + 1) / 2);
+  // up to 512 rows one workgroup takes the whole cache, four blocks a wave, and needs no merge launch (one token,
+  // 8 -> 4 heads of the split form, 500 rows: 17.8 us of GPU time in four launches, 12.9 in two
+  // with the query transform in the split kernel too; 33.4 -> 27.6 us a step with the host's share)
+  if (nkb <= 16) nu = 4;
   nu = std::max<int64_t>(4, std::min<int64_t>(512, (nu + 3) / 4 * 4));
   d.nunit = (int)nu;
   size_t rows = (size_t)tiles * d.nunit * 32;
@@ -724,7 +728,7 @@ int pe_attn_decode(const pe_attn_params* p, const pe_tensor_t* qc, const pe_tens
   fill_prep(a, p, 0, qc, qr, freqs, nullptr, ws, dqk);
   // a tile of few query rows (one decoded token of a small GQA group) is transformed inside the
   // split kernel, with the prologue's arithmetic, instead of in a launch of its own
-  const bool fuse_q = p->dtype == PE_DTYPE_BF16 && (int64_t)(p->Hq / p->Hkv) * p->Sq <= pe::DECODE_FUSED_ROWS &&
+  const bool fuse_q = half_dt(p->dtype) && (int64_t)(p->Hq / p->Hkv) * p->Sq <= pe::DECODE_FUSED_ROWS &&
                       pe::prep_vec_query_ok(a);
   if (!fuse_q && (rc = pe::launch_prep(a, s))) return rc;
   pe::DecodeArgs da;
@@ -733,6 +737,11 @@ int pe_attn_decode(const pe_attn_params* p, const pe_tensor_t* qc, const pe_tens
     da.qraw = qr->data;
     for (int i = 0; i < 4; ++i) da.qr_s[i] = qr->stride[i];
     da.freqs = freqs; da.Dr = p->Dr; da.start_pos = p->start_pos_q; da.pos_round = p->position_rounding;
+    da.Dc = p->Dc;
+    if (p->Dc > 0) {
+      da.qcraw = qc->data;
+      for (int i = 0; i < 4; ++i) da.qc_s[i] = qc->stride[i];
+    }
   }
   da.q = ws; da.k = k_cache; da.v = v_cache;
   da.B = p->B; da.Hq = p->Hq; da.Hkv = p->Hkv; da.Sq = p->Sq; da.L = p->Sk; da.cap = capacity;

@@ -104,31 +104,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const uint32_t qrd = (uint32_t)l32 * QROW;
   const uint32_t qsw = (uint32_t)(l32 & (NCQ - 1));
   bool staged = false;
-  if constexpr (DT == 0) {
+  if constexpr (DT != 1) {
     if (a.qraw) {
       // the raw rows transformed here, element by element with the vectorised prologue's arithmetic
-      // (softplus magnitude times cos / sin of fl(pos * freq), rounded to bf16), so the operand
+      // (softplus magnitude times cos / sin of fl(pos * freq), rounded to the 16-bit type), so the operand
       // rows are bitwise those the prologue would write; tile rows past the query rows are zero
-      // (their columns are never stored).  Element (x, d) of the tile goes to column d (cos) and
-      // Dr + d (sin) of row x, chunk-swizzled as above.
-      const int tid = threadIdx.x, Dr = a.Dr;
+      // (their columns are never stored).  Element (x, d) of the tile goes to column Dc + d (cos) and
+      // Dc + Dr + d (sin) of row x, chunk-swizzled as above, after the Dc content columns and before the
+      // padding's zeros.
+      const int tid = threadIdx.x, Dr = a.Dr, Dc = a.Dc;
       const int nreal = min(32, nrows - qt * 32);
-      for (int i = tid; i < (32 - nreal) * NCQ; i += 256) {
-        const int x = nreal + i / NCQ, c = i % NCQ;
-        *(u32x4*)(qlds + x * QROW + ((c ^ (x & (NCQ - 1))) << 4)) = u32x4{0u, 0u, 0u, 0u};
+      auto chunk = [&](int x, int c) { return (u32x4*)(qlds + x * QROW + (((uint32_t)c ^ (uint32_t)(x & (NCQ - 1))) << 4)); };
+      for (int i = tid; i < (32 - nreal) * NCQ; i += 256) *chunk(nreal + i / NCQ, i % NCQ) = u32x4{0u, 0u, 0u, 0u};
+      const int npad = NCQ - (Dc + 2 * Dr) / 8;
+      for (int i = tid; i < nreal * npad; i += 256) *chunk(i / npad, NCQ - 1 - i % npad) = u32x4{0u, 0u, 0u, 0u};
+      const int ncc = Dc / 8;
+      for (int i = tid; i < nreal * ncc; i += 256) {
+        const int x = i / ncc, rq = qt * 32 + x, hq = hk * grp + rq / a.Sq, iq = rq % a.Sq;
+        *chunk(x, i % ncc) = *(const u32x4*)((const uint16_t*)a.qcraw + b * a.qc_s[0] + hq * a.qc_s[1] +
+                                             (int64_t)iq * a.qc_s[2] + (i % ncc) * 8);
       }
       for (int i = tid; i < nreal * Dr; i += 256) {
         const int x = i / Dr, d = i % Dr;
         const int rq = qt * 32 + x, hq = hk * grp + rq / a.Sq, iq = rq % a.Sq;
-        const uint16_t raw = ((const uint16_t*)a.qraw)[b * a.qr_s[0] + hq * a.qr_s[1] + (int64_t)iq * a.qr_s[2] + d];
-        const float mu = softplus_f(__builtin_bit_cast(float, (uint32_t)raw << 16));
+        const float mu = softplus_f(load_as_float_t<DT>(a.qraw, b * a.qr_s[0] + hq * a.qr_s[1] + (int64_t)iq * a.qr_s[2] + d, DT));
         float sn, cs;
         pe_sincos(mul_nc(pe_pos(a.start_pos + iq, a.pos_round), a.freqs[d]), sn, cs);
-        const uint32_t pr = pack_bf2(mul_nc(mu, cs), mul_nc(mu, sn));
-        const int cc = d, cs_ = Dr + d;
-        *(uint16_t*)(qlds + x * QROW + ((((uint32_t)cc >> 3) ^ (uint32_t)(x & (NCQ - 1))) << 4) + (cc & 7) * 2) = (uint16_t)pr;
-        *(uint16_t*)(qlds + x * QROW + ((((uint32_t)cs_ >> 3) ^ (uint32_t)(x & (NCQ - 1))) << 4) + (cs_ & 7) * 2) =
-            (uint16_t)(pr >> 16);
+        const uint32_t pr = pack2<DT>(mul_nc(mu, cs), mul_nc(mu, sn));
+        const int cc = Dc + d, cs_ = Dc + Dr + d;
+        *((uint16_t*)chunk(x, cc >> 3) + (cc & 7)) = (uint16_t)pr;
+        *((uint16_t*)chunk(x, cs_ >> 3) + (cs_ & 7)) = (uint16_t)(pr >> 16);
       }
       staged = true;
     }
@@ -215,6 +220,44 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   // are neither written nor read)
   const int64_t pb = ((int64_t)bh * a.nqt + qt) * a.nunit + u;
   const float lt = l + xor32(l);
+  if (a.nunit == 4) {
+    // the whole cache in one workgroup (short caches, or many tiles): its four ranges merged here in LDS, in
+    // range order, with the merge kernel's formula, in place of that kernel's launch
+    constexpr int RS = DV + 4;
+    static_assert((4 * 32 * RS + 2 * 4 * 32) * 4 <= 8 * SV + 32 * QROW, "the ranges fit the tile's LDS");
+    float* const ro = (float*)smem;        // [4][32][RS]
+    float* const rm = ro + 4 * 32 * RS;    // [4][32] running max
+    float* const rl = rm + 4 * 32;         // [4][32] row sum
+    const int nreal = min(32, nrows - qt * 32);
+    __syncthreads();  // every wave has read its last v block
+    if (l32 < nreal) {
+#pragma unroll
+      for (int t = 0; t < NOT; ++t)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) ro[(w * 32 + l32) * RS + t * 32 + c_row(j, g)] = o[t][j];
+      if (g == 0) {
+        rm[w * 32 + l32] = m;
+        rl[w * 32 + l32] = lt;
+      }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < nreal * DV; i += 256) {
+      const int x = i / DV, c = i % DV, rq = qt * 32 + x;
+      const float M = fmaxf(fmaxf(rm[x], rm[32 + x]), fmaxf(rm[64 + x], rm[96 + x]));
+      float acc = 0.f, lsum = 0.f;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float wt = exp2f(rm[u * 32 + x] - M);
+        lsum += rl[u * 32 + x] * wt;
+        acc += ro[(u * 32 + x) * RS + c] * wt;
+      }
+      const int ho = hk * grp + rq / a.Sq, iq = rq % a.Sq;
+      if (c < a.dv_real)
+        store_from_float(a.o, b * a.o_sb + ho * a.o_sh + (int64_t)iq * a.o_ss + c, a.o_dtype, lsum > 0.f ? acc * (1.f / lsum) : 0.f);
+      if (c == 0) a.lse[(int64_t)(b * a.Hq + ho) * a.Sq + iq] = lsum > 0.f ? (M + log2f(lsum)) * LN2 : -INFINITY;
+    }
+    return;
+  }
   if (r >= nrows) return;
   float* po = a.part_o + pb * 32 * DV;
 #pragma unroll
@@ -305,8 +348,10 @@ template <int DT, int DQK, int DV>
 static int run_decode(const DecodeArgs& a, hipStream_t s) {
   const int64_t blocks = (int64_t)a.B * a.Hkv * a.nqt * (a.nunit / 4);
   hipLaunchKernelGGL((decode_split_kernel<DT, DQK, DV>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-  const int64_t rows = (int64_t)a.B * a.Hkv * a.nqt * std::min(32, (a.Hq / a.Hkv) * a.Sq);
-  hipLaunchKernelGGL((decode_merge_kernel<DV>), dim3((unsigned)rows), dim3(1024), 0, s, a);
+  if (a.nunit > 4) {  // four ranges are one workgroup, which merges them itself
+    const int64_t rows = (int64_t)a.B * a.Hkv * a.nqt * std::min(32, (a.Hq / a.Hkv) * a.Sq);
+    hipLaunchKernelGGL((decode_merge_kernel<DV>), dim3((unsigned)rows), dim3(1024), 0, s, a);
+  }
   return hipGetLastError() == hipSuccess ? 0 : -7;
 }
 

@@ -653,8 +653,7 @@ bool prep_vec_copy_ok(const PrepArgs& a) {
 }
 
 bool prep_vec_query_ok(const PrepArgs& a) {
-  return prep_vec_ok(a) && a.xr_dtype == a.dst_dtype && a.dst_dtype != 1 && !a.is_key && a.Dc == 0 &&
-         a.width == 2 * a.Dr;
+  return prep_vec_ok(a) && a.xr_dtype == a.dst_dtype && (a.dst_dtype == 0 || a.dst_dtype == 2) && !a.is_key;
 }
 
 int launch_prep(const PrepArgs& a, hipStream_t s) {

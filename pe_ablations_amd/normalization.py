@@ -34,7 +34,8 @@ class RMSNorm(nn.Module):
                 and self.weight.dtype in (torch.bfloat16, torch.float32)):
             if not torch.is_grad_enabled():
                 return _hip_rms_norm(x, self.weight, self.eps)
-            if self.weight.shape == (n,) and self.weight.device == x.device and plain_autograd(x, self.weight):
+            if (x.numel() > 0 and self.weight.shape == (n,) and self.weight.device == x.device
+                    and plain_autograd(x, self.weight)):
                 return RMSNormFn.apply(x, self.weight, self.eps)
         return self._norm(x.float()).type_as(x) * self.weight
 

@@ -1,0 +1,50 @@
+"""Decode with the query transform inside the split kernel (content part, fp16, padded widths) and with the
+ranges merged in the workgroup, against the paths they replace.
+
+A query view whose rows start at an odd element is transformed by the prologue launch, an aligned one in the
+kernel, with the same arithmetic: bitwise equal results.  Caches of up to 512 rows are merged in the
+workgroup, longer ones by the merge kernel; both are held to the oracle at the decode bars.
+"""
+
+import math
+
+import pytest
+import torch
+
+from oracle import pe_oracle as O
+from pe_ablations_amd.functional import cache_widths, pe_attention_decode, pe_cache_append
+from tests._cmp import err
+from tests.test_gpu_prep_types import off_by_one
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dt,B,Hq,Hkv,L,Sq,Dc,Dr,Dv", [
+    (torch.bfloat16, 1, 8, 4, 500, 1, 64, 32, 64),     # the reference's shape
+    (torch.float16, 3, 8, 1, 512, 1, 0, 64, 64),
+    (torch.bfloat16, 2, 4, 4, 33, 2, 32, 16, 128),     # padded width, a block and a row
+    (torch.float16, 1, 6, 2, 1, 1, 64, 32, 48),        # one row, padded values
+    (torch.bfloat16, 1, 2, 1, 513, 4, 0, 128, 128),    # the merge kernel
+    (torch.bfloat16, 1, 16, 2, 300, 1, 128, 64, 128),  # QK width 256, eight rows a tile
+    (torch.bfloat16, 2, 12, 2, 200, 9, 0, 64, 64),     # 54 rows, two tiles, prologue launch
+])
+def test_decode_matches_oracle_and_the_prologue_launch(cuda, dt, B, Hq, Hkv, L, Sq, Dc, Dr, Dv):
+    g = torch.Generator().manual_seed(L)
+    x = {n: torch.randn(B, S, H, D, generator=g).to(dt).transpose(1, 2) for n, H, S, D in
+         (("q", Hq, Sq, Dr), ("k", Hkv, L, Dr), ("v", Hkv, L, Dv), ("qc", Hq, Sq, Dc), ("kc", Hkv, L, Dc)) if D}
+    on = (lambda n: x[n].cuda() if n in x else None)
+    Sq = min(Sq, L)
+    freqs, delta = O.pope_freqs(Dr), torch.rand(Dr, generator=g) * (-2 * math.pi)
+    wk, wv = cache_widths(d_content=Dc, d_pe=Dr, d_v=Dv)
+    kc, vc = (torch.full((B, Hkv, L + 5, w), float("nan"), dtype=dt, device=cuda) for w in (wk, wv))
+    pe_cache_append(on("k"), on("v"), kc, vc, start_pos=0, k_c=on("kc"), freqs=freqs.cuda(), delta=delta.cuda())
+    kw = dict(d_v=Dv, freqs=freqs.cuda(), scale=0.1, return_lse=True)
+    with torch.no_grad():
+        out, lse = pe_attention_decode(on("q"), kc, vc, L, q_c=on("qc"), **kw)
+        out2, lse2 = pe_attention_decode(off_by_one(on("q")), kc, vc, L, q_c=on("qc"), **kw)
+    assert torch.equal(out, out2) and torch.equal(lse, lse2)
+    tq, tk = O.pope_transform(x["q"], freqs, L - Sq), O.pope_transform(x["k"], freqs, 0, delta)
+    if Dc:
+        tq, tk = torch.cat([x["qc"].float(), tq], -1), torch.cat([x["kc"].float(), tk], -1)
+    ref, rlse = O.attention(tq.to(dt).float(), tk.to(dt).float(), x["v"].float(), 0.1, causal=True)
+    assert err(out, ref) < (2e-2 if dt == torch.bfloat16 else 2.5e-3) and err(lse, rlse) < 2e-3
