@@ -691,6 +691,8 @@ class RMSNormFn(torch.autograd.Function):
             need = [t for t, n in zip((x, weight), ctx.needs_input_grad) if n]
             grads = iter(torch.autograd.grad(y, need, dy, create_graph=True))
             return tuple(next(grads) if n else None for n in ctx.needs_input_grad[:2]) + (None,)
+        if dy.data_ptr() % 16:  # contiguous() would return such a view as it is
+            dy = dy.clone(memory_format=torch.contiguous_format)
         return rms_norm_backward(x, weight, dy, ctx.eps) + (None,)
 
 

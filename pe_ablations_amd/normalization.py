@@ -35,8 +35,10 @@ class RMSNorm(nn.Module):
             if not torch.is_grad_enabled():
                 return _hip_rms_norm(x, self.weight, self.eps)
             if (x.numel() > 0 and self.weight.shape == (n,) and self.weight.device == x.device
-                    and plain_autograd(x, self.weight)):
-                return RMSNormFn.apply(x, self.weight, self.eps)
+                    and plain_autograd(x, self.weight) and (x.data_ptr() | self.weight.data_ptr()) % 16 == 0):
+                # the expression's fp32 cast leaves a 16-bit x free to be changed in place afterwards; the
+                # Function keeps x itself, so it is given a copy (an fp32 x the expression keeps as well)
+                return RMSNormFn.apply(x if x.dtype == torch.float32 else x.clone(), self.weight, self.eps)
         return self._norm(x.float()).type_as(x) * self.weight
 
 

@@ -109,3 +109,34 @@ def test_swiglu_gradients(cuda, shape):
     assert (got[1].float() - want[1].float()).abs().max() <= 2 ** -7 * want[1].float().abs().max()
     t = gate.detach().t().contiguous().t().requires_grad_() if gate.dim() == 2 else gate.detach().requires_grad_()
     assert torch.equal(torch.autograd.grad(SwiGLU()(x, t), t, dy)[0], got[1])  # a transposed gate
+
+
+@pytest.mark.parametrize("xt", [F32, B16])
+@pytest.mark.parametrize("what", ["x", "weight", "dy"])
+def test_rmsnorm_unaligned_operands(cuda, xt, what):
+    """Views two or four bytes past a 16-byte boundary: x and the weight take the expression, dy a copy."""
+    def off(t, shift):
+        flat = torch.empty(t.numel() + 8, dtype=t.dtype, device="cuda")
+        v = flat[shift:shift + t.numel()].view(t.shape)
+        v.copy_(t)
+        return v.detach()
+    g = torch.Generator(device="cuda").manual_seed(3)
+    m = RMSNorm(64).cuda()
+    m.weight.data = off(1 + 0.1 * torch.randn(64, generator=g, device="cuda"), int(what == "weight"))
+    x = off(torch.randn(9, 64, generator=g, device="cuda").to(xt), int(what == "x")).requires_grad_()
+    y, ref = m(x), rms_norm_expression(x, m.weight, m.eps)
+    dy = off(torch.randn(9, 64, generator=g, device="cuda").to(y.dtype), int(what == "dy"))
+    for a, b in zip(torch.autograd.grad(y, (x, m.weight), dy), torch.autograd.grad(ref, (x, m.weight), dy)):
+        assert near(a, b, 2 ** -7 if xt == B16 else 2e-6)
+
+
+def test_rmsnorm_half_input_changed_in_place_afterwards(cuda):
+    m = RMSNorm(64).cuda()
+    grads = []
+    for norm in (m, lambda t: rms_norm_expression(t, m.weight, m.eps)):
+        leaf = torch.linspace(-2, 3, 9 * 64, device="cuda").view(9, 64).to(B16).requires_grad_()
+        x = leaf * 1.0
+        y = norm(x)
+        x += 1.0
+        grads.append(torch.autograd.grad((y * y * y).sum() + x.sum(), leaf)[0])
+    assert near(grads[0], grads[1], 2 ** -7)
