@@ -48,3 +48,28 @@ def test_decode_matches_oracle_and_the_prologue_launch(cuda, dt, B, Hq, Hkv, L, 
         tq, tk = torch.cat([x["qc"].float(), tq], -1), torch.cat([x["kc"].float(), tk], -1)
     ref, rlse = O.attention(tq.to(dt).float(), tk.to(dt).float(), x["v"].float(), 0.1, causal=True)
     assert err(out, ref) < (2e-2 if dt == torch.bfloat16 else 2.5e-3) and err(lse, rlse) < 2e-3
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("step", [0.0, 3.0, 5.9, 6.1, 80.0, -5.0, -80.0])
+def test_reference_follows_falling_and_rising_blocks(cuda, dt, step):
+    """Short caches whose 32-key blocks' largest scores fall (or rise) by ``step`` powers of two a block.
+    Bar: half an ulp for each probability and for the result, so 2^-8 (fp16: 2^-11) of the largest value; lse
+    from fp32 sums of magnitudes up to 80 * 16 * ln 2: 2^-21 of that."""
+    g = torch.Generator().manual_seed(5)
+    L, Hq, Hkv, Dc, Dr, Dv = 512, 4, 2, 64, 32, 64
+    qc, kc = torch.zeros(1, Hq, 1, Dc, dtype=dt), torch.zeros(1, Hkv, L, Dc, dtype=dt)
+    qc[..., 0] = 8.0
+    kc[..., 0] = (-step * math.log(2.0) * (torch.arange(L) // 32) + torch.randn(Hkv, L, generator=g)).to(dt)
+    qr = torch.full((1, Hq, 1, Dr), -30.0, dtype=dt)  # softplus 1e-13: the position part adds nothing
+    kr, v = torch.randn(1, Hkv, L, Dr, generator=g).to(dt), torch.randn(1, Hkv, L, Dv, generator=g).to(dt)
+    freqs, delta = O.pope_freqs(Dr).cuda(), torch.zeros(Dr, device=cuda)
+    wk, wv = cache_widths(d_content=Dc, d_pe=Dr, d_v=Dv)
+    ck, cv = (torch.zeros(1, Hkv, L, w, dtype=dt, device=cuda) for w in (wk, wv))
+    pe_cache_append(kr.cuda(), v.cuda(), ck, cv, start_pos=0, k_c=kc.cuda(), freqs=freqs, delta=delta)
+    with torch.no_grad():
+        out, lse = pe_attention_decode(qr.cuda(), ck, cv, L, q_c=qc.cuda(), d_v=Dv, freqs=freqs, scale=0.125, return_lse=True)
+    s = kc[..., 0].double().repeat_interleave(Hq // Hkv, 1)
+    ref = s.softmax(-1).unsqueeze(-2) @ v.double().repeat_interleave(Hq // Hkv, 1)
+    assert err(out, ref) < (2 ** -8 if dt == torch.bfloat16 else 2 ** -11) * float(v.abs().max())
+    assert err(lse[..., 0], s.logsumexp(-1)) < 2 ** -21 * max(16.0, abs(step) * 16)
