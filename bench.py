@@ -22,7 +22,8 @@ More workloads, selected with ``--workload`` (the default is the headline above)
 
 * ``fwd``: the long-context evaluation forward (the same shape, forward only, under
   ``torch.inference_mode``; 3*B*H*S^2*D FLOPs per step); ``fwd32`` the same in fp32, the
-  precision of the reference's 16k evaluation, against the fp32 MFMA peak.
+  precision of the reference's 16k evaluation, against a sixth of the bf16 MFMA peak (an fp32
+  product is six bf16 plane products).
 * ``c2``: PoPE fwd+bwd at B=8, H=12, S=2048, D=64 (~125M GPT shape).
 * ``c3``: FoPE fwd+bwd at B=4, H=16, S=4096, D=128, M=4 frequencies per dim; the FoPE collapse
   (FoPEPoPEEmbedding) runs in each step and the Fourier coefficients get gradients.
@@ -65,7 +66,7 @@ import sys
 import time
 
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA (published)
-PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA (published)
+PEAK_FP32_TFLOPS = PEAK_BF16_TFLOPS / 6   # six bf16 plane products each; the fp32 matrix unit's own peak is 157.3
 HBM_PEAK_GBS = 8000.0
 
 WORKLOAD = dict(B=1, H=16, S=16384, D=128)
@@ -84,7 +85,7 @@ ATTN_WORKLOADS = {
                 metric="fused PoPE attn fwd TFLOP/s @S=16k,D=128 (long-context eval forward); % of bf16 MFMA peak"),
     "fwd32": dict(B=1, Hq=16, Hkv=16, S=16384, Dc=0, Dr=128, Dv=128, dtype="fp32", backward=False, delta="head",
                   name="PoPE causal attention forward in fp32 (the reference's 16k evaluation precision)",
-                  metric="fused PoPE attn fwd TFLOP/s @S=16k,D=128, fp32; % of fp32 MFMA peak"),
+                  metric="fused PoPE attn fwd TFLOP/s @S=16k,D=128, fp32; % of a sixth of the bf16 MFMA peak"),
     "c2": dict(B=8, Hq=12, Hkv=12, S=2048, Dc=0, Dr=64, Dv=64, dtype="bf16", backward=True, delta="head",
                name="PoPE causal attention fwd+bwd, ~125M GPT shape",
                metric="fused PoPE attn fwd+bwd TFLOP/s @B=8,H=12,S=2048,D=64; % of bf16 MFMA peak"),
