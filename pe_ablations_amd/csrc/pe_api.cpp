@@ -41,7 +41,7 @@ struct Layout {
   bool split;  // fp32 compute with its operands as three bf16 planes (pe_split.hip)
   size_t q_off, k_off, v_off, tab_off, fwd_total;
   size_t do_off, di_off, l2_off, dq_off, dk_off, pq_off, pk_off, pkd_off, dvp_off, rtab_off, ds_off, bwd_total;
-  int ksplit;    // query-head split of the dK/dV pair kernel (pe::CoreArgs::qsplit)
+  int ksplit;    // query split of the dK/dV pair kernel (pe::CoreArgs::qsplit)
   int sq_pad;
   int ds_nqt, ds_rows, ds_e;
   int64_t ds_head;
@@ -60,7 +60,7 @@ bool fused_bwd(const pe_attn_params* p) {
          pad_qk(qk_width(p)) == 2 * p->Dr;
 }
 
-// Compute units of an MI355X.  The query-head split of dK/dV below depends on the shape only (not
+// Compute units of an MI355X.  The query split of dK/dV below depends on the shape only (not
 // on the device queried), so a workspace size taken before any device call stays valid.
 constexpr int kSplitCus = 256;
 
@@ -116,7 +116,7 @@ bool fused_split_bwd(const pe_attn_params* p, const pe_tensor_t* qr, const pe_te
 }
 
 // The explicit-mask backward (pe_attn_bwd_masked) at the pair kernel's 16-bit widths runs the same
-// kernels as the unmasked one, without the query-head split; elsewhere it runs the generic kernels,
+// kernels as the unmasked one, without the query split; elsewhere it runs the generic kernels,
 // which write fp32 dq~ / dk~ for the stand-alone inverse transform and store no dS.
 bool generic_masked(const pe_attn_params* p, bool masked) {
   return masked && !(half_dt(p->dtype) && pe::pair_shape(pad_qk(qk_width(p)), pad_v(p->Dv)));

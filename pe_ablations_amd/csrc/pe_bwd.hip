@@ -1830,7 +1830,7 @@ static int run_bwd(int which, const CoreArgs& a, hipStream_t s) {
   constexpr int NW = 4;
   constexpr bool PAIR = DT != 1 && (DQK == 128 || DQK == 256) && (DV == 128 || DV == 64);
   if constexpr (PAIR) {
-    if (a.mask) {  // explicit mask: the pair kernel's mask instantiation (no query-head split), then the dQ GEMM
+    if (a.mask) {  // explicit mask: the pair kernel's mask instantiation (no query split), then the dQ GEMM
       if (which == 0) {
         constexpr int QT = DQK == 128 && DV == 64 && DT != 2 ? 2 : 1;
         const int nkb = (a.Sk + NW * 32 - 1) / (NW * 32);
