@@ -396,6 +396,7 @@ __global__ __launch_bounds__(NW * 64, 1) void dkdv_bf16_kernel(CoreArgs a) {
     for (int kk = 0; kk < NKF; ++kk) kf[kk] = *(const u32x4*)(krow + kk * 16 + g * 8);
 #pragma unroll
     for (int kk = 0; kk < NVF; ++kk) vf[kk] = *(const u32x4*)(vrow + kk * 16 + g * 8);
+    apply_scale_sign(a.scale, kf);
   }
   f32x16 dk[NDK], dv[NDV];
 #pragma unroll
@@ -413,7 +414,7 @@ __global__ __launch_bounds__(NW * 64, 1) void dkdv_bf16_kernel(CoreArgs a) {
   if (qb0 > nqb) qb0 = nqb;
   const int nper = nqb - qb0;
   const int niter = nper * grp;
-  const float sl2 = a.scale * LOG2E;
+  const float sl2 = score_factor(a.scale);
   const int64_t qrs = (int64_t)DQK * 2;
 
   auto issue = [&](int it, char* st) {
@@ -1005,7 +1006,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_pair_kernel(CoreArgs a) {
   const int niter = QS ? __builtin_amdgcn_readfirstlane((uint32_t)(ntot * (jq + 1)) / (uint32_t)a.qsplit) - it0 : ntot;
   const int h_first = hk * grp + (QS && nper > 0 ? it0 / nper : 0);
   const int qt_first = qb0 + (QS && nper > 0 ? it0 % nper : 0);
-  const float sl2 = a.scale * LOG2E;
+  const float sl2 = score_factor(a.scale);
   const int64_t qrs = (int64_t)DQK * 2;
 
   // tiles are issued in loop order: query tile qt of query head h advances qt, then h
@@ -1146,6 +1147,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_pair_kernel(CoreArgs a) {
       // into the score products of every step, which also drains the tile loads issued a step
       // earlier.  Here it costs one wait for tile 1's loads.
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0) expcnt(7) lgkmcnt(15)
+      apply_scale_sign(a.scale, kf);
     }
     f32x16 dv[NDV];
 #pragma unroll

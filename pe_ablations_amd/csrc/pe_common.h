@@ -175,6 +175,20 @@ __device__ __forceinline__ void row_store(void* dst, int64_t row, int width, int
   }
 }
 
+// Kernels that mask raw scores, take their max and form exp2(fma(s, factor, -max)) need a positive factor.
+// A negative scale goes into one operand's fragments instead, whose sign bits it flips (exact); scale 0
+// becomes 2^-126, which takes every finite score to 0 and keeps a masked one at -inf.
+__device__ __forceinline__ float score_factor(float scale) {
+  return scale == 0.f ? 0x1p-126f : __builtin_fabsf(scale) * LOG2E;
+}
+template <int N> __device__ __forceinline__ void apply_scale_sign(float scale, u32x4 (&f)[N]) {
+  const uint32_t flip = scale < 0.f ? 0x80008000u : 0u;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[i][e] ^= flip;
+}
+
 // 8 consecutive elements of type XT kept as loaded (16 or 32 bytes) until they are used
 template <int XT> struct Raw8 {
   u32x4 r[XT == 1 ? 2 : 1];

@@ -233,6 +233,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void fwd_bf16_kernel(Core
     // products of every tile, right after the DMA waves have issued the next tile.  (Removing that
     // chain measured no faster: the DMA waves are held about as long at the issue of the burst.)
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0) expcnt(7) lgkmcnt(15)
+    apply_scale_sign(a.scale, qf);
   }
 
   int kend = a.Sk;
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void fwd_bf16_kernel(Core
 #pragma unroll
     for (int j = 0; j < 16; ++j) o[t][j] = 0.f;
   float m = -1e30f, l = 0.f;
-  const float sl2 = a.scale * LOG2E;
+  const float sl2 = score_factor(a.scale);
 
   // The last NDW waves issue every tile load (per-lane offsets computed once; full tiles need no
   // vector math), NSTG - 1 tiles ahead.  Waves that issue none go straight to their products after
