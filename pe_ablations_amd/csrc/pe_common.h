@@ -189,6 +189,13 @@ template <int N> __device__ __forceinline__ void apply_scale_sign(float scale, u
     for (int e = 0; e < 4; ++e) f[i][e] ^= flip;
 }
 
+// Online softmax whose reference m may step down to a tile's own max mx, so that the tile's largest
+// probability is 1 and has no rounding: allowed as long as the sum so far, lsum, stays below 480 relative
+// to it (a tile adds at most 32 or 96), which bounds the accumulators by 576 times the largest value.
+__device__ __forceinline__ bool own_max_ok(float lsum, float m, float mx) {
+  return lsum * __builtin_amdgcn_exp2f(m - mx) < 480.f;  // false for a tile without a key: mx = -inf
+}
+
 // 8 consecutive elements of type XT kept as loaded (16 or 32 bytes) until they are used
 template <int XT> struct Raw8 {
   u32x4 r[XT == 1 ? 2 : 1];

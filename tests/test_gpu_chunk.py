@@ -16,7 +16,7 @@ import torch
 
 from oracle import pe_oracle as O
 from pe_ablations_amd.functional import cache_widths, pe_attention_decode, pe_cache_append
-from tests._cmp import err
+from tests._cmp import err, half_ulp_bf16
 
 pytestmark = pytest.mark.gpu
 
@@ -66,3 +66,26 @@ def test_chunk_matches_oracle(cuda, mode, dtype, B, Hq, Hkv, L, Sq, Dc, Dr, Dv, 
     ref, rlse = O.attention(tq.to(dt).float(), tk.to(dt).float(), v.float(), scale, causal=causal != "none")
     assert err(out, ref) < (2e-2 if dt == torch.bfloat16 else 2.5e-3), err(out, ref)
     assert err(lse, rlse) < 2e-3, err(lse, rlse)
+
+
+@pytest.mark.parametrize("dt,Hq,Sq,Dr", [(torch.bfloat16, 4, 300, 64), (torch.float16, 10, 64, 128), (torch.bfloat16, 4, 300, 256)])
+def test_the_largest_probability_of_a_tile_is_not_rounded(cuda, dt, Hq, Sq, Dr):
+    """Key 150, in a later tile of the first key range, stands x in (0, 7.5] powers of two above all others and
+    alone has a value, so out = v 2^x / (2^x + 999): as P is relative to its tile's max, its probability there
+    is 1, and all that is left is the result's own rounding, half an ulp (and 2^-18 for exp2 and the fp32 sums)."""
+    g = torch.Generator().manual_seed(Sq)
+    L, j, Dv = 1000, 150, 64
+    x = torch.rand(1, Hq, Sq, generator=g) * 7.5
+    q, k, v = torch.zeros(1, Hq, Sq, Dr), torch.zeros(1, Hq, L, Dr), torch.zeros(1, Hq, L, Dv)
+    q[..., 0], k[:, :, j, 0] = x, 1.0
+    v[:, :, j] = torch.randn(1, Hq, Dv, generator=g)
+    q, k, v = q.to(dt), k.to(dt), v.to(dt)
+    wk, wv = cache_widths(mode="none", d_pe=Dr, d_v=Dv)
+    kcache, vcache = (torch.zeros(1, Hq, L, w, dtype=dt, device=cuda) for w in (wk, wv))
+    pe_cache_append(k.to(cuda), v.to(cuda), kcache, vcache, start_pos=0, mode="none")
+    with torch.no_grad():
+        out = pe_attention_decode(q.to(cuda), kcache, vcache, L, d_v=Dv, mode="none", scale=math.log(2.0), causal=False)
+    e = torch.exp2(q[..., :1].double())
+    ref = v[:, :, j:j + 1].double() * e / (e + (L - 1))
+    half = half_ulp_bf16(ref) if dt == torch.bfloat16 else (half_ulp_bf16(ref) / 8).clamp_min(2.0 ** -25)  # fp16 subnormals
+    assert ((out.double().cpu() - ref).abs() <= half + ref.abs() * 2.0 ** -18).all()
