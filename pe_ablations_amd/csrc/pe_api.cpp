@@ -609,6 +609,7 @@ namespace {
 // Work split and workspace of pe_attn_decode: transformed queries, then the per-range partials.
 struct DecodePlan {
   int nqt, nunit;
+  bool own_max;       // see DecodeArgs
   bool chunk;         // many query rows: the forward kernel over key ranges (cp), not the decode kernel
   pe::ChunkPlan cp;
   size_t q_bytes, po_off, pm_off, pl_off, total;
@@ -638,7 +639,8 @@ DecodePlan decode_plan(const pe_attn_params* p) {
   // up to 512 rows one workgroup takes the whole cache, four blocks a wave, and needs no merge launch (one token,
   // 8 -> 4 heads of the split form, 500 rows: 17.8 us of GPU time in four launches, 12.9 in two
   // with the query transform in the split kernel too; 33.4 -> 27.6 us a step with the host's share)
-  if (nkb <= 16) nu = 4;
+  d.own_max = nkb <= 16;
+  if (d.own_max) nu = 4;
   nu = std::max<int64_t>(4, std::min<int64_t>(512, (nu + 3) / 4 * 4));
   d.nunit = (int)nu;
   size_t rows = (size_t)tiles * d.nunit * 32;
@@ -748,7 +750,7 @@ int pe_attn_decode(const pe_attn_params* p, const pe_tensor_t* qc, const pe_tens
   da.causal = p->causal != PE_CAUSAL_NONE;
   da.off = p->causal == PE_CAUSAL_BOTTOM_RIGHT ? p->Sk - p->Sq : 0;
   da.scale = p->scale;
-  da.nqt = d.nqt; da.nunit = d.nunit;
+  da.nqt = d.nqt; da.nunit = d.nunit; da.own_max = d.own_max;
   da.part_o = (float*)(ws + d.po_off);
   da.part_m = (float*)(ws + d.pm_off);
   da.part_l = (float*)(ws + d.pl_off);

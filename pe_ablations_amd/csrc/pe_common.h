@@ -190,10 +190,11 @@ template <int N> __device__ __forceinline__ void apply_scale_sign(float scale, u
 }
 
 // Online softmax whose reference m may step down to a tile's own max mx, so that the tile's largest
-// probability is 1 and has no rounding: allowed as long as the sum so far, lsum, stays below 480 relative
-// to it (a tile adds at most 32 or 96), which bounds the accumulators by 576 times the largest value.
-__device__ __forceinline__ bool own_max_ok(float lsum, float m, float mx) {
-  return lsum * __builtin_amdgcn_exp2f(m - mx) < 480.f;  // false for a tile without a key: mx = -inf
+// probability is 1 and has no rounding: allowed as long as the sum so far, lsum, stays below `limit`
+// relative to it, so that with the tile's own at most 32 or 96 the accumulators stay below limit + 96 times
+// the largest value, as they do without stepping down over a range of that many keys.
+__device__ __forceinline__ bool own_max_ok(float lsum, float m, float mx, float limit) {
+  return lsum * __builtin_amdgcn_exp2f(m - mx) < limit;  // false for a tile without a key: mx = -inf
 }
 
 // 8 consecutive elements of type XT kept as loaded (16 or 32 bytes) until they are used

@@ -182,16 +182,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       mx = fmaxf(mx, x);
     }
     mx = fmaxf(mx, xor32(mx));
-    // the reference is the running max; with four ranges (a few blocks a wave) it steps down to the block's own
-    // where that is at most 2^6 below and the sum small, so that each block's largest probability is 1 and has
-    // no rounding, as with a range a block (512 rows, split form, relative to 64 bits: 2.18e-3 with 16 ranges,
-    // 2.23e-3 with four and the running max)
-    if (a.nunit == 4) {
-      const float lsum = l + xor32(l);
-      mx = mx > m - 6.f && lsum < 1024.f ? mx : fmaxf(m, mx);
-    } else {
-      mx = fmaxf(m, mx);
-    }
+    // the reference is the running max; in the plan of a short cache (a few blocks a wave) it steps down to the
+    // block's own, so that each block's largest probability is 1 and has no rounding, as with a range a block
+    // (512 rows, split form, relative to 64 bits: 2.18e-3 with 16 ranges, 2.23e-3 with four and the running
+    // max).  Longer ranges keep the running max: their sums would be at the limit most of the time
+    mx = DT != 1 && a.own_max && own_max_ok(l + xor32(l), m, mx, 96.f) ? mx : fmaxf(m, mx);
     const float alpha = exp2f(m - mx);
     m = mx;
     float rs = 0.f;

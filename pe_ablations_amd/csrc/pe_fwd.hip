@@ -383,7 +383,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void fwd_bf16_kernel(Core
       for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[nt][j]);
     mx = fmaxf(mx, xor32(mx)) * (MB ? 1.f : sl2);
     // SK: P relative to the tile's own max, see own_max_ok
-    const float mn = SK && own_max_ok(l + xor32(l), m, mx) ? mx : fmaxf(m, mx);
+    const float mn = SK && own_max_ok(l + xor32(l), m, mx, 480.f) ? mx : fmaxf(m, mx);
     if (__any(SK ? mn != m : mx > m + tau)) {
       const float alpha = fast_exp2(m - mn);
       m = mn;

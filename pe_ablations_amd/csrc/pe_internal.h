@@ -205,6 +205,7 @@ struct DecodeArgs {
   // qcraw (B, Hq, Sq, Dc); null: q holds the rows the prologue transformed
   const void* qraw; int64_t qr_s[4]; const float* freqs; int Dr, start_pos, pos_round;
   const void* qcraw; int64_t qc_s[4]; int Dc;
+  int own_max;      // short cache: each block's probabilities relative to its own max (16-bit types)
 };
 int launch_decode(int dt, int dqk, int dv, const DecodeArgs& a, hipStream_t s);
 // Many new query rows against a cache (a prompt prefilled in chunks), 16-bit operands: the forward

@@ -73,3 +73,30 @@ def test_reference_follows_falling_and_rising_blocks(cuda, dt, step):
     ref = s.softmax(-1).unsqueeze(-2) @ v.double().repeat_interleave(Hq // Hkv, 1)
     assert err(out, ref) < (2 ** -8 if dt == torch.bfloat16 else 2 ** -11) * float(v.abs().max())
     assert err(lse[..., 0], s.logsumexp(-1)) < 2 ** -21 * max(16.0, abs(step) * 16)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("step", [0.0, 4.9, 5.9])
+def test_long_caches_of_many_tiles(cuda, dt, step):
+    """256 (batch entry, kv head) units leave four ranges each, merged in the workgroup, also for a cache of
+    1100 rows: nine blocks a wave, whose scores fall by ``step`` powers of two a block.  Values of 2^114 (not
+    in fp16): sums must stay within 2^14 of the largest value.  Bar as above, fp32 sums: 2^-18."""
+    g = torch.Generator(device="cuda").manual_seed(7)
+    B, Hq, Hkv, L, Dc, Dr, Dv = 32, 16, 8, 1100, 64, 32, 64
+    qc, kc = torch.zeros(B, Hq, 1, Dc, dtype=dt, device=cuda), torch.zeros(B, Hkv, L, Dc, dtype=dt, device=cuda)
+    qc[..., 0] = 8.0
+    kc[..., 0] = (-step * math.log(2.0) * (torch.arange(L, device=cuda) // 32)).to(dt)
+    qr = torch.full((B, Hq, 1, Dr), -30.0, dtype=dt, device=cuda)
+    kr = torch.zeros(B, Hkv, L, Dr, dtype=dt, device=cuda)
+    v = ((1 + torch.rand(B, Hkv, L, Dv, generator=g, device=cuda)) * (1.0 if dt == torch.float16 else 2.0 ** 114)).to(dt)
+    freqs = O.pope_freqs(Dr).cuda()
+    wk, wv = cache_widths(d_content=Dc, d_pe=Dr, d_v=Dv)
+    ck, cv = (torch.zeros(B, Hkv, L, w, dtype=dt, device=cuda) for w in (wk, wv))
+    pe_cache_append(kr, v, ck, cv, start_pos=0, k_c=kc, freqs=freqs)
+    with torch.no_grad():
+        out, lse = pe_attention_decode(qr, ck, cv, L, q_c=qc, d_v=Dv, freqs=freqs, scale=0.125, return_lse=True)
+    s = kc[..., 0].double().repeat_interleave(Hq // Hkv, 1)
+    ref = s.softmax(-1).unsqueeze(-2) @ v.double().repeat_interleave(Hq // Hkv, 1)
+    bar = {torch.bfloat16: 2 ** -8, torch.float16: 2 ** -11, torch.float32: 2 ** -18}[dt]
+    assert err(out, ref) < bar * float(v.abs().max())
+    assert err(lse[..., 0], s.logsumexp(-1)) < 2 ** -21 * max(16.0, abs(step) * 35)
