@@ -27,7 +27,10 @@ class SwiGLU(nn.Module):
         if x.is_cuda and x.dtype == torch.bfloat16 and gate.dtype == torch.bfloat16 and x.shape == gate.shape:
             if not torch.is_grad_enabled():
                 return _hip_swiglu(x, gate)
-            if x.numel() > 0 and x.numel() % 8 == 0 and x.device == gate.device and plain_autograd(x, gate):
+            # the Function keeps both inputs, the expression the gate only where the gate needs a gradient and
+            # x likewise only then
+            if (x.requires_grad and gate.requires_grad and x.numel() > 0 and x.numel() % 8 == 0
+                    and x.device == gate.device and plain_autograd(x, gate)):
                 return SwiGLUFn.apply(x, gate)
         return F.silu(gate) * x
 

@@ -34,10 +34,12 @@ class RMSNorm(nn.Module):
                 and self.weight.dtype in (torch.bfloat16, torch.float32)):
             if not torch.is_grad_enabled():
                 return _hip_rms_norm(x, self.weight, self.eps)
-            if (x.numel() > 0 and self.weight.shape == (n,) and self.weight.device == x.device
+            # the Function keeps x and the weight, the expression only where x needs a gradient: without one,
+            # both may be changed in place afterwards, and x may be an inference tensor
+            if (x.requires_grad and x.numel() > 0 and self.weight.shape == (n,) and self.weight.device == x.device
                     and plain_autograd(x, self.weight) and (x.data_ptr() | self.weight.data_ptr()) % 16 == 0):
-                # the expression's fp32 cast leaves a 16-bit x free to be changed in place afterwards; the
-                # Function keeps x itself, so it is given a copy (an fp32 x the expression keeps as well)
+                # the expression's fp32 cast leaves a 16-bit x free to be changed in place as well; the
+                # Function keeps x itself, so it is given a copy
                 return RMSNormFn.apply(x if x.dtype == torch.float32 else x.clone(), self.weight, self.eps)
         return self._norm(x.float()).type_as(x) * self.weight
 

@@ -140,3 +140,58 @@ def test_rmsnorm_half_input_changed_in_place_afterwards(cuda):
         x += 1.0
         grads.append(torch.autograd.grad((y * y * y).sum() + x.sum(), leaf)[0])
     assert near(grads[0], grads[1], 2 ** -7)
+
+
+def outcome(fn, make, needs, touch):
+    """What a call and its backward give when the tensor named by ``touch`` is changed in place between the
+    two: the gradients, or "error"."""
+    t = make()
+    for n in needs:
+        t[n].requires_grad_()
+    y = fn(t)
+    if touch:
+        with torch.no_grad():
+            t[touch].add_(1.0)
+    try:
+        return torch.autograd.grad(y.sum(), [t[n] for n in needs])
+    except RuntimeError:
+        return "error"
+
+
+@pytest.mark.parametrize("touch", ["", "x", "w"])
+@pytest.mark.parametrize("needs", [("x",), ("w",), ("x", "w")])
+@pytest.mark.parametrize("op", ["norm32", "norm16", "swiglu"])
+def test_changes_in_place_are_refused_where_the_expression_refuses_them(cuda, op, needs, touch):
+    def make():
+        g = torch.Generator(device="cuda").manual_seed(11)
+        x = torch.randn(6, 64, generator=g, device="cuda")
+        w = torch.randn(6, 64, generator=g, device="cuda") if op == "swiglu" else 1 + 0.1 * torch.randn(64, generator=g, device="cuda")
+        return {"x": x if op == "norm32" else x.to(B16), "w": w.to(B16) if op == "swiglu" else w}
+
+    def module(t):
+        if op == "swiglu":
+            return SwiGLU()(t["x"], t["w"])
+        m = RMSNorm(64).cuda()
+        del m.weight
+        m.weight = t["w"]
+        return m(t["x"])
+
+    def expression(t):
+        return F.silu(t["w"]) * t["x"] if op == "swiglu" else rms_norm_expression(t["x"], t["w"], 1e-6)
+
+    got, want = outcome(module, make, needs, touch), outcome(expression, make, needs, touch)
+    assert (got == "error") == (want == "error")
+    if got != "error":
+        for a, b in zip(got, want):
+            assert near(a, b, 2e-6 if op == "norm32" else 2 ** -7)
+
+
+def test_inference_tensors_without_a_gradient(cuda):
+    """Frozen features made under inference mode, in front of a norm that is trained."""
+    with torch.inference_mode():
+        x = torch.randn(6, 64, device="cuda")
+    m = RMSNorm(64).cuda()
+    dy = torch.randn(6, 64, device="cuda")
+    got, = torch.autograd.grad(m(x), m.weight, dy)
+    want, = torch.autograd.grad(rms_norm_expression(x.clone(), m.weight, m.eps), m.weight, dy)
+    assert near(got, want, 2e-6)
