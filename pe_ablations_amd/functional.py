@@ -658,12 +658,15 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.
 def plain_autograd(*tensors: torch.Tensor) -> bool:
     """Whether ordinary eager autograd is all that looks at these tensors, so that one fused Function may
     stand for a chain of torch ops: plain CUDA tensors, no functorch transform (vmap, jvp, grad), no
-    forward-mode level, no tracing or compiling, and no dispatch or function mode that would see the ops."""
-    return (all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+    batched gradients (is_grads_batched runs the backward under the older vmap), no forward-mode level, no
+    tracing or compiling, and no dispatch or function mode that would see the ops."""
+    return (not torch.compiler.is_compiling()  # first: a compiler traces nothing of the rest
+            and all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter)
+                    and not torch._C._functorch.is_legacy_batchedtensor(t) for t in tensors)
             and torch._C._functorch.peek_interpreter_stack() is None
             and torch.autograd.forward_ad._current_level < 0
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing())
+            and not torch.jit.is_tracing())
 
 
 def rms_norm_expression(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
@@ -672,10 +675,20 @@ def rms_norm_expression(x: torch.Tensor, weight: torch.Tensor, eps: float) -> to
     return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps)).type_as(x) * weight
 
 
+def _expression_grads(expression, inputs, ctx, dy):
+    """The gradients that ctx needs of its first inputs, through the torch expression a Function stands for."""
+    create_graph = torch.is_grad_enabled()
+    need = [t for t, n in zip(inputs, ctx.needs_input_grad) if n]
+    with torch.enable_grad():
+        grads = iter(torch.autograd.grad(expression(), need, dy, create_graph=create_graph))
+    return tuple(next(grads) if n else None for n in ctx.needs_input_grad[:len(inputs)])
+
+
 class RMSNormFn(torch.autograd.Function):
     """rms_norm with pe_rmsnorm_bwd as its backward (one launch forward, two backward, in place of the
-    expression's six and about twelve).  Under create_graph the backward differentiates the torch
-    expression instead, so higher derivatives are those of the expression."""
+    expression's six and about twelve).  Under create_graph, and where dy is not a plain tensor (batched
+    gradients: is_grads_batched, jacobian(vectorize=True)), the backward differentiates the torch expression
+    instead, so higher derivatives and batches of them are those of the expression."""
 
     @staticmethod
     def forward(ctx, x, weight, eps):
@@ -686,19 +699,16 @@ class RMSNormFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, weight = ctx.saved_tensors
-        if torch.is_grad_enabled():
-            y = rms_norm_expression(x, weight, ctx.eps)
-            need = [t for t, n in zip((x, weight), ctx.needs_input_grad) if n]
-            grads = iter(torch.autograd.grad(y, need, dy, create_graph=True))
-            return tuple(next(grads) if n else None for n in ctx.needs_input_grad[:2]) + (None,)
+        if torch.is_grad_enabled() or not plain_autograd(dy):
+            return _expression_grads(lambda: rms_norm_expression(x, weight, ctx.eps), (x, weight), ctx, dy) + (None,)
         if dy.data_ptr() % 16:  # contiguous() would return such a view as it is
             dy = dy.clone(memory_format=torch.contiguous_format)
         return rms_norm_backward(x, weight, dy, ctx.eps) + (None,)
 
 
 class SwiGLUFn(torch.autograd.Function):
-    """swiglu (bf16) with pe_swiglu_bwd as its backward; under create_graph the backward differentiates
-    F.silu(gate) * x."""
+    """swiglu (bf16) with pe_swiglu_bwd as its backward; under create_graph and with batched gradients the
+    backward differentiates F.silu(gate) * x (as RMSNormFn)."""
 
     @staticmethod
     def forward(ctx, x, gate):
@@ -708,10 +718,8 @@ class SwiGLUFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, gate = ctx.saved_tensors
-        if torch.is_grad_enabled():
-            need = [t for t, n in zip((x, gate), ctx.needs_input_grad) if n]
-            grads = iter(torch.autograd.grad(torch.nn.functional.silu(gate) * x, need, dy, create_graph=True))
-            return tuple(next(grads) if n else None for n in ctx.needs_input_grad)
+        if torch.is_grad_enabled() or not plain_autograd(dy):
+            return _expression_grads(lambda: torch.nn.functional.silu(gate) * x, (x, gate), ctx, dy)
         xc, gc, dc = x.contiguous(), gate.contiguous(), dy.contiguous()
         if any(t.data_ptr() % 16 for t in (xc, gc, dc)):
             xc, gc, dc = (t.clone(memory_format=torch.contiguous_format) for t in (xc, gc, dc))

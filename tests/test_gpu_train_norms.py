@@ -195,3 +195,23 @@ def test_inference_tensors_without_a_gradient(cuda):
     got, = torch.autograd.grad(m(x), m.weight, dy)
     want, = torch.autograd.grad(rms_norm_expression(x.clone(), m.weight, m.eps), m.weight, dy)
     assert near(got, want, 2e-6)
+
+
+def test_batched_gradients(cuda):
+    """is_grads_batched and jacobian(vectorize=True), whose backward sees functorch tensors."""
+    g = torch.Generator(device="cuda").manual_seed(13)
+    m = RMSNorm(16).cuda()
+    x = torch.randn(4, 16, generator=g, device="cuda", requires_grad=True)
+    dys = torch.randn(5, 4, 16, generator=g, device="cuda")
+    y, ref = m(x), rms_norm_expression(x, m.weight, m.eps)
+    assert y.grad_fn.name().startswith("RMSNormFn")
+    for a, b in zip(torch.autograd.grad(y, (x, m.weight), dys, is_grads_batched=True),
+                    torch.autograd.grad(ref, (x, m.weight), dys, is_grads_batched=True)):
+        assert near(a, b, 2e-6)
+    jac = torch.autograd.functional.jacobian
+    assert near(jac(m, x, vectorize=True), jac(lambda z: rms_norm_expression(z, m.weight, m.eps), x, vectorize=True), 2e-6)
+    u, v, d = (torch.randn(n, 4, 16, generator=g, device="cuda").to(B16) for n in (1, 1, 5))
+    u, v = u[0].requires_grad_(), v[0].requires_grad_()
+    for a, b in zip(torch.autograd.grad(SwiGLU()(u, v), (u, v), d, is_grads_batched=True),
+                    torch.autograd.grad(F.silu(v) * u, (u, v), d, is_grads_batched=True)):
+        assert torch.equal(a, b)

@@ -96,3 +96,10 @@ def test_hot_path_refuses_cpu_tensors():
         m(torch.randn(1, 4, 64))
     with pytest.raises(RuntimeError, match="GPU only"):
         PoPEEmbedding(8, 64).forward_query(torch.randn(1, 4, 2, 8))
+
+
+def test_a_compiler_takes_the_torch_expressions_in_one_graph():
+    from pe_ablations_amd.functional import plain_autograd
+    f = torch.compile(lambda t: t * 2 if plain_autograd(t) else t * 3, fullgraph=True, backend="eager")
+    t = torch.ones(3, requires_grad=True)
+    assert torch.equal(f(t), t * 3)
