@@ -44,7 +44,11 @@ enum {
 
 /* element types of tensors crossing the boundary.  A compute dtype (pe_attn_params.dtype) of bf16
  * or fp16 runs the matrix products on 16-bit operands with fp32 accumulation (fp16: the reference
- * trainer's mixed_precision fp16, src/training/trainer.py:343-347); fp32 runs them in fp32. */
+ * trainer's mixed_precision fp16, src/training/trainer.py:343-347); fp32 runs them to fp32's precision:
+ * with an explicit mask on the fp32 matrix unit, else as products of operands held exactly in three bf16
+ * values.  The latter keep an operand below 2^-109 to 2^-134 absolute, give infinities and NaN where fp32
+ * products do for infinite operands (0 times an infinity of a tensor's last row, in a tile that reaches past
+ * it, is NaN there too), and NaN in dq / dk where dS overflows. */
 enum { PE_DTYPE_BF16 = 0, PE_DTYPE_FP32 = 1, PE_DTYPE_FP16 = 2 };
 /* element type of an explicit attention mask only: one byte per element, nonzero = the key takes
  * part (torch.bool, SDPA's boolean attn_mask) */

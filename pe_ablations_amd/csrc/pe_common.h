@@ -142,9 +142,37 @@ __device__ __forceinline__ void split_bf3(float x0, float x1, uint32_t& h, uint3
   l = pack_bf2(x0, x1);
 }
 
+// split_bf3 of operand values, any of which may be infinite or round to a bf16 infinity.  An infinity goes
+// into l alone: l meets only the other operand's h, which has that value's sign and is 0 for 0 alone, so the
+// products are an infinity or, with 0, NaN, as fp32's are (in h it would meet planes of either sign and
+// zeros).  A finite value that rounds up to infinity has h cut short instead, 16 more bits for m and l.
+__device__ __forceinline__ void split_operand(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+  split_bf3(x0, x1, h, m, l);
+  const uint32_t u0 = __builtin_bit_cast(uint32_t, x0) & 0x7fffffffu, u1 = __builtin_bit_cast(uint32_t, x1) & 0x7fffffffu;
+  if ((u0 > u1 ? u0 : u1) < 0x7f7f8000u) return;  // 2^128 (1 - 2^-9)
+  auto one = [](float x, uint32_t& a, uint32_t& b, uint32_t& c) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, x);
+    if ((u & 0x7fffffffu) == 0x7f800000u) {
+      a = b = 0u;
+      c = u >> 16;
+    } else if ((u & 0x7fffffffu) >= 0x7f7f8000u && (u & 0x7fffffffu) < 0x7f800000u) {
+      a = u >> 16;
+      x -= __builtin_bit_cast(float, u & 0xffff0000u);
+      b = pack_bf2(x, 0.f) & 0xffffu;
+      c = pack_bf2(x - __builtin_bit_cast(float, b << 16), 0.f) & 0xffffu;
+    }
+  };
+  uint32_t a = h & 0xffffu, b = m & 0xffffu, c = l & 0xffffu, d = h >> 16, e = m >> 16, f = l >> 16;
+  one(x0, a, b, c);
+  one(x1, d, e, f);
+  h = a | d << 16;
+  m = b | e << 16;
+  l = c | f << 16;
+}
+
 // Operand rows (the prologue's output): row `row`, columns c .. c + 7 of rows of `width` elements.
 // dtype 3: three bf16 planes of `width` elements one after another in each row, holding h, m and l of
-// split_bf3 (the fp32 compute type's operands for the matrix cores)
+// split_operand (the fp32 compute type's operands for the matrix cores)
 constexpr int DT_SPLIT = 3;  // DT_SPLIT_CODE on the host side
 __device__ __forceinline__ void row_store8(void* dst, int64_t row, int width, int c, int dtype, const float (&x)[8]) {
   if (dtype == DT_SPLIT) {
@@ -153,7 +181,7 @@ __device__ __forceinline__ void row_store8(void* dst, int64_t row, int width, in
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       uint32_t a, b, d;
-      split_bf3(x[2 * e], x[2 * e + 1], a, b, d);
+      split_operand(x[2 * e], x[2 * e + 1], a, b, d);
       h[e] = a; m[e] = b; l[e] = d;
     }
     *(u32x4*)p = h;
@@ -168,7 +196,7 @@ __device__ __forceinline__ void row_store(void* dst, int64_t row, int width, int
   if (dtype == DT_SPLIT) {
     uint16_t* p = (uint16_t*)dst + row * 3 * width + c;
     uint32_t h, m, l;
-    split_bf3(x, 0.f, h, m, l);
+    split_operand(x, 0.f, h, m, l);
     p[0] = (uint16_t)h; p[width] = (uint16_t)m; p[2 * width] = (uint16_t)l;
   } else {
     store_from_float(dst, row * width + c, dtype, x);

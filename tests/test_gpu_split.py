@@ -86,3 +86,42 @@ def test_noalloc_takes_fp32_calls_that_fit_only_as_fp32_operands(cuda):
     assert rc0 == 0 and rc1 == 0
     assert (out0 - out1).abs().max() < 1e-5 and (lse0 - lse1).abs().max() < 1e-5
     assert math.isfinite(out1.sum().item())
+
+
+@pytest.mark.parametrize("D,Dv,causal", [(64, 64, True), (128, 64, False), (256, 128, True), (40, 48, True)])
+def test_infinite_operands(cuda, D, Dv, causal):
+    """Infinities in the values, a key and the output's gradient, against the fp32 unit (which an explicit mask
+    selects): out, lse and dv infinite, NaN and finite at the same places.  (Whole tiles: the two fill a tile's
+    missing rows differently, and 0 times an infinity there is NaN.)"""
+    x, dout = case(1, 2, 2, 96, 96, D, Dv, "top_left", 0.1, seed=3)
+    x["v"][0, 0, 5, 3], x["v"][0, 0, 40, 7], x["v"][0, 1, 0, 1] = math.inf, -math.inf, math.inf
+    x["q"][0, :, :, 2] = x["q"][0, :, :, 2].abs() + 0.1
+    x["k"][0, 1, 50, 2] = -math.inf  # never attended to: q there is positive
+    dout[0, 0, 60, 9], dout[0, 1, 95, 0] = -math.inf, math.inf
+    res = []
+    for mask in (None, torch.ones(1, 1, 1, 96, dtype=torch.bool, device=cuda)):
+        leaves = [x[n].to(cuda).requires_grad_() for n in "qkv"]
+        out, lse = pe_attention(*leaves, mode="none", scale=0.1, causal=causal, mask=mask, return_lse=True)
+        res.append((out, lse, torch.autograd.grad(out, leaves[2], dout.to(cuda))[0]))
+    for a, b in zip(*res):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()) and torch.equal(a[a.isinf()], b[b.isinf()])
+        fin = b.isfinite()
+        assert fin.any() and (a - b)[fin].abs().max() < 2e-5
+    assert res[0][0].isinf().any() and res[0][2].isinf().any()
+
+
+def test_values_at_the_ends_of_the_range(cuda):
+    """The largest finite values, whose bf16 rounding is infinite, and small ones.  Of an operand below
+    2^-109 the planes hold what is at least 2^-134 of it (half the smallest bf16 subnormal)."""
+    q = torch.zeros(1, 1, 64, 64, device=cuda)
+    v = torch.full((1, 1, 64, 64), torch.finfo(torch.float32).max, device=cuda)
+    v[..., 1::2] *= -1.0
+    out = pe_attention(q, q, v, mode="none", scale=0.1, causal="top_left")
+    assert torch.equal(out[0, 0, 0], v[0, 0, 0])  # one key: its value
+    g = torch.Generator(device=cuda).manual_seed(2)
+    q, k, v = (torch.randn(1, 1, 64, 64, generator=g, device=cuda) for _ in range(3))
+    for e in (-100, -110, -116, -120):
+        out = pe_attention(q, k, v * 2.0 ** e, mode="none", scale=0.1)
+        ref, _ = O.attention(q.cpu().double(), k.cpu().double(), (v * 2.0 ** e).cpu().double(), 0.1, True)
+        d = (out.cpu().double() - ref).abs().max().item()
+        assert d < 1e-5 * 2.0 ** e + 2.0 ** -133
