@@ -172,7 +172,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       if constexpr (NEXT) kf[kk] = *(const u32x4*)(krn + kk * KC + g * EPL);
     }
     __builtin_amdgcn_sched_barrier(0);
-    float mx = -INFINITY;
+    float mx = DT == 1 ? m : -INFINITY;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       const int key = k0 + c_logical<DT>(j, g);
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // block's own, so that each block's largest probability is 1 and has no rounding, as with a range a block
     // (512 rows, split form, relative to 64 bits: 2.18e-3 with 16 ranges, 2.23e-3 with four and the running
     // max).  Longer ranges keep the running max: their sums would be at the limit most of the time
-    mx = DT != 1 && a.own_max && own_max_ok(l + xor32(l), m, mx, 96.f) ? mx : fmaxf(m, mx);
+    if constexpr (DT != 1) mx = a.own_max && own_max_ok(l + xor32(l), m, mx, 96.f) ? mx : fmaxf(m, mx);
     const float alpha = exp2f(m - mx);
     m = mx;
     float rs = 0.f;
@@ -239,28 +239,42 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
       for (int t = 0; t < NOT; ++t)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) ro[(w * 32 + l32) * RS + t * 32 + c_row(j, g)] = o[t][j];
+        for (int j = 0; j < 16; j += 4)
+          *(f32x4*)(ro + (w * 32 + l32) * RS + t * 32 + c_row(j, g)) = f32x4{o[t][j], o[t][j + 1], o[t][j + 2], o[t][j + 3]};
       if (g == 0) {
         rm[w * 32 + l32] = m;
         rl[w * 32 + l32] = lt;
       }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < nreal * DV; i += 256) {
-      const int x = i / DV, c = i % DV, rq = qt * 32 + x;
-      const float M = fmaxf(fmaxf(rm[x], rm[32 + x]), fmaxf(rm[64 + x], rm[96 + x]));
-      float acc = 0.f, lsum = 0.f;
+    // W columns a thread: one for a few rows, whose columns the threads just cover, four for more: the weights
+    // of a row are worked out by each of its threads, and with one column each a tile of 32 rows of 128 took
+    // longer than the merge kernel's launch (one kv head, 64 rows against 64, 200 and 256 cached ones: 14.2 /
+    // 17.7 / 18.9 us of GPU time with that launch, 16.3 / 19.5 / 20.3 by columns, 12.4 / 15.7 / 16.5 by fours)
+    auto merge = [&](auto width) {
+      constexpr int W = decltype(width)::value, CPR = DV / W;
+      for (int i = threadIdx.x; i < nreal * CPR; i += 256) {
+        const int x = i / CPR, c = i % CPR * W, rq = qt * 32 + x;
+        const float M = fmaxf(fmaxf(rm[x], rm[32 + x]), fmaxf(rm[64 + x], rm[96 + x]));
+        float acc[W] = {}, lsum = 0.f;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float wt = exp2f(rm[u * 32 + x] - M);
-        lsum += rl[u * 32 + x] * wt;
-        acc += ro[(u * 32 + x) * RS + c] * wt;
+        for (int u = 0; u < 4; ++u) {
+          const float wt = exp2f(rm[u * 32 + x] - M);
+          lsum += rl[u * 32 + x] * wt;
+#pragma unroll
+          for (int e = 0; e < W; ++e) acc[e] += ro[(u * 32 + x) * RS + c + e] * wt;
+        }
+        const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+        const int ho = hk * grp + rq / a.Sq, iq = rq % a.Sq;
+        const int64_t o0 = b * a.o_sb + ho * a.o_sh + (int64_t)iq * a.o_ss + c;
+#pragma unroll
+        for (int e = 0; e < W; ++e)
+          if (c + e < a.dv_real) store_from_float(a.o, o0 + e, a.o_dtype, lsum > 0.f ? acc[e] * inv : 0.f);
+        if (c == 0) a.lse[(int64_t)(b * a.Hq + ho) * a.Sq + iq] = lsum > 0.f ? (M + log2f(lsum)) * LN2 : -INFINITY;
       }
-      const int ho = hk * grp + rq / a.Sq, iq = rq % a.Sq;
-      if (c < a.dv_real)
-        store_from_float(a.o, b * a.o_sb + ho * a.o_sh + (int64_t)iq * a.o_ss + c, a.o_dtype, lsum > 0.f ? acc * (1.f / lsum) : 0.f);
-      if (c == 0) a.lse[(int64_t)(b * a.Hq + ho) * a.Sq + iq] = lsum > 0.f ? (M + log2f(lsum)) * LN2 : -INFINITY;
-    }
+    };
+    if (nreal * DV <= 512) merge(std::integral_constant<int, 1>{});
+    else merge(std::integral_constant<int, 4>{});
     return;
   }
   if (r >= nrows) return;

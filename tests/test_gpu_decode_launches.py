@@ -27,6 +27,8 @@ pytestmark = pytest.mark.gpu
     (torch.bfloat16, 1, 2, 1, 513, 4, 0, 128, 128),    # the merge kernel
     (torch.bfloat16, 1, 16, 2, 300, 1, 128, 64, 128),  # QK width 256, eight rows a tile
     (torch.bfloat16, 2, 12, 2, 200, 9, 0, 64, 64),     # 54 rows, two tiles, prologue launch
+    (torch.bfloat16, 1, 12, 1, 200, 2, 64, 32, 48),    # 24 rows merged four columns at a time, padded values
+    (torch.float16, 1, 10, 2, 90, 7, 0, 128, 128),     # 35 rows: a full tile and three rows
 ])
 def test_decode_matches_oracle_and_the_prologue_launch(cuda, dt, B, Hq, Hkv, L, Sq, Dc, Dr, Dv):
     g = torch.Generator().manual_seed(L)
