@@ -24,7 +24,8 @@ namespace pe {
 // file then holds the q~ fragments' ring, the k~ fragments of the block in flight and the PV
 // accumulators without spills (352 VGPRs at QK 256 / V 128 in bf16; 2.7 % faster than the
 // 256-register build, which spilled around its loop).
-template <int DT, int DQK, int DV>
+// MERGE: four ranges are merged in the workgroup.
+template <int DT, int DQK, int DV, bool MERGE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void decode_split_kernel(DecodeArgs a) {
   using E = typename Elem<DT>::T;
   using M = MT<DT>;
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   // are neither written nor read)
   const int64_t pb = ((int64_t)bh * a.nqt + qt) * a.nunit + u;
   const float lt = l + xor32(l);
-  if (a.nunit == 4) {
+  if (MERGE && a.nunit == 4) {
     // the whole cache in one workgroup (short caches, or many tiles): its four ranges merged here in LDS, in
     // range order, with the merge kernel's formula, in place of that kernel's launch
     constexpr int RS = DV + 4;
@@ -366,7 +367,13 @@ __global__ __launch_bounds__(1024) void decode_merge_kernel(DecodeArgs a) {
 template <int DT, int DQK, int DV>
 static int run_decode(const DecodeArgs& a, hipStream_t s) {
   const int64_t blocks = (int64_t)a.B * a.Hkv * a.nqt * (a.nunit / 4);
-  hipLaunchKernelGGL((decode_split_kernel<DT, DQK, DV>), dim3((unsigned)blocks), dim3(256), 0, s, a);
+  // fp32 at QK width 256, V width 128 has no registers to spare (the merge spills 48 instead of 15, 16 heads
+  // behind 16384 rows 112 instead of 107 us): longer caches run it without the merge
+  constexpr bool MERGE = !(DT == 1 && DQK == 256 && DV == 128);
+  if (MERGE || a.nunit == 4)
+    hipLaunchKernelGGL((decode_split_kernel<DT, DQK, DV, true>), dim3((unsigned)blocks), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((decode_split_kernel<DT, DQK, DV, MERGE>), dim3((unsigned)blocks), dim3(256), 0, s, a);
   if (a.nunit > 4) {  // four ranges are one workgroup, which merges them itself
     const int64_t rows = (int64_t)a.B * a.Hkv * a.nqt * std::min(32, (a.Hq / a.Hkv) * a.Sq);
     hipLaunchKernelGGL((decode_merge_kernel<DV>), dim3((unsigned)rows), dim3(1024), 0, s, a);
