@@ -656,6 +656,12 @@ bool prep_vec_query_ok(const PrepArgs& a) {
   return prep_vec_ok(a) && a.xr_dtype == a.dst_dtype && (a.dst_dtype == 0 || a.dst_dtype == 2) && !a.is_key;
 }
 
+// Up to this many transformed elements, fp32 rows keep a wave per row: eight softplus and sin / cos in series
+// per thread take longer than a few thousand rows' traffic (an append of key and value rows of width 64, with
+// a wave per row against eight columns a thread: one row 4.0 / 4.9 us, 1024 rows 4.8 / 5.8, 4096 5.8 / 6.2; of
+// width 128: 4.3 / 4.9, 5.4 / 5.8, 4096 rows 6.6 / 6.6).
+constexpr int64_t PREP_FEW_F32_ELEMS = 4096 * 128;
+
 int launch_prep(const PrepArgs& a, hipStream_t s) {
   const int64_t nrows = (int64_t)a.B * a.H * a.S;
   const bool vec = prep_vec_ok(a);
@@ -667,7 +673,7 @@ int launch_prep(const PrepArgs& a, hipStream_t s) {
     const dim3 grid((unsigned)((nthr + 255) / 256));
     if (a.dst_dtype == 0) hipLaunchKernelGGL(prep_pope_small_kernel<0>, grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL(prep_pope_small_kernel<2>, grid, dim3(256), 0, s, a);
-  } else if (vec) {
+  } else if (vec && (a.dst_dtype != 1 || nrows * a.Dr > PREP_FEW_F32_ELEMS)) {
     const int64_t nthr = nrows * (a.Dr / 8);
     with_prep_types(prep_vec_types(a), [&](auto xt, auto dt) {
       hipLaunchKernelGGL((prep_pope_vec_kernel<decltype(xt)::value, decltype(dt)::value>),
