@@ -609,7 +609,7 @@ namespace {
 // Work split and workspace of pe_attn_decode: transformed queries, then the per-range partials.
 struct DecodePlan {
   int nqt, nunit;
-  bool own_max;       // see DecodeArgs
+  bool short_cache;   // the whole cache in one workgroup, a few blocks a wave
   bool chunk;         // many query rows: the forward kernel over key ranges (cp), not the decode kernel
   pe::ChunkPlan cp;
   size_t q_bytes, po_off, pm_off, pl_off, total;
@@ -636,11 +636,15 @@ DecodePlan decode_plan(const pe_attn_params* p) {
   // count, not the device's: the workspace query and the call must size the partials alike.
   int64_t nu = (1024 + tiles - 1) / tiles;
   nu = std::min<int64_t>(nu, (nkb + 1) / 2);
-  // up to 512 rows one workgroup takes the whole cache, four blocks a wave, and needs no merge launch (one token,
-  // 8 -> 4 heads of the split form, 500 rows: 17.8 us of GPU time in four launches, 12.9 in two
-  // with the query transform in the split kernel too; 33.4 -> 27.6 us a step with the host's share)
-  d.own_max = nkb <= 16;
-  if (d.own_max) nu = 4;
+  // A short cache goes to one workgroup, a few blocks a wave, which merges its four ranges itself and needs no
+  // merge launch, as long as that takes no more GPU time than more ranges and the launch (us, that / this):
+  // one token, 8 -> 4 heads of the split form, 512 rows 14.2 / 10.8; QK width 256, one head, 384 rows 12.9 /
+  // 13.0, 448 rows 13.0 / 14.8; fp32, split form, 320 rows 19.6 / 21.5, 512 rows 19.8 / 25.8; 64 rows of values
+  // 128 wide, 320 cached ones 16.9 / 18.9.  Up to 256 rows the count above gives four ranges anyway.
+  const int tile_rows = (int)std::min<int64_t>(32, (int64_t)grp * p->Sq);
+  const bool more = half_dt(p->dtype) && (pad_v(p->Dv) == 64 || tile_rows <= 16);
+  d.short_cache = nkb <= (!more ? 8 : pad_qk(qk_width(p)) < 256 ? 16 : 12);
+  if (d.short_cache) nu = 4;
   nu = std::max<int64_t>(4, std::min<int64_t>(512, (nu + 3) / 4 * 4));
   d.nunit = (int)nu;
   size_t rows = (size_t)tiles * d.nunit * 32;
@@ -750,7 +754,7 @@ int pe_attn_decode(const pe_attn_params* p, const pe_tensor_t* qc, const pe_tens
   da.causal = p->causal != PE_CAUSAL_NONE;
   da.off = p->causal == PE_CAUSAL_BOTTOM_RIGHT ? p->Sk - p->Sq : 0;
   da.scale = p->scale;
-  da.nqt = d.nqt; da.nunit = d.nunit; da.own_max = d.own_max;
+  da.nqt = d.nqt; da.nunit = d.nunit; da.own_max = d.short_cache;
   da.part_o = (float*)(ws + d.po_off);
   da.part_m = (float*)(ws + d.pm_off);
   da.part_l = (float*)(ws + d.pl_off);

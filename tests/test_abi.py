@@ -274,3 +274,22 @@ def test_masked_entry_points_validate_the_mask(lib):
         assert call(mask(dtype=_lib.PE_DTYPE_BF16, offset=1)) == _lib.ERRORS["PE_ERR_STRIDE"]
         # a valid mask passes on to the operand checks (qr missing: PE_ERR_NULL from them)
         assert call(mask()) == _lib.ERRORS["PE_ERR_NULL"]
+
+
+def test_decode_ranges_of_short_caches(lib):
+    """The key ranges of a decode call, read off its workspace (per range and 32-row tile Wv + 2 floats a
+    row): four, merged in one workgroup, up to 512 cached rows in 16 bits with narrow operands, 384 at QK
+    width 256 and 256 in fp32 and for tiles of many rows of wide values; beyond, one per two 32-key blocks."""
+    lib.pe_attn_decode_workspace_bytes.restype = ctypes.c_size_t
+
+    def ranges(L, Dv=64, rows=1, **kw):
+        p = params(**dict(dict(Hq=rows, Hkv=1, Sq=1, Sk=L, Dv=Dv, causal=_lib.PE_CAUSAL_BOTTOM_RIGHT), **kw))
+        queries = rows * lib.pe_attn_operand_width(ctypes.byref(p)) * (4 if p.dtype == _lib.PE_DTYPE_FP32 else 2)
+        return int((lib.pe_attn_decode_workspace_bytes(ctypes.byref(p)) - queries) / (32 * 4 * (Dv + 2)))
+
+    f32 = dict(dtype=_lib.PE_DTYPE_FP32)
+    for L in (1, 256):
+        assert ranges(L) == ranges(L, **f32) == ranges(L, Dr=128, Dv=128, rows=32) == 4
+    assert ranges(512) == ranges(512, rows=32) == ranges(384, Dr=128, Dv=128) == 4
+    assert ranges(513) == ranges(576) == 12
+    assert ranges(385, Dr=128, Dv=128) == ranges(257, **f32) == ranges(257, Dr=128, Dv=128, rows=32) == 8
