@@ -624,6 +624,21 @@ struct DecodePlan {
 // each 22.9 / 27.0 against 16000.
 constexpr int64_t CHUNK_MIN_ROWS = 64, CHUNK_MIN_ALL_ROWS = 640;
 
+// Whether `rows` query rows of each of `heads` kv heads go to the forward kernel.  Not where the decode kernel
+// merges a short cache in one round of workgroups: GPU time of decode / forward kernel, us, at 512 rows, 16
+// heads of 64 (split form), 64 new rows 14.9 / 15.7, 500 new rows 16.1 / 21.7, 4 x 16 heads, 100 new rows 18.8 /
+// 18.6, 8 x 16, 250: 53 / 30; at QK width 256, 384 rows, 4 x 16 heads, 100: 24.5 / 25.8, 512 rows: 28.2 / 25.9.
+// Beyond, up to 1024 rows in all, the forward kernel needs key tiles enough to have ranges: QK width 256, one
+// kv head, 800 new rows against 300 / 600 / 800 / 1100 cached ones 22.4 / 27.0, 24.5 / 25.5, 25.3 / 25.5, 26.5 /
+// 26.2 (256-row blocks), 8 kv heads, 128 rows each 300: 22.7 / 24.5, 384: 23.6 / 19.7 (128-row blocks); QK
+// width 128, 4 kv heads, 200 rows each 300: 20.8 / 22.0, 384: 21.3 / 17.3.
+bool chunk_pays(const pe::ChunkPlan& cp, int64_t rows, int64_t heads, int sk, int dqk, int nunit) {
+  if (rows < CHUNK_MIN_ROWS || rows * heads < CHUNK_MIN_ALL_ROWS) return false;
+  if (nunit == 4 && heads * ((rows + 31) / 32) <= kSplitCus && sk <= (dqk < 256 ? 512 : 384)) return false;
+  const int few = cp.bm == 256 ? (dqk < 256 ? 384 : 1024) : (dqk < 256 ? 0 : 384);
+  return rows * heads > 1024 || sk >= few;
+}
+
 DecodePlan decode_plan(const pe_attn_params* p) {
   DecodePlan d{};
   const int grp = p->Hq / p->Hkv;
@@ -647,12 +662,15 @@ DecodePlan decode_plan(const pe_attn_params* p) {
   if (d.short_cache) nu = 4;
   nu = std::max<int64_t>(4, std::min<int64_t>(512, (nu + 3) / 4 * 4));
   d.nunit = (int)nu;
+  // the partials hold either kernel's: a cache grows from one plan into the other in the same workspace
   size_t rows = (size_t)tiles * d.nunit * 32;
-  const int64_t crows = (int64_t)grp * p->Sq;
-  d.chunk = half_dt(p->dtype) && crows >= CHUNK_MIN_ROWS && crows * p->B * p->Hkv >= CHUNK_MIN_ALL_ROWS;
-  if (d.chunk) {
-    d.cp = pe::chunk_plan(crows, (int64_t)p->B * p->Hkv, p->Sk, pad_qk(qk_width(p)));
-    rows = (size_t)d.cp.nblk * d.cp.bm * d.cp.nsplit * p->B * p->Hkv;
+  const int64_t crows = (int64_t)grp * p->Sq, heads = (int64_t)p->B * p->Hkv;
+  if (half_dt(p->dtype)) {
+    const int dqk = pad_qk(qk_width(p));
+    d.cp = pe::chunk_plan(crows, heads, p->Sk, dqk);
+    d.chunk = chunk_pays(d.cp, crows, heads, p->Sk, dqk, d.nunit);
+    if (crows >= CHUNK_MIN_ROWS && crows * heads >= CHUNK_MIN_ALL_ROWS)
+      rows = std::max(rows, (size_t)d.cp.nblk * d.cp.bm * d.cp.nsplit * heads);
   }
   d.q_bytes = align_up((size_t)p->B * p->Hq * p->Sq * pad_qk(qk_width(p)) * esz(p));
   d.po_off = d.q_bytes;

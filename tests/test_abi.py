@@ -293,3 +293,16 @@ def test_decode_ranges_of_short_caches(lib):
     assert ranges(512) == ranges(512, rows=32) == ranges(384, Dr=128, Dv=128) == 4
     assert ranges(513) == ranges(576) == 12
     assert ranges(385, Dr=128, Dv=128) == ranges(257, **f32) == ranges(257, Dr=128, Dv=128, rows=32) == 8
+
+
+@pytest.mark.parametrize("kw", [dict(Hq=16, Hkv=16, Sq=64, Dr=128, Dv=128), dict(Hq=8, Hkv=1, Sq=100), dict(Hq=4, Hkv=4, Sq=200),
+                                dict(B=2, Hq=8, Hkv=4, Sq=1), dict(B=4, Hq=16, Hkv=16, Sq=100, dtype=_lib.PE_DTYPE_FP16),
+                                dict(Hq=1, Hkv=1, Sq=700, Dr=128, Dv=128), dict(Hq=8, Hkv=8, Sq=8, dtype=_lib.PE_DTYPE_FP32)])
+def test_decode_workspace_for_the_capacity_serves_every_length(lib, kw):
+    """A cache's workspace is sized once, for its capacity; as it fills, calls pass from plan to plan (ranges
+    per workgroup, the forward kernel over key ranges) and none may ask for more."""
+    lib.pe_attn_decode_workspace_bytes.restype = ctypes.c_size_t
+    lengths = [n for n in list(range(1, 1300)) + list(range(1300, 20000, 97)) if n >= kw["Sq"]]
+    sizes = [lib.pe_attn_decode_workspace_bytes(ctypes.byref(params(**dict(kw, Sk=n, causal=_lib.PE_CAUSAL_BOTTOM_RIGHT))))
+             for n in lengths]
+    assert sizes[0] > 0 and all(a <= b for a, b in zip(sizes, sizes[1:]))

@@ -29,6 +29,9 @@ CASES = [  # mode, dtype, B, Hq, Hkv, L, Sq, Dc, Dr, Dv, causal
     ("none", "fp16", 1, 3, 3, 640, 600, 0, 64, 128, "bottom_right"),    # the first range ends before the diagonal
     ("pope", "bf16", 1, 2, 2, 1100, 321, 0, 128, 64, "none"),           # QK width 256, no mask
     ("pope", "bf16", 1, 1, 1, 1300, 1300, 0, 128, 128, "bottom_right"),  # every row new: rows with one visible key
+    ("rope", "bf16", 4, 16, 4, 256, 100, 0, 64, 64, "bottom_right"),     # short caches: the decode kernel, 208 tiles
+    ("pope", "bf16", 2, 16, 16, 300, 64, 0, 128, 128, "bottom_right"),   # one range, 2048 rows in all
+    ("pope", "fp16", 4, 16, 4, 200, 200, 64, 32, 64, "bottom_right"),    # more tiles than the decode kernel takes at once
 ]
 
 
