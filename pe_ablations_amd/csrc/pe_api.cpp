@@ -64,22 +64,34 @@ bool fused_bwd(const pe_attn_params* p) {
 // on the device queried), so a workspace size taken before any device call stays valid.
 constexpr int kSplitCus = 256;
 
-// dK/dV pair kernel (16-bit, transformed width 128 / 256, value width 64 / 128): workgroups per key block.
-// A causal block's work falls with its key position, from every query tile to one, so a grid of one
-// workgroup per compute unit waits for its first blocks; from one and a half a unit on, issued longest
-// first, they even out (384 blocks: as fast whole as halved).  Below that the query heads of the GQA group are shared out (a power of two dividing it) and, past
-// 512 queries, their query tiles, as long as a range keeps four 64-query tiles (up to 512 the workspace
-// keeps the size it had).  Forward and backward on one GPU, without against with: 16 -> 4 heads of 128, RoPE,
-// 4 x 2048 rows 502 / 433 us; 16 heads of 128, 1024 rows 157 / 147; 4 heads of 128, 4096 rows 403 / 333,
-// 1200 rows 162 / 124; 8 heads of 128, 4 x 600 rows 127 / 114; 16 heads of 64, 2048 rows 175 / 160.
+// dK/dV pair kernel (16-bit, transformed width 128 / 256, value width 64 / 128): workgroups per key block, which
+// share out its list of (query head of the GQA group, query tile).  Below one workgroup per compute unit a power
+// of two of the group's heads, or past 512 queries of the list (up to 512 the workspace keeps its size; sharing
+// out would gain there too: 16 heads of 64, 512 rows 70 / 63 us), as long as a range keeps four 64-query tiles;
+// past eight ranges 32, or adding them up costs more than it saves (16 -> 1 heads of 64, forward and backward
+// in a graph, 8 / 16 ranges: 512 rows 85 / 97 us, 1024 rows 120 / 124, 2048 rows 200 / 173; 64 -> 1, 1024 rows,
+// 8 / 32: 277 / 231).
+// A causal block's work falls with its key position, from every query tile to one, so a grid of one workgroup
+// per compute unit still waits for its first blocks, a longer one the less the more blocks even out.  Two
+// ranges then pay for long lists only (whole / halved, us): 256 blocks, QK width 128: 4 x 8 heads, 1024 rows
+// 116 / 110, 4 x 16 -> 4, 2048 rows 361 / 326; QK width 256: 4 x 16 -> 8, 1024 rows 220 / 230, 2 x 16 -> 8, 2048
+// rows 344 / 327; 320 blocks: 10 x 16 -> 8, 512 rows 138 / 152, 5 x 8 heads, 1024 rows 126 / 137, 10 heads, 2048
+// rows 178 / 176 (QK width 256: 268 / 289), 4096 rows 298 / 281; 312 blocks, 6 x 16 -> 4 RoPE heads, 1600 rows
+// (100 tiles) 462 / 444; 384 blocks: as fast whole as halved.
 int key_split(const pe_attn_params* p, int dqk, int dv) {
   if (!half_dt(p->dtype) || !((dqk == 128 || dqk == 256) && (dv == 64 || dv == 128))) return 1;
   const int grp = p->Hq / p->Hkv;
   const int64_t blocks = (int64_t)p->B * p->Hkv * ((p->Sk + 127) / 128);
-  const int64_t even = p->causal != PE_CAUSAL_NONE ? kSplitCus * 3 / 2 : kSplitCus;
-  const int tiles = grp * ((p->Sq + 63) / 64);
+  const int64_t tiles = (int64_t)grp * ((p->Sq + 63) / 64);
+  const bool waits = p->causal != PE_CAUSAL_NONE &&
+                     (blocks <= kSplitCus ? p->Sq >= (dqk < 256 ? 1024 : 2048)
+                                          : blocks < kSplitCus * 3 / 2 && (p->Sq >= 4096 || tiles >= 96));
   int ks = 1;
-  while (ks < 8 && blocks * ks < (ks == 1 ? even : kSplitCus) && (grp % (2 * ks) == 0 || (p->Sq > 512 && tiles / (2 * ks) >= 4))) ks *= 2;
+  while (blocks * ks < kSplitCus || (ks == 1 && waits)) {
+    const bool heads = grp % (2 * ks) == 0;
+    if (!(ks < 8 ? heads || (p->Sq > 512 && tiles / (2 * ks) >= 4) : heads && tiles / (2 * ks) >= 32)) break;
+    ks *= 2;
+  }
   return ks;
 }
 

@@ -1001,9 +1001,14 @@ __global__ __launch_bounds__(512, 1) void dkdv_pair_kernel(CoreArgs a) {
   if (a.causal) qb0 = max(0, k0 - off) / BMQ;
   if (qb0 > nqt) qb0 = nqt;
   const int nper = nqt - qb0, ntot = nper * grp;
-  // (ntot * qsplit < 2^31: at most 8 ranges; in scalar registers, as the tile addresses are)
-  const int it0 = QS ? __builtin_amdgcn_readfirstlane((uint32_t)(ntot * jq) / (uint32_t)a.qsplit) : 0;
-  const int niter = QS ? __builtin_amdgcn_readfirstlane((uint32_t)(ntot * (jq + 1)) / (uint32_t)a.qsplit) - it0 : ntot;
+  // the jq-th of qsplit ranges: ntot jq / qsplit without the product; in scalar registers, as the tile
+  // addresses are
+  auto range = [&](int j) {
+    const uint32_t n = (uint32_t)ntot / (uint32_t)a.qsplit, r = (uint32_t)ntot % (uint32_t)a.qsplit;
+    return (int)__builtin_amdgcn_readfirstlane(n * (uint32_t)j + r * (uint32_t)j / (uint32_t)a.qsplit);
+  };
+  const int it0 = QS ? range(jq) : 0;
+  const int niter = QS ? range(jq + 1) - it0 : ntot;
   const int h_first = hk * grp + (QS && nper > 0 ? it0 / nper : 0);
   const int qt_first = qb0 + (QS && nper > 0 ? it0 % nper : 0);
   const float sl2 = score_factor(a.scale);

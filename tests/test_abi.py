@@ -306,3 +306,19 @@ def test_decode_workspace_for_the_capacity_serves_every_length(lib, kw):
     sizes = [lib.pe_attn_decode_workspace_bytes(ctypes.byref(params(**dict(kw, Sk=n, causal=_lib.PE_CAUSAL_BOTTOM_RIGHT))))
              for n in lengths]
     assert sizes[0] > 0 and all(a <= b for a, b in zip(sizes, sizes[1:]))
+
+
+@pytest.mark.parametrize("kw,slices", [
+    (dict(B=1, Hq=16, Hkv=1, Sq=512), 8), (dict(B=1, Hq=16, Hkv=1, Sq=1024), 8), (dict(B=1, Hq=16, Hkv=1, Sq=2048), 16),
+    (dict(B=1, Hq=64, Hkv=1, Sq=1024), 32), (dict(B=1, Hq=8, Hkv=8, Sq=512), 1), (dict(B=1, Hq=8, Hkv=8, Sq=513), 2),
+    (dict(B=10, Hq=16, Hkv=8, Sq=512), 1), (dict(B=4, Hq=8, Hkv=8, Sq=1024), 2), (dict(B=4, Hq=8, Hkv=8, Sq=1024, Dr=128, Dv=128), 1),
+    (dict(B=5, Hq=8, Hkv=8, Sq=1024), 1), (dict(B=1, Hq=10, Hkv=10, Sq=4096), 2), (dict(B=6, Hq=16, Hkv=4, Sq=1600), 2),
+    (dict(B=1, Hq=12, Hkv=12, Sq=4096), 1), (dict(B=1, Hq=8, Hkv=8, Sq=4096, causal=_lib.PE_CAUSAL_NONE), 1)])
+def test_bwd_workspace_reserves_the_query_range_partials(lib, kw, slices):
+    """The slices of fp32 dK~ and dV partials of the 16-bit backward: what its workspace holds more than the
+    explicit-mask backward's at the pair kernel's widths, which has none."""
+    p = params(**dict(kw, Sk=kw["Sq"]))
+    lib.pe_attn_bwd_workspace_bytes.restype = lib.pe_attn_bwd_masked_workspace_bytes.restype = ctypes.c_size_t
+    extra = lib.pe_attn_bwd_workspace_bytes(ctypes.byref(p)) - lib.pe_attn_bwd_masked_workspace_bytes(ctypes.byref(p))
+    each = p.B * p.Hkv * p.Sk * (2 * p.Dr + p.Dv) * 4
+    assert abs(extra - (slices * each if slices > 1 else 0)) < 4096, (extra / each, slices)

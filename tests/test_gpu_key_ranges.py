@@ -23,6 +23,8 @@ pytestmark = pytest.mark.gpu
     ("bf16", 1, 4, 2, 600, 777, 256, 128, "bottom_right"),
     ("bf16", 2, 2, 1, 530, 530, 256, 64, False),
     ("fp16", 1, 4, 1, 640, 640, 200, 96, True),            # padded widths
+    ("bf16", 1, 16, 1, 2001, 2001, 128, 64, True),         # sixteen ranges, last block with as many tiles
+    ("fp16", 1, 64, 1, 520, 1000, 128, 128, "bottom_right"),  # sixteen ranges of four heads
 ])
 def test_ranges_match_oracle(cuda, dtype, B, Hq, Hkv, Sq, Sk, D, Dv, causal):
     dt = torch.bfloat16 if dtype == "bf16" else torch.float16
