@@ -97,10 +97,11 @@ int key_split(const pe_attn_params* p, int dqk, int dv) {
 
 // Ranges that the split backward (pe_split.hip) cuts each 128-key block's list of (query head, query tile)
 // into: doubled up to 4 while the key blocks give fewer workgroups than two per compute unit and the first
-// block keeps at least eight tiles a range (4 x 8 -> 4 heads, 1024 rows, 128 key blocks, the longest of 64
-// tiles: see split_sum_kernel).  `batch` 1: the ranges that the workspace reserves, whatever the batch.
-int split_ranges(const pe_attn_params* p, int batch) {
-  const int64_t blocks = (int64_t)batch * p->Hkv * ((p->Sk + 127) / 128);
+// block keeps at least eight tiles a range (whole / two / four ranges, forward and backward, us: 4 x 8 -> 4
+// heads of the split form, 1024 rows, 128 key blocks, 400 / 346 / 331; 16 x 8 -> 4, 512 rows, 256 blocks 354 /
+// 352 / 381; 64 x 8 -> 4, 1024 blocks 1222 / 1307 / 1437).
+int split_ranges(const pe_attn_params* p) {
+  const int64_t blocks = (int64_t)p->B * p->Hkv * ((p->Sk + 127) / 128);
   const int tiles = p->Hq / p->Hkv * ((p->Sq + 31) / 32);
   int n = 1;
   while (n < 4 && blocks * n < 2 * kSplitCus && tiles / (2 * n) >= 8) n *= 2;
@@ -165,18 +166,14 @@ Layout layout(const pe_attn_params* p, bool masked = false, bool unit = false) {
   L.dq_off = L.l2_off + align_up(nq_pad * 4);
   const bool fb = !gm && fused_bwd(p);
   L.ksplit = masked ? 1 : key_split(p, L.dqk, L.dv);
-  int slices = L.ksplit;
-  if (L.split) {
-    L.ksplit = split_ranges(p, p->B);
-    slices = split_ranges(p, 1);
-  }
+  if (L.split) L.ksplit = split_ranges(p);
   L.dk_off = L.dq_off + (fb ? 0 : align_up(nq * L.dqk * 4));
   // dk~ (unfused) or the split's partial dk~ slices
-  L.pq_off = L.dk_off + (fb && slices == 1 ? 0 : align_up(nk * L.dqk * 4 * slices));
+  L.pq_off = L.dk_off + (fb && L.ksplit == 1 ? 0 : align_up(nk * L.dqk * 4 * L.ksplit));
   L.pk_off = L.pq_off + align_up((size_t)L.nq_blocks * p->Dr * 4);
   L.pkd_off = L.pk_off + align_up((size_t)L.nk_blocks * p->Dr * 4);
   L.dvp_off = L.pkd_off + align_up((size_t)L.nk_blocks * p->Dr * 4);
-  L.rtab_off = L.dvp_off + (slices > 1 ? align_up(nk * L.dv * 4 * slices) : 0);
+  L.rtab_off = L.dvp_off + (L.ksplit > 1 ? align_up(nk * L.dv * 4 * L.ksplit) : 0);
   // the fused RoPE gradient's angles (cos / sin, fp32 [Sq][2][Dr / 2]), written by the backward's dO pass
   L.ds_off = L.rtab_off + (half_dt(p->dtype) && p->mode == PE_MODE_ROPE ? align_up((size_t)p->Sq * p->Dr * 4) : 0);
   // bf16 path: dS in fragment order, 4 KiB blocks packed per (b, h) to the blocks the causal
