@@ -47,8 +47,9 @@ enum {
  * trainer's mixed_precision fp16, src/training/trainer.py:343-347); fp32 runs them to fp32's precision:
  * with an explicit mask on the fp32 matrix unit, else as products of operands held exactly in three bf16
  * values.  The latter keep an operand below 2^-109 to 2^-134 absolute, give infinities and NaN where fp32
- * products do for infinite operands (0 times an infinity of a tensor's last row, in a tile that reaches past
- * it, is NaN there too), and NaN in dq / dk where dS overflows. */
+ * products do for infinite values, gradients, content parts and keys or queries without PoPE (0 times an
+ * infinity of a tensor's last row, in a tile that reaches past it, is NaN there too), NaN for infinite
+ * inputs of PoPE, and NaN in dq / dk where dS overflows. */
 enum { PE_DTYPE_BF16 = 0, PE_DTYPE_FP32 = 1, PE_DTYPE_FP16 = 2 };
 /* element type of an explicit attention mask only: one byte per element, nonzero = the key takes
  * part (torch.bool, SDPA's boolean attn_mask) */

@@ -142,8 +142,8 @@ __device__ __forceinline__ void prep_pope_norm_body(const PrepArgs& a, int blk, 
         store8(tab_out, (int64_t)s * 2 * a.Dr + a.Dr + t * 8, 1, sn8);
       }
       const int64_t drow = (int64_t)(b * a.H + h) * a.S + s;
-      row_store8(a.dst, drow, a.width, a.Dc + t * 8, DDT, cv);
-      row_store8(a.dst, drow, a.width, a.Dc + a.Dr + t * 8, DDT, sv);
+      row_store8<false>(a.dst, drow, a.width, a.Dc + t * 8, DDT, cv);
+      row_store8<false>(a.dst, drow, a.width, a.Dc + a.Dr + t * 8, DDT, sv);
     }
   }
   if (a.Dc > 0) {  // content part: converted copy
@@ -160,7 +160,7 @@ __device__ __forceinline__ void prep_pope_norm_body(const PrepArgs& a, int blk, 
   for (int c = lane; c < a.H * ppr; c += 64) {
     const int h = c / ppr, j = c - h * ppr;
     const float z[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    row_store8(a.dst, (int64_t)(b * a.H + h) * a.S + s, a.width, used + j * 8, DDT, z);
+    row_store8<false>(a.dst, (int64_t)(b * a.H + h) * a.S + s, a.width, used + j * 8, DDT, z);
   }
 }
 

@@ -342,8 +342,8 @@ __device__ __forceinline__ void prep_pope_vec_body(const PrepArgs& a, int64_t gi
       }
     }
   }
-  row_store8(a.dst, drow, a.width, a.Dc + t * 8, DT, cv);
-  row_store8(a.dst, drow, a.width, a.Dc + a.Dr + t * 8, DT, sv);
+  row_store8<false>(a.dst, drow, a.width, a.Dc + t * 8, DT, cv);
+  row_store8<false>(a.dst, drow, a.width, a.Dc + a.Dr + t * 8, DT, sv);
   if (a.Dc > 0) {
     const int64_t xc0 = b * a.xc_s[0] + h * a.xc_s[1] + (int64_t)s * a.xc_s[2];
     if constexpr (XT == DT) {  // content rows of the same type (prep_vec_ok)
@@ -361,7 +361,7 @@ __device__ __forceinline__ void prep_pope_vec_body(const PrepArgs& a, int64_t gi
     }
   }
   const float zero[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int j = (a.Dc + 2 * a.Dr) / 8 + t; j < a.width / 8; j += tpr) row_store8(a.dst, drow, a.width, j * 8, DT, zero);
+  for (int j = (a.Dc + 2 * a.Dr) / 8 + t; j < a.width / 8; j += tpr) row_store8<false>(a.dst, drow, a.width, j * 8, DT, zero);
   if (a.cdst) {  // the row's companion copy (KV-cache append: the value row), 16-bit elements
     const uint16_t* crow = (const uint16_t*)a.cv + b * a.cv_s[0] + h * a.cv_s[1] + (int64_t)s * a.cv_s[2];
     uint16_t* cd = (uint16_t*)a.cdst + ((int64_t)bh * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s) * a.cwidth;
@@ -505,7 +505,7 @@ __global__ __launch_bounds__(256) void prep_rope_vec_kernel(PrepArgs a, int lg_t
     }
   }
   const float zero[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int j = (a.Dc + a.Dr) / 8 + t; j < a.width / 8; j += tpr) row_store8(a.dst, drow, a.width, j * 8, a.dst_dtype, zero);
+  for (int j = (a.Dc + a.Dr) / 8 + t; j < a.width / 8; j += tpr) row_store8<false>(a.dst, drow, a.width, j * 8, a.dst_dtype, zero);
 }
 
 // Both sides of a RoPE / no-PE prologue without a content part in one launch, RHG heads per thread: thread
@@ -759,8 +759,8 @@ __device__ __forceinline__ void prep_pope_qheads_body(const PrepArgs& a, int64_t
       sv[e] = mul_nc(mu, sn[e]);
     }
     const int64_t drow = (int64_t)(b * a.H + h) * (a.dst_rows ? a.dst_rows : a.S) + a.dst_row0 + s;
-    row_store8(a.dst, drow, a.width, t * 8, DT, cv);
-    row_store8(a.dst, drow, a.width, a.Dr + t * 8, DT, sv);
+    row_store8<false>(a.dst, drow, a.width, t * 8, DT, cv);
+    row_store8<false>(a.dst, drow, a.width, a.Dr + t * 8, DT, sv);
   }
 }
 

@@ -4,7 +4,7 @@
 // h l' + m m' + l h' are kept, six bf16 instructions for sixteen times the rate.  What is left out
 // (m l' + l m' + l l') is below 2^-24 of the product, with the sign of rounding errors: less than the
 // rounding of one fp32 product.  The products themselves are exact and the sums are fp32, as on the fp32
-// unit.  Infinite operands give infinities and NaN where the fp32 unit gives them (split_operand); a dS that
+// unit.  Infinite operands give infinities and NaN where the fp32 unit gives them (split_big); a dS that
 // overflows gives NaN in dq and dk.
 //
 // Operand rows hold their planes one after another (row_store8, DT_SPLIT), so a tile is three bf16 tiles
