@@ -1768,6 +1768,7 @@ __global__ __launch_bounds__(NW * 64, 1) void dq_gemm_kernel(CoreArgs a) {
   }
   if constexpr (DQK == 128) {
     if (a.rope_fuse) {  // 128 of the block's 256 queries at a time
+      static_assert(SMEM >= 128 * DQK * 4, "staged dq~ rows fit the ring");
       float* st = (float*)smem;  // [128 queries][128]
       for (int half = 0; half < 2; ++half)
         rope_epi_rows<HT, DQK, NW * 64, 128>(a, a.eq, st, tid, q0 + half * 128, a.Sq, b, h, [&] {

@@ -432,7 +432,7 @@ int launch_swiglu_bwd(const void* x, const void* gate, const void* dy, void* dx,
 
 static int prep_norm_check(const PrepArgs& a) {
   if (a.mode != 0 || !a.norm_w || a.norm_w_dtype < 0 || a.norm_w_dtype > 2 || a.xr_dtype < 0 || a.xr_dtype > 2 ||
-      a.dst_dtype < 0 || a.dst_dtype > DT_SPLIT)
+      !(a.dst_dtype == 0 || a.dst_dtype == 2 || a.dst_dtype == DT_SPLIT))
     return -4;
   if (a.dst_rows != 0 || a.dst_row0 != 0) return -2;  // writes contiguous (B, H, S, width) rows only
   if (a.Dr <= 0 || a.Dr % 8 != 0 || a.Dc % 8 != 0 || a.width % 8 != 0 || a.H * (a.Dr / 8) > 64 * MAXCPL) return -3;
@@ -456,7 +456,6 @@ int launch_prep_norm(const PrepArgs& aq, const PrepArgs& ak, float* tab, hipStre
     auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(WPB * 64), 0, s, aq, ak, (unsigned)nq, tab); };
     if (aq.dst_dtype == 0) go(prep_pope_norm_kernel<0, C>);
     else if (aq.dst_dtype == 2) go(prep_pope_norm_kernel<2, C>);
-    else if (aq.dst_dtype == 1) go(prep_pope_norm_kernel<1, C>);
     else go(prep_pope_norm_kernel<DT_SPLIT, C>);
   });
   return hipGetLastError() == hipSuccess ? 0 : -7;
