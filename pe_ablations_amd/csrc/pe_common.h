@@ -220,12 +220,14 @@ __device__ __forceinline__ void row_store(void* dst, int64_t row, int width, int
 __device__ __forceinline__ float score_factor(float scale) {
   return scale == 0.f ? 0x1p-126f : __builtin_fabsf(scale) * LOG2E;
 }
+// (In a branch: as an unconditional xor it cost fp16 dK/dV at QK width 128, V width 64, 2 % of its 96 us.)
 template <int N> __device__ __forceinline__ void apply_scale_sign(float scale, u32x4 (&f)[N]) {
-  const uint32_t flip = scale < 0.f ? 0x80008000u : 0u;
+  if (__builtin_expect(scale < 0.f, 0)) {
 #pragma unroll
-  for (int i = 0; i < N; ++i)
+    for (int i = 0; i < N; ++i)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) f[i][e] ^= flip;
+      for (int e = 0; e < 4; ++e) f[i][e] ^= 0x80008000u;
+  }
 }
 
 // Online softmax whose reference m may step down to a tile's own max mx, so that the tile's largest
