@@ -298,8 +298,7 @@ int pe_rmsnorm_bwd(const void* x, int32_t x_dtype, int64_t x_row_stride, int64_t
 /* SwiGLU forward of the feed-forward block (src/model/ffn.py:17-27, SwiGLU.forward(x, gate) =
  * F.silu(gate) * x): out = bf16(bf16(gate / (1 + exp(-gate))) * x) element by element over n
  * contiguous bf16 values, bitwise what torch computes for the two bf16 ops.  n % 8 == 0, 16-byte
- * aligned pointers (out may alias x or gate).  Forward only: the module calls it when no gradient
- * is needed. */
+ * aligned pointers (out may alias x or gate). */
 int pe_swiglu_fwd(const void* x, const void* gate, void* out, int64_t n, void* stream);
 /* Its gradients for the output gradient dy, as autograd computes them through the two torch ops:
  * dx = dy * silu(gate), dgate = (dy * x) * silu'(gate); same layout and alignment. */

@@ -1396,8 +1396,9 @@ __global__ __launch_bounds__(512, 1) void dkdv_pair_kernel(CoreArgs a) {
   if constexpr (!QS) dk_epilogue<HT, DQK, DV>(a, st_epi, tid, b, hk, kb, bh, nkb);
 }
 
-// The query split of the pair kernel (a.qsplit > 1, see key_split in pe_api.cpp): one workgroup of 512 threads per key block of (b, hk) adds the qsplit fp32 partials of
-// dV and dK~ in slice order, stores dV in dv's dtype, and either runs the dK~ epilogue
+// The query split of the pair kernel (a.qsplit > 1, see key_split in pe_api.cpp): one workgroup of 512
+// threads per key block of (b, hk) adds the qsplit fp32 partials of dV and dK~ in slice order, stores dV in
+// dv's dtype, and either runs the dK~ epilogue
 // (a.fuse_inv, a.rope_fuse) or leaves the sum in slice 0 of dk_t for the stand-alone inverse-transform kernels.
 // Both paths see the same sums, so the fused and unfused gradients stay bitwise equal.  It runs as
 // extra workgroups of the dQ GEMM's launch (the two are independent), on the compute units that a

@@ -631,7 +631,7 @@ def rms_norm_backward(x: torch.Tensor, weight: torch.Tensor, dy: torch.Tensor, e
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
     """RMSNorm forward over the last dim through pe_rmsnorm_fwd (src/model/normalization.py:22-27):
     (x * rsqrt(mean(x^2) + eps)).type_as(x) * weight, result dtype bf16 when x and weight are both
-    bf16, else fp32.  No autograd: the module uses it when no gradient is needed."""
+    bf16, else fp32.  No autograd of its own (RMSNormFn)."""
     if not x.is_cuda:
         raise RuntimeError("rms_norm runs on the GPU only (got a CPU tensor)")
     if x.dtype not in (torch.bfloat16, torch.float32, torch.float16) or \
@@ -732,8 +732,8 @@ class SwiGLUFn(torch.autograd.Function):
 
 def swiglu(x: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     """F.silu(gate) * x over bf16 through pe_swiglu_fwd (src/model/ffn.py:17-27), bitwise torch's
-    result for the two bf16 ops, in one pass.  Both tensors bf16, same shape, on the GPU.  No
-    autograd: the module uses it when no gradient is needed."""
+    result for the two bf16 ops, in one pass.  Both tensors bf16, same shape, on the GPU.  No autograd of
+    its own (SwiGLUFn)."""
     if not (x.is_cuda and gate.is_cuda):
         raise RuntimeError("swiglu runs on the GPU only")
     if x.dtype != torch.bfloat16 or gate.dtype != torch.bfloat16 or x.shape != gate.shape:

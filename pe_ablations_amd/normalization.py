@@ -3,8 +3,9 @@
 RMSNorm: x * rsqrt(mean(x^2) + eps) in fp32, cast back to x's dtype, times the weight (which
 promotes the result to fp32 when the weight is fp32, the precision the PoPE transform then sees).
 On the GPU it runs the library's one-pass HIP kernel (pe_rmsnorm_fwd), in training with
-pe_rmsnorm_bwd as its backward (RMSNormFn); elsewhere, and where something other than plain autograd
-looks at the ops (functorch, forward mode, tracing), it is the reference's torch expression.  On the position projections of the PoPE attention, inference skips the module
+pe_rmsnorm_bwd as its backward (RMSNormFn) where x needs a gradient; elsewhere, and where something
+other than plain autograd looks at the ops (functorch, forward mode, tracing), it is the reference's
+torch expression.  On the position projections of the PoPE attention the module is skipped
 altogether: the norm is fused into the attention's transform kernel.  QKNorm is fused into the
 attention kernel for the RoPE / no-PE modules (qk_l2norm); the module form here serves direct
 callers.

@@ -2,8 +2,9 @@
 ranges merged in the workgroup, against the paths they replace.
 
 A query view whose rows start at an odd element is transformed by the prologue launch, an aligned one in the
-kernel, with the same arithmetic: bitwise equal results.  Caches of up to 512 rows are merged in the
-workgroup, longer ones by the merge kernel; both are held to the oracle at the decode bars.
+kernel, with the same arithmetic: bitwise equal results.  Short caches (see decode_plan in pe_api.cpp) and
+those of 256 or more tiles are merged in the workgroup, the others by the merge kernel; all are held to the
+oracle at the decode bars.
 """
 
 import math
