@@ -25,7 +25,7 @@ __device__ __forceinline__ float wave_sum(float x) {
 
 constexpr int MAX_PAIRS_PER_LANE = 4;  // RoPE rows up to 512 dims
 
-__global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
+template <bool SPLIT> __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int64_t nrows = (int64_t)a.B * a.H * a.S;
@@ -38,7 +38,7 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
 
   for (int c = lane; c < a.Dc; c += 64) {
     const float x = load_as_float(a.xc, b * a.xc_s[0] + h * a.xc_s[1] + (int64_t)s * a.xc_s[2] + c * a.xc_s[3], a.xc_dtype);
-    row_store(a.dst, drow, a.width, c, a.dst_dtype, x);
+    row_store<SPLIT>(a.dst, drow, a.width, c, a.dst_dtype, x);
   }
   const int64_t xr0 = b * a.xr_s[0] + h * a.xr_s[1] + (int64_t)s * a.xr_s[2];
   int used = a.Dc;
@@ -50,8 +50,8 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
       if (a.is_key && a.delta) ph = add_nc(ph, a.delta[h * a.delta_hs + c]);
       float sn, cs;
       pe_sincos(ph, sn, cs);
-      row_store(a.dst, drow, a.width, a.Dc + c, a.dst_dtype, mul_nc(mu, cs));
-      row_store(a.dst, drow, a.width, a.Dc + a.Dr + c, a.dst_dtype, mul_nc(mu, sn));
+      row_store<SPLIT>(a.dst, drow, a.width, a.Dc + c, a.dst_dtype, mul_nc(mu, cs));
+      row_store<SPLIT>(a.dst, drow, a.width, a.Dc + a.Dr + c, a.dst_dtype, mul_nc(mu, sn));
     }
     used += 2 * a.Dr;
   } else {  // RoPE (mode 1) or plain (mode 2): values kept in registers for the optional L2 norm
@@ -79,14 +79,14 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
     for (int k = 0; k < MAX_PAIRS_PER_LANE; ++k) {
       const int i = 4 * lane + k;
       if (i < npairs) {
-        row_store(a.dst, drow, a.width, a.Dc + 2 * i, a.dst_dtype, a.l2norm ? y0[k] / den : y0[k]);
+        row_store<SPLIT>(a.dst, drow, a.width, a.Dc + 2 * i, a.dst_dtype, a.l2norm ? y0[k] / den : y0[k]);
         if (2 * i + 1 < a.Dr)
-          row_store(a.dst, drow, a.width, a.Dc + 2 * i + 1, a.dst_dtype, a.l2norm ? y1[k] / den : y1[k]);
+          row_store<SPLIT>(a.dst, drow, a.width, a.Dc + 2 * i + 1, a.dst_dtype, a.l2norm ? y1[k] / den : y1[k]);
       }
     }
     used += a.Dr;
   }
-  for (int c = used + lane; c < a.width; c += 64) row_store(a.dst, drow, a.width, c, a.dst_dtype, 0.f);
+  for (int c = used + lane; c < a.width; c += 64) row_store<SPLIT>(a.dst, drow, a.width, c, a.dst_dtype, 0.f);
 }
 
 __device__ __forceinline__ void phase_table_body(const float* freqs, int start, int S, int Dr, int pos_round,
@@ -102,7 +102,7 @@ __device__ __forceinline__ void phase_table_body(const float* freqs, int start, 
 // One wave per padded row (b, h, s < S_pad).  Rows s < S: dO repack, Di, L2 = lse*log2(e) (a row
 // without visible keys, lse = -inf, gets +inf so that its probabilities are 0).  Padding rows:
 // Di = 0, L2 = +inf.
-__global__ __launch_bounds__(256) void prebwd_kernel(PreBwdArgs a) {
+template <bool SPLIT> __global__ __launch_bounds__(256) void prebwd_kernel(PreBwdArgs a) {
   const int lane = threadIdx.x & 63;
   const int64_t prow = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int64_t nprows = (int64_t)a.B * a.H * a.s_pad;
@@ -124,13 +124,13 @@ __global__ __launch_bounds__(256) void prebwd_kernel(PreBwdArgs a) {
       d = load_as_float(a.dout, d0 + c * a.do_s[3], a.dout_dtype);
       acc += d * load_as_float(a.out, o0 + c * a.o_s[3], a.out_dtype);
     }
-    if (a.dO_op) row_store(a.dO_op, row, a.width, c, a.op_dtype, d);
+    if (a.dO_op) row_store<SPLIT>(a.dO_op, row, a.width, c, a.op_dtype, d);
   }
   acc = wave_sum(acc);
   if (lane == 0) {
     a.Di[prow] = acc;
     const float lv = a.lse[row];
-    a.L2[prow] = lv == -INFINITY ? INFINITY : (a.op_dtype == DT_SPLIT ? lv : lv * LOG2E);
+    a.L2[prow] = lv == -INFINITY ? INFINITY : (SPLIT ? lv : lv * LOG2E);
   }
 }
 
@@ -683,7 +683,9 @@ int launch_prep(const PrepArgs& a, hipStream_t s) {
     const int64_t nthr = nrows << lg;
     hipLaunchKernelGGL(prep_rope_vec_kernel, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, s, a, lg);
   } else {
-    hipLaunchKernelGGL(prep_kernel, dim3((unsigned)((nrows + 3) / 4)), dim3(256), 0, s, a);
+    const dim3 grid((unsigned)((nrows + 3) / 4));
+    if (a.dst_dtype == DT_SPLIT) hipLaunchKernelGGL(prep_kernel<true>, grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(prep_kernel<false>, grid, dim3(256), 0, s, a);
   }
   return hipGetLastError() == hipSuccess ? 0 : -7;
 }
@@ -879,7 +881,9 @@ int launch_prebwd(const PreBwdArgs& a, const TabArgs& t, hipStream_t s) {
     else if (a.op_dtype != DT_SPLIT) hipLaunchKernelGGL((prebwd_vec_kernel<1, 1>), grid, dim3(256), 0, s, a, lg);
     else hipLaunchKernelGGL((prebwd_vec_kernel<1, DT_SPLIT>), grid, dim3(256), 0, s, a, lg);
   } else {
-    hipLaunchKernelGGL(prebwd_kernel, dim3((unsigned)((nrows + 3) / 4)), dim3(256), 0, s, a);
+    const dim3 grid((unsigned)((nrows + 3) / 4));
+    if (a.op_dtype == DT_SPLIT) hipLaunchKernelGGL(prebwd_kernel<true>, grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(prebwd_kernel<false>, grid, dim3(256), 0, s, a);
   }
   if (t.tab) return launch_phase_table(t.freqs, t.start, t.S, t.D, t.pos_round, t.tab, s);
   return hipGetLastError() == hipSuccess ? 0 : -7;
